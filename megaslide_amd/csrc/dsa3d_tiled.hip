@@ -24,401 +24,6 @@ namespace {
 
 using namespace tiled;
 
-// The S (pass 1) and A (pass 2) tables are double-buffered where that keeps
-// the workgroups per CU: a step's table is written while the other buffer may
-// still be read for the previous step, so pass 1 needs one barrier per step and
-// pass 2 two (instead of two and three).  bf16 head_dim 96 keeps one buffer:
-// two would drop it to one workgroup per CU (measured 30% slower).  bf16
-// head_dim 128 without extra keys stages V^T in two 64-channel rounds per
-// step, which leaves room for two workgroups per CU; with extra keys it, and
-// every fp32 head, stages too much V^T for two and runs one, with the
-// register cap raised to match.
-constexpr int kLdsBytes = 160 * 1024;
-constexpr int kTabBytes = kTQ * kSRow * 4;
-
-template <int HD, typename E, bool XK>
-constexpr bool fwd_half_v() {
-  return !XK && ((sizeof(E) == 2 && HD == 128) || (sizeof(E) == 4 && HD == 64));
-}
-
-// bf16 V^T chunks take the swizzled (bank-conflict-free) layout.
-template <typename E>
-constexpr int fwd_vt_row() {
-  return sizeof(E) == 2 ? kVRowSwz : ElemT<E>::kRow;
-}
-
-template <int HD, typename E, bool XK = false>
-constexpr int fwd_vt_bytes() {
-  return (fwd_half_v<HD, E, XK>() ? HD / 2 : HD) * fwd_vt_row<E>() *
-         static_cast<int>(sizeof(word_t<E>));
-}
-
-template <int HD, typename E, bool XK = false>
-constexpr int fwd_table_bufs() {
-  constexpr int vt = fwd_vt_bytes<HD, E, XK>();
-  if (2 * (2 * kTabBytes + vt) <= kLdsBytes) return 2;  // two workgroups per CU
-  if (2 * (kTabBytes + vt) <= kLdsBytes) return 1;      // two workgroups per CU
-  return 2 * kTabBytes + vt <= kLdsBytes ? 2 : 1;       // one workgroup per CU
-}
-
-// Minimum waves per SIMD: 4 when two 512-thread workgroups fit in a CU's LDS
-// (bf16; the fp32 operands need more than 128 registers).
-template <int HD, typename E, bool XK = false>
-constexpr int fwd_min_waves() {
-  if constexpr (sizeof(E) == 4 && !fwd_half_v<HD, E, XK>()) return 2;
-  return 2 * (fwd_table_bufs<HD, E, XK>() * kTabBytes + fwd_vt_bytes<HD, E, XK>()) <= kLdsBytes
-             ? 4
-             : 2;
-}
-
-// Slot words as used in the forward's plane loops: at head_dim 96 (128
-// registers at 4 waves/SIMD) opaque, which stops the hoisting that spilled
-// (10% faster); elsewhere the hoisted keys and weights are cheaper (5%).
-template <int HD>
-__device__ __forceinline__ Slot fwd_slot(const Slot& s) {
-  if constexpr (HD == 96) return opaque(s);
-  return s;
-}
-
-// XK: the call has extra keys (a.G > 0); without them the kernel compiles to
-// the plain tap path.
-template <int HD, typename E, bool XK>
-__global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E, XK>())) void dsa3d_fwd_tiled_kernel(
-    Args a, E* __restrict__ out, float* __restrict__ lse) {
-  constexpr int NB = fwd_table_bufs<HD, E, XK>();
-  constexpr int VR = fwd_vt_row<E>();
-  constexpr bool kHV = fwd_half_v<HD, E, XK>();  // V^T in two 64-channel rounds
-  constexpr int VC = kHV ? HD / 2 : HD;           // V^T channels staged at once
-  __shared__ __attribute__((aligned(16))) float s_tab[NB][kTQ * kSRow];  // S, then A
-  __shared__ __attribute__((aligned(16))) word_t<E> s_vt[VC * VR];      // V^T chunk
-  __shared__ int s_red[kWaves][6];
-  // per query: 1, or NaN when a score is not finite (its output is NaN then, as
-  // softmax makes it in the reference; the fixed-point weights alone would drop it)
-  __shared__ float s_qnan[kTQ];
-
-  const Tile tl = make_tile<1, kSubs>(a);
-  // the tile's q rows load while the slots are set up
-  op_t<E> qx[HD / 32];
-  load_rows_operand<HD, E>(a, tl, static_cast<const E*>(a.q), a.qs, qx);
-  // finite tables before the first step (the paired corner reads may read an
-  // entry no step has written yet); the setup's barrier orders this before
-  // the first table store
-  zero_tables_all<NB>(&s_tab[0][0]);
-  Slot sl[kSlots];
-  Box box;
-  setup_slots<E, kSubs, kSlots>(a, tl, sl, box, s_red, true);
-  const int nchunks = box.ncy * box.ncx;
-  const int nit = (box.zhi - box.zlo + 1) * nchunks;
-  const E* const kp = static_cast<const E*>(a.k);
-  const E* const vp = static_cast<const E*>(a.v);
-
-  // ---- pass 1: scores -------------------------------------------------------
-  // K rows of the next (plane, chunk) are loaded while the current one is used
-  float sc[kSlots];
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) sc[i] = 0.0f;
-  TableRows<HD, E> rows;
-  Walk w = walk_begin(box);
-  if (nit > 0) load_table_rows<HD, E>(a, tl, w.c, w.z, kp, a.ks, rows);
-  for (int it = 0; it < nit; ++it) {
-    const Walk wn = walk_next(box, w);
-    const Chunk& c = w.c;
-    const int z = w.z;
-    // buffer it % NB was last read for step it - NB, before the previous barrier
-    float* tab = s_tab[it % NB];
-    store_table<HD, E>(tl, c, qx, rows, tab);
-    if (it + 1 < nit) load_table_rows<HD, E>(a, tl, wn.c, wn.z, kp, a.ks, rows);
-    __syncthreads();
-    // only the lanes whose tap has corners on this step read them; a slot that
-    // no lane of the wave hits (about a third of them) is skipped
-    const float* my_row = &tab[tl.q * kSRow];
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      const Slot si = fwd_slot<HD>(sl[i]);
-      float wz, dwz;
-      if (!slot_hits(si, step_key(c.id, z), wz, dwz)) continue;
-      float t0, t1, t2, t3;
-      corners4(si, my_row, t0, t1, t2, t3);
-      sc[i] = __builtin_fmaf(wz, bilerp(si, t0, t1, t2, t3).val, sc[i]);
-    }
-    if constexpr (NB == 1) __syncthreads();  // the next step overwrites the table
-    w = wn;
-  }
-
-  // ---- extra keys (attention.py:160-173): S_e[q][g] = q . ek_g (MFMA) into the
-  // first table, read back by the lanes of each query: lane `sub` takes keys
-  // sub + 32 j ------------------------------------------------------------------
-  constexpr int EPL = XK ? kMaxExtra / kSubs : 1;
-  const int G = XK ? a.G : 0, Gp = (G + 31) & ~31;
-  float se[EPL];
-  if constexpr (XK) {
-    __syncthreads();  // every pass-1 read of the tables is done
-    for (int eb = tl.wave; eb < Gp / 16; eb += kWaves) {
-      op_t<E> y[HD / 32];
-      load_extra_rows<HD, E>(a, tl, a.ek, eb, y);
-      f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int cc = 0; cc < HD / 32; ++cc) acc = mma16(qx[cc], y[cc], acc);
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr)
-        s_tab[0][(4 * (tl.lane >> 4) + rr) * kSRow + 16 * eb + (tl.lane & 15)] = acc[rr];
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < EPL; ++j) {
-    const int g = tl.sub + kSubs * j;
-    se[j] = XK && g < G ? s_tab[0][tl.q * kSRow + g] * a.softmax_scale : -INFINITY;
-  }
-
-  // ---- softmax over each query's taps (32 lanes x kSlots) and extra keys ----
-  float mx = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) {
-    sc[i] = slot_z0(sl[i]) >= 0 ? sc[i] * a.softmax_scale : -INFINITY;
-    mx = fmaxf(mx, sc[i]);
-  }
-  if constexpr (XK) {
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) mx = fmaxf(mx, se[j]);
-  }
-#pragma unroll
-  for (int m = 1; m < kSubs; m <<= 1) mx = fmaxf(mx, __shfl_xor(mx, m));
-  float den = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) {
-    sc[i] = slot_z0(sl[i]) >= 0 ? __expf(sc[i] - mx) : 0.0f;
-    den += sc[i];
-  }
-  if constexpr (XK) {
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      se[j] = tl.sub + kSubs * j < G ? __expf(se[j] - mx) : 0.0f;
-      den += se[j];
-    }
-  }
-#pragma unroll
-  for (int m = 1; m < kSubs; m <<= 1) den += __shfl_xor(den, m);
-  const float inv_den = 1.0f / den;
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i)
-    sc[i] *= inv_den * slot_dropout(sl[i], a.drop) * a.fix_a;  // p (dropped), fixed-point units
-  {
-    // the query index from the wave (a scalar) and the lane id: a per-lane
-    // index kept across the plane loops spilled
-    const unsigned tid = 64u * static_cast<unsigned>(__builtin_amdgcn_readfirstlane(tl.wave)) +
-                         __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    if (tid % kSubs == 0) s_qnan[tid / kSubs] = den == den ? 1.0f : __builtin_nanf("");
-  }
-  if (lse != nullptr && tl.sub == 0 && !kHV) {
-    if (tl.q_ok) lse[tl.qn * a.nh + tl.head] = mx + logf(den);
-  } else if (lse != nullptr && tl.sub == 0) {
-    // V^T in rounds (bf16 head_dim 128, fp32 64): the query's token row rebuilt
-    // from the wave (a scalar) and the lane id (kept across the plane loop, it
-    // spilled)
-    const unsigned tid = 64u * static_cast<unsigned>(__builtin_amdgcn_readfirstlane(tl.wave)) +
-                         __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    const int64_t qn = tile_row(a, tl, static_cast<int>(tid / kSubs));
-    if (qn >= 0) lse[qn * a.nh + tl.head] = mx + logf(den);
-  }
-
-  // ---- output.  The waves form CG channel groups of KP waves; wave w of group
-  // g takes the k-steps w % KP, + KP, ... of a table for the TPW channel tiles of
-  // group g: one A operand feeds TPW independent MFMAs, and the KP partial O
-  // are summed once at the end.  hd 64 and 128: one group of 8 waves (fp32
-  // hd 128: two groups of 4, for registers).  hd 96: six single-tile groups
-  // (waves 6, 7 idle), which stays within 128 registers and measured faster
-  // than groups of several tiles.
-  constexpr int CT = HD / 16, CG = HD == 96 ? CT : (sizeof(E) == 4 && HD == 128 ? 2 : 1);
-  constexpr int TPW = CT / CG, KP = HD == 96 ? 1 : kWaves / CG;
-  static_assert(TPW * CG == CT && CG * KP <= kWaves, "channel tiles split over the waves");
-  const int mq = tl.lane & 15, kq = 8 * (tl.lane >> 4);
-  // bf16 V^T chunks are stored swizzled (row 16 t + mq: channel bits 2, 3 = those of mq)
-  constexpr bool kSwz = sizeof(E) == 2;
-  const int sw = kSwz ? vt_swz(mq) : 0;
-  const int cg = tl.wave / KP, kph = tl.wave % KP;
-  const bool av_wave = tl.wave < CG * KP;
-  f32x4_t oacc[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) oacc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  if constexpr (XK) {
-    // extra keys: O += P_e . EV with P_e = p f (fixed-point units, as floats)
-    // in place of S_e (each entry is read and written by its own lane) and EV
-    // staged transposed in the V^T buffer
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      const int g = tl.sub + kSubs * j;
-      if (g < Gp)
-        s_tab[0][tl.q * kSRow + g] =
-            g < G ? se[j] * inv_den * a.fix_a *
-                        (a.drop.threshold == 0
-                             ? 1.0f
-                             : dropout_factor(a.drop, tl.qn, tl.head, a.K + g))
-                  : 0.0f;
-    }
-    stage_extra_t<HD, E>(a, tl, a.ev, 0, Gp, VR, s_vt, kThreads);
-    __syncthreads();
-    for (int kc = 32 * kph; av_wave && kc < Gp; kc += 32 * KP) {
-      const op_t<E> av = f32_to_op<E>(&s_tab[0][mq * kSRow + kc + kq]);
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-        oacc[t] = mma16(av, load_op<E>(&s_vt[(16 * (cg * TPW + t) + mq) * VR + kc + kq]), oacc[t]);
-    }
-  }
-
-  // ---- pass 2: O += A . V over the taps --------------------------------------
-  if constexpr (kHV) {
-    // channels [0, 64) then [64, 128) of each step's V^T through one buffer;
-    // wave w takes channel tile w % 4 of each round and the k-steps w / 4,
-    // + 2, ...; the two partial O are summed at the end
-    constexpr int RT = VC / 16, KPH = kWaves / RT;
-    const int tt = tl.wave % RT, kh2 = tl.wave / RT;
-    f32x4_t oh[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
-    StageRows<kThreads, VC, E> vh;
-    w = walk_begin(box);
-    if (nit > 0)
-      load_stage_rows<kThreads, VC, E, true>(a, tl, w.c, w.z, vp, a.vs, tl.head * HD, vh);
-    __syncthreads();  // pass-1 reads of both buffers are done
-    zero_table(s_tab[0], kChunkNV);
-    for (int it = 0; it < nit; ++it) {
-      const Walk wn = walk_next(box, w);
-      const Chunk& c = w.c;
-      const int z = w.z;
-      int* const s_atab = reinterpret_cast<int*>(s_tab[it % NB]);
-      int* row = &s_atab[tl.q * kSRow];
-      __syncthreads();  // the previous step's MFMAs are done with V^T; this buffer is zeroed
-      store_stage<kThreads, VC, E, kSwz>(c, vh, s_vt);
-      load_stage_rows<kThreads, VC, E, true>(a, tl, c, z, vp, a.vs, tl.head * HD + VC, vh);
-#pragma unroll
-      for (int i = 0; i < kSlots; ++i) {
-        const Slot si = fwd_slot<HD>(sl[i]);
-        float wz, dwz;
-        if (!slot_hits(si, step_key(c.id, z), wz, dwz)) continue;
-        const float pz = sc[i] * wz;
-        const float gx = 1.0f - si.fx, gy = 1.0f - si.fy;
-        const int base = si.idx & 0x1ff, dy = (si.idx >> 9) & 0x1f;
-        atomicAdd(&row[base], to_fix(pz * (gy * gx)));
-        atomicAdd(&row[base + 1], to_fix(pz * (gy * si.fx)));
-        atomicAdd(&row[base + dy], to_fix(pz * (si.fy * gx)));
-        atomicAdd(&row[base + dy + 1], to_fix(pz * (si.fy * si.fx)));
-      }
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        if (r == 1) {
-          __syncthreads();  // every wave is done with the first round's V^T
-          store_stage<kThreads, VC, E, kSwz>(c, vh, s_vt);
-          if (it + 1 < nit)
-            load_stage_rows<kThreads, VC, E, true>(a, tl, wn.c, wn.z, vp, a.vs, tl.head * HD, vh);
-          __syncthreads();
-        }
-        for (int kc = 32 * kh2; kc < c.nvp; kc += 32 * KPH) {
-          const op_t<E> av = fix_to_op<E>(&s_atab[mq * kSRow + kc + kq]);
-          oh[r] = mma16(av, load_op<E>(&s_vt[(16 * tt + mq) * VR + ((kc + kq) ^ sw)]), oh[r]);
-        }
-      }
-      if constexpr (NB == 1) __syncthreads();
-      if (it + 1 < nit) zero_table(s_tab[(it + 1) % NB], kChunkNV);
-      w = wn;
-    }
-    __syncthreads();
-    // oh[r][i] = partial O[query 4 (lane / 16) + i][channel 16 (4 r + tt) + lane % 16]
-    // of k phase kh2, through the (free) V^T buffer: red[k phase][16][HD]
-    float* red = reinterpret_cast<float*>(s_vt);
-    static_assert(KPH * kTQ * HD * 4 <= fwd_vt_bytes<HD, E, XK>(), "partials fit the V^T buffer");
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        red[(kh2 * kTQ + 4 * (tl.lane >> 4) + i) * HD + 16 * (RT * r + tt) + mq] = oh[r][i];
-    __syncthreads();
-    for (int e = threadIdx.x; e < kTQ * HD; e += kThreads) {
-      float o = 0.0f;
-#pragma unroll
-      for (int kp = 0; kp < KPH; ++kp) o += red[kp * kTQ * HD + e];
-      const int m = e / HD, ch = e - m * HD;
-      const int64_t n = tile_row(a, tl, m);
-      if (n >= 0)
-        out[n * (static_cast<int64_t>(a.nh) * HD) + tl.head * HD + ch] =
-            from_f32<E>(o * a.fix_a_inv * s_qnan[m]);
-    }
-    return;
-  }
-  StageRows<kThreads, HD, E> vr;
-  w = walk_begin(box);
-  if (nit > 0) load_stage_rows<kThreads, HD, E, true>(a, tl, w.c, w.z, vp, a.vs, tl.head * HD, vr);
-  __syncthreads();  // pass-1 reads of both buffers are done
-  zero_table(s_tab[0], kChunkNV);
-  for (int it = 0; it < nit; ++it) {
-    const Walk wn = walk_next(box, w);
-    const Chunk& c = w.c;
-    const int z = w.z;
-    // A in fixed point (scale fix_a), buffer it % NB: zeroed during the previous step
-    int* const s_atab = reinterpret_cast<int*>(s_tab[it % NB]);
-    int* row = &s_atab[tl.q * kSRow];
-    __syncthreads();  // the previous step's MFMAs are done with V^T; this buffer is zeroed
-    store_stage<kThreads, HD, E, kSwz>(c, vr, s_vt);
-    if (it + 1 < nit)
-      load_stage_rows<kThreads, HD, E, true>(a, tl, wn.c, wn.z, vp, a.vs, tl.head * HD, vr);
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      const Slot si = fwd_slot<HD>(sl[i]);
-      float wz, dwz;
-      if (!slot_hits(si, step_key(c.id, z), wz, dwz)) continue;
-      const float pz = sc[i] * wz;
-      const float gx = 1.0f - si.fx, gy = 1.0f - si.fy;
-      const int base = si.idx & 0x1ff, dy = (si.idx >> 9) & 0x1f;
-      // an upper corner outside the volume has weight 0, so all four adds run
-      // without branches: a y corner (offset 0) adds 0 to the lower one, an x
-      // corner adds 0 to the next entry (at most column kChunkNV, inside the
-      // row), and the x pair keeps one address with immediate offsets
-      atomicAdd(&row[base], to_fix(pz * (gy * gx)));
-      atomicAdd(&row[base + 1], to_fix(pz * (gy * si.fx)));
-      atomicAdd(&row[base + dy], to_fix(pz * (si.fy * gx)));
-      atomicAdd(&row[base + dy + 1], to_fix(pz * (si.fy * si.fx)));
-    }
-    __syncthreads();
-    for (int kc = 32 * kph; av_wave && kc < c.nvp; kc += 32 * KP) {
-      const op_t<E> av = fix_to_op<E>(&s_atab[mq * kSRow + kc + kq]);
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-        oacc[t] = mma16(av, load_op<E>(&s_vt[(16 * (cg * TPW + t) + mq) * VR + ((kc + kq) ^ sw)]),
-                        oacc[t]);
-    }
-    // the next buffer was last read for step it + 1 - NB, before the barrier
-    // above (with one buffer: this step, so wait for every wave's MFMAs first)
-    if constexpr (NB == 1) __syncthreads();
-    if (it + 1 < nit) zero_table(s_tab[(it + 1) % NB], kChunkNV);
-    w = wn;
-  }
-  __syncthreads();
-  // oacc[t][r] = wave partial of O[query 4*(lane/16) + r][channel 16*(cg*TPW +
-  // t) + lane%16] in fixed-point units of A.  The V^T buffer (free after the
-  // barrier above) takes the KP partials of every channel; every thread then
-  // sums KP for its outputs, consecutive threads on consecutive channels.
-  float* red = reinterpret_cast<float*>(s_vt);  // [k phase][16][HD]
-  static_assert(kHV || KP * kTQ * HD * 4 <= fwd_vt_bytes<HD, E, XK>(),
-                "partials fit the V^T buffer");
-  if (av_wave) {
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[(kph * kTQ + 4 * (tl.lane >> 4) + r) * HD + 16 * (cg * TPW + t) + mq] = oacc[t][r];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < kTQ * HD; e += kThreads) {
-    float o = 0.0f;
-#pragma unroll
-    for (int kp = 0; kp < KP; ++kp) o += red[kp * kTQ * HD + e];
-    const int m = e / HD, ch = e - m * HD;
-    const int64_t n = tile_row(a, tl, m);
-    if (n >= 0)
-      out[n * (static_cast<int64_t>(a.nh) * HD) + tl.head * HD + ch] =
-          from_f32<E>(o * a.fix_a_inv * s_qnan[m]);
-  }
-}
-
 // 32 x 16 block vb of a transposed [voxel][query] fixed-point table (row stride
 // `row`, queries from column col0) as the A operand of the 32x32 MFMA: lane l
 // holds voxel 32*vb + l%32, queries col0 + 8*(l/32) + j, in fixed-point units
@@ -2182,10 +1787,25 @@ __global__ __launch_bounds__(256) void extra_grad_kernel(const E* __restrict__ d
 
 }  // namespace
 
+// CUs of the current device (the persistent grids),
+// cached per device; 256 (MI355X) if the query fails.
+int device_cus() {
+  static int cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int n = 0;
+    cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
+                              hipSuccess && n > 0
+                      ? n
+                      : 256;
+  }
+  return cached[dev];
+}
+
 // Kernel arguments for a launch over `tiles` workgroups per head.
 tiled::Args make_tiled_args(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,
-                            const void* off, int64_t tiles, const void* ek = nullptr,
-                            const void* ev = nullptr) {
+                            const void* off, int64_t tiles, const void* ek, const void* ev) {
   tiled::Args a;
   a.ek = ek;
   a.ev = ev;
@@ -2211,6 +1831,13 @@ tiled::Args make_tiled_args(const msd_dsa3d_desc& d, const void* q, const void* 
   a.C = d.num_heads * a.K * 3;
   a.tiles_h = (d.H + tiled::kTileH - 1) / tiled::kTileH;
   a.tiles_w = (d.W + tiled::kTileW - 1) / tiled::kTileW;
+  auto recip = [](int d) {
+    return static_cast<uint32_t>(std::min<uint64_t>((uint64_t{1} << 32) / static_cast<uint32_t>(d), 0xffffffffu));
+  };
+  a.m_t = recip(a.T);
+  a.m_tw = recip(a.tiles_w);
+  a.m_th = recip(a.tiles_h);
+  a.m_b = recip(a.B);
   a.xcd_remap = (tiles % 8 == 0) ? static_cast<int>(tiles / 8) : 0;
   a.head0 = 0;
   a.offset_scale = d.offset_scale;
@@ -2281,37 +1908,6 @@ bool dsa3d_tiled_supported(const msd_dsa3d_desc& d, const void* q, const void* k
   for (const void* p : {q, k, v})
     if (reinterpret_cast<uintptr_t>(p) % 16) return false;
   return true;
-}
-
-namespace {
-template <typename E>
-hipError_t fwd_tiled_typed(const msd_dsa3d_desc& d, const tiled::Args& a, void* out, float* lse,
-                           hipStream_t s) {
-  const dim3 grid = tiled_grid<1>(d), block(tiled::kThreads);
-  E* o = static_cast<E*>(out);
-  auto go = [&]<int HD>() {
-    if (a.G > 0)
-      hipLaunchKernelGGL((dsa3d_fwd_tiled_kernel<HD, E, true>), grid, block, 0, s, a, o, lse);
-    else
-      hipLaunchKernelGGL((dsa3d_fwd_tiled_kernel<HD, E, false>), grid, block, 0, s, a, o, lse);
-  };
-  switch (d.head_dim) {
-    case 32: go.template operator()<32>(); break;
-    case 64: go.template operator()<64>(); break;
-    case 96: go.template operator()<96>(); break;
-    case 128: go.template operator()<128>(); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-}  // namespace
-
-hipError_t launch_dsa3d_fwd_tiled(const msd_dsa3d_desc& d, const void* q, const void* k,
-                                  const void* v, const void* off, const void* ek, const void* ev,
-                                  void* out, float* lse, hipStream_t s) {
-  const tiled::Args a = make_tiled_args(d, q, k, v, off, tiled_tiles<1>(d), ek, ev);
-  if (d.dtype == MSD_BF16) return fwd_tiled_typed<bf16>(d, a, out, lse, s);
-  return fwd_tiled_typed<float>(d, a, out, lse, s);
 }
 
 // Largest power of two s with s * bound <= 2^14 (1 for a zero or non-finite
@@ -2525,22 +2121,6 @@ struct BwdBufs {
   float* dlt;      // extra keys: Delta per (token, head), fp32 [rows, nh] (null without them)
   RecArgs rec;     // column-streaming kernel's records (rec.rec null: not used)
 };
-
-// CUs of the current device (the column-streaming kernel's persistent grid),
-// cached per device; 256 (MI355X) if the query fails.
-int device_cus() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
-                              hipSuccess && n > 0
-                      ? n
-                      : 256;
-  }
-  return cached[dev];
-}
 
 template <int HD, typename E>
 void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,

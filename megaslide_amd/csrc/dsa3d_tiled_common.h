@@ -143,6 +143,7 @@ struct Args {
   int64_t N;
   int B, T, H, W, nh, kt, kh, kw, K, C;
   int tiles_h, tiles_w;
+  uint32_t m_t, m_tw, m_th, m_b;  // floor(2^32 / d) of T, tiles_w, tiles_h, B (2^32 - 1 for 1)
   int xcd_remap;       // tiles per XCD when tiles are spread XCD-contiguously, else 0
   int head0;           // head of blockIdx.y 0 (a launch over a group of heads)
   float offset_scale, softmax_scale;
@@ -160,6 +161,14 @@ struct Args {
   float* dlt;                    // backward with extra keys: per (token, head) fp32 Delta,
                                  //   their part, then (first backward kernel) the whole
 };
+
+// Kernel arguments for a launch over `tiles` workgroups per head (dsa3d_tiled.hip).
+}  // namespace tiled
+tiled::Args make_tiled_args(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,
+                            const void* off, int64_t tiles, const void* ek, const void* ev);
+// CUs of the current device (dsa3d_tiled.hip).
+int device_cus();
+namespace tiled {
 
 constexpr int kMaxExtra = 256;   // extra keys the tiled kernels take (a table row)
 

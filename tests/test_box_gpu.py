@@ -1,0 +1,72 @@
+"""The whole-box forward kernel where its table, pieces and transposition can go wrong.
+
+Against the direct kernels on the same inputs (their own oracle tests pin them): boxes of one
+piece and of many (offsets of many voxels), boxes reaching past every face of the volume, unit
+axes, partial tiles, windows of 1 to 160 taps (one to five taps per lane, the last partly
+filled).  fp32: both sum the same products in fp32, the tiled weights in fixed point of 2^-30
+per corner (at most 8 * 160 corners per output, |V| < 6): 1e-5.  bf16: the weights are rounded
+to bf16 (2^-9) and so is the output: 2e-2 of the largest value.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # T, H, W, heads, window, offset std in voxels
+    (1, 4, 4, 1, (1, 1, 1), 0.0),
+    (7, 12, 12, 2, (3, 7, 7), 0.5),    # the usual box: one piece
+    (9, 13, 21, 1, (3, 7, 7), 6.0),    # cut along several axes
+    (5, 30, 33, 1, (3, 7, 7), 30.0),   # clamped onto every face, most of the volume
+    (40, 5, 1, 1, (5, 7, 4), 9.0),     # a unit axis, a long one, 140 taps
+    (1, 3, 70, 2, (1, 4, 40), 2.0),    # 160 taps, wide and flat
+    (6, 1, 9, 1, (3, 1, 11), 1.0),     # 33 taps
+]
+
+
+def _inputs(case, hd, dt):
+    T, H, W, nh, win, std = case
+    g = torch.Generator().manual_seed(5)
+    N, K = T * H * W, win[0] * win[1] * win[2]
+    q, k, v = (torch.randn(1, N, nh * hd, generator=g) for _ in range(3))
+    # slot 0 moves x by W / 2 / max(T - 1, 1) voxels a unit, slot 2 z by T / 2 / max(W - 1, 1)
+    unit = torch.tensor([max(T - 1, 1) / W, max(H - 1, 1) / H, max(W - 1, 1) / T]) * 2
+    off = (torch.randn(1, N, nh * K, 3, generator=g) * std * unit).view(1, N, -1)
+    return [t.to(dt).cuda() for t in (q, k, v, off)]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("case", CASES)
+def test_box_forward_matches_direct(case, hd, dt):
+    from megaslide_amd import dsa3d_core
+
+    print(f"[box forward] {case} {hd} {dt}", flush=True)
+    T, H, W, nh, win, _ = case
+    ins = _inputs(case, hd, dt)
+    with torch.no_grad():
+        a, la = dsa3d_core(*ins, (T, H, W), nh, win, algo="tiled", return_lse=True)
+        b, lb = dsa3d_core(*ins, (T, H, W), nh, win, algo="direct", return_lse=True)
+    tol = 1e-5 if dt == torch.float32 else 2e-2
+    assert (a.float() - b.float()).abs().max() <= tol * b.float().abs().max()
+    assert (la - lb).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+def test_infinite_value_stays_in_its_channel(hd):
+    """bf16: a V row with one infinite element spoils that channel of the queries whose box
+    holds it, no other channel."""
+    from megaslide_amd import dsa3d_core
+
+    case = (5, 9, 11, 1, (3, 7, 7), 0.5)
+    q, k, v, off = _inputs(case, hd, torch.bfloat16)
+    with torch.no_grad():
+        ref = dsa3d_core(q, k, v, off, case[:3], 1)
+        ch, vox = hd - 3, (2 * 9 + 4) * 11 + 5
+        v[0, vox, ch] = float("inf")
+        out = dsa3d_core(q, k, v, off, case[:3], 1)
+    keep = torch.arange(hd, device="cuda") != ch
+    assert torch.isfinite(out[..., keep]).all()
+    assert (out[..., keep].float() - ref[..., keep].float()).abs().max() < 2e-2
+    assert not torch.isfinite(out[0, vox, ch])
