@@ -94,8 +94,9 @@ typedef enum msd_accum { MSD_ACCUM_F32 = 0, MSD_ACCUM_F16 = 1 } msd_accum;
 
 /* Kernel family for the attention core.  AUTO picks the matrix-core tiled
  * kernels when the call qualifies (bf16 or fp32, head_dim 32/64/96/128, <= 160
- * taps, token strides multiples of 8 elements, 16-byte aligned rows) and the
- * direct kernels otherwise.  DIRECT and TILED force one family (TILED fails
+ * taps, token strides multiples of 8 elements, 16-byte aligned rows; also other
+ * head_dim that are multiples of 8 up to 120, in the backward given the workspace
+ * of msd_dsa3d_bwd_best_workspace_size) and the direct kernels otherwise.  DIRECT and TILED force one family (TILED fails
  * with MSD_ERR_UNSUPPORTED if not eligible). */
 typedef enum msd_algo { MSD_ALGO_AUTO = 0, MSD_ALGO_DIRECT = 1, MSD_ALGO_TILED = 2 } msd_algo;
 
@@ -136,6 +137,15 @@ int msd_dsa3d_fwd(const msd_dsa3d_desc* desc, const void* q, const void* k, cons
 
 /* Bytes of device workspace msd_dsa3d_bwd needs for `desc`. */
 size_t msd_dsa3d_bwd_workspace_size(const msd_dsa3d_desc* desc);
+
+/*
+ * Bytes with which msd_dsa3d_bwd is fastest for `desc`, at least what it needs.
+ * More than that for MSD_ALGO_AUTO calls whose head_dim is a multiple of 8 up to
+ * 120 but not of 32: with that much workspace they take the matrix-core kernels
+ * on padded fp32 copies, else the direct kernels (e.g. 4,096 tokens, 16 x 80,
+ * window 3x5x5, bf16: 3 ms against 113).
+ */
+size_t msd_dsa3d_bwd_best_workspace_size(const msd_dsa3d_desc* desc);
 
 /*
  * Backward of the attention core: the gradients autograd takes through

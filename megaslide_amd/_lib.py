@@ -97,6 +97,8 @@ def load() -> ctypes.CDLL:
         lib.msd_dsa3d_fwd.argtypes = [ctypes.POINTER(DsaDesc)] + [_vp] * 9
         lib.msd_dsa3d_bwd_workspace_size.restype = ctypes.c_size_t
         lib.msd_dsa3d_bwd_workspace_size.argtypes = [ctypes.POINTER(DsaDesc)]
+        lib.msd_dsa3d_bwd_best_workspace_size.restype = ctypes.c_size_t
+        lib.msd_dsa3d_bwd_best_workspace_size.argtypes = [ctypes.POINTER(DsaDesc)]
         lib.msd_dsa3d_bwd.restype = ctypes.c_int
         lib.msd_dsa3d_bwd.argtypes = [ctypes.POINTER(DsaDesc)] + [_vp] * 17 + [ctypes.c_size_t, _vp]
         lib.msd_dsa3d_bwd_noalloc.restype = ctypes.c_int

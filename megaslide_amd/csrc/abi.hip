@@ -171,6 +171,14 @@ int dsa3d_bwd_impl(const msd_dsa3d_desc* desc, const void* q, const void* k, con
                                                      lse, dlse, dq, dk, dv, doffsets, dek, dev,
                                                      workspace, s),
                          "dsa3d_bwd");
+  // head sizes between the compiled ones: on padded copies, where the workspace
+  // holds them
+  if (msd::dsa3d_ragged_supported(*desc, q, k, v) &&
+      workspace_bytes >= msd::dsa3d_ragged_bwd_ws_bytes(*desc))
+    return launch_status(msd::launch_dsa3d_bwd_ragged(*desc, q, k, v, offsets, ek, ev, dout, lse,
+                                                      dlse, dq, dk, dv, doffsets, dek, dev,
+                                                      workspace, s),
+                         "dsa3d_bwd");
   return launch_status(msd::launch_dsa3d_bwd_direct(*desc, q, k, v, offsets, ek, ev, out, dout,
                                                     lse, dlse, dq, dk, dv, doffsets, dek, dev,
                                                     workspace, s),
@@ -208,6 +216,10 @@ int msd_dsa3d_fwd(const msd_dsa3d_desc* desc, const void* q, const void* k, cons
     return launch_status(msd::launch_dsa3d_fwd_tiled(*desc, q, k, v, offsets, extra_k, extra_v,
                                                      out, lse, s),
                          "dsa3d_fwd");
+  if (msd::dsa3d_ragged_supported(*desc, q, k, v))
+    return launch_status(msd::launch_dsa3d_fwd_ragged(*desc, q, k, v, offsets, extra_k, extra_v,
+                                                      out, lse, s),
+                         "dsa3d_fwd");
   return launch_status(msd::launch_dsa3d_fwd_direct(*desc, q, k, v, offsets, extra_k, extra_v, out,
                                                     lse, s),
                        "dsa3d_fwd");
@@ -216,6 +228,14 @@ int msd_dsa3d_fwd(const msd_dsa3d_desc* desc, const void* q, const void* k, cons
 size_t msd_dsa3d_bwd_workspace_size(const msd_dsa3d_desc* desc) {
   if (check_dsa(desc) != MSD_OK) return 0;
   return msd::dsa3d_bwd_ws_bytes(*desc);
+}
+
+size_t msd_dsa3d_bwd_best_workspace_size(const msd_dsa3d_desc* desc) {
+  if (check_dsa(desc) != MSD_OK) return 0;
+  const size_t need = msd::dsa3d_bwd_ws_bytes(*desc);
+  if (!msd::dsa3d_ragged_supported(*desc, nullptr, nullptr, nullptr)) return need;
+  const size_t ragged = msd::dsa3d_ragged_bwd_ws_bytes(*desc);
+  return ragged > need ? ragged : need;
 }
 
 int msd_dsa3d_bwd(const msd_dsa3d_desc* desc, const void* q, const void* k, const void* v,

@@ -117,6 +117,16 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
                                   void* dek, void* dev, void* ws, hipStream_t s);
+bool dsa3d_ragged_supported(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v);
+hipError_t launch_dsa3d_fwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,
+                                   const void* v, const void* off, const void* ek, const void* ev,
+                                   void* out, float* lse, hipStream_t s);
+hipError_t launch_dsa3d_bwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,
+                                   const void* v, const void* off, const void* ek, const void* ev,
+                                   const void* dout, const float* lse, const float* dlse, void* dq,
+                                   void* dk, void* dv, void* doff, void* dek, void* dev, void* ws,
+                                   hipStream_t s);
+size_t dsa3d_ragged_bwd_ws_bytes(const msd_dsa3d_desc& d);
 size_t dsa3d_bwd_ws_bytes(const msd_dsa3d_desc& d);
 size_t dsa3d_tiled_bwd_ws_bytes(const msd_dsa3d_desc& d);
 hipError_t launch_dwconv3d_fwd(const msd_dwconv3d_desc& d, const void* x, const void* w,

@@ -713,32 +713,41 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
 }
 
 // box_weighted by plain arithmetic, one lane per output (register layout of
-// acc): taken after a non-finite result of the bf16 products, whose
-// transposition spreads a non-finite value over the channels of its row.
-template <int HD, typename S, typename Off>
+// acc), over the voxels a query's taps touch (a non-zero table entry: see
+// box_scatter), as grid_sample reads them: taken after a non-finite result, where
+// a product of a row's non-finite value and a zero weight would spoil queries
+// that do not sample the row, and the transposition the row's other channels.
+template <int HD, typename S, typename E, bool RG, typename Off>
 __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
-                                                  const Off& off, int n, const int* table,
+                                                  const Off& off, int n, int hd, const int* table,
                                                   f32x4_t (&acc)[HD / 16]) {
   const int m = tl.lane & 15, g = tl.lane >> 4;
 #pragma nounroll
   for (int e = 0;; ++e) {  // the wave's voxels: pairs w, w + 8, ... of blocks
     const int v = 32 * (tl.wave + kWaves * (e >> 5)) + (e & 31);
-    if (v >= n) break;  // n is a multiple of 32 or the rest has no rows
+    if (v >= n) break;
     const uint32_t o = off(v);
     if (o == kNoRow) continue;  // every lane: v is wave-uniform
-    float w[4];
+    int w[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float f = static_cast<float>(table[(4 * g + r) * kBoxRow + v]);
-      w[r] = to_f32(from_f32<S>(f));  // the products' operand
-    }
+    for (int r = 0; r < 4; ++r) w[r] = table[(4 * g + r) * kBoxRow + v];
 #pragma unroll
     for (int t = 0; t < HD / 16; ++t) {
-      const uint32_t x = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(
-          rows, o + static_cast<uint32_t>(16 * t + m) * 2u, 0, 0));
-      const float y = __uint_as_float(x << 16);
+      const int ch = box_channel<HD, E>(t, m);
+      const uint32_t at = RG && ch >= hd ? kNoRow : o + static_cast<uint32_t>(ch * sizeof(S));
+      float y;
+      if constexpr (sizeof(S) == 2)
+        y = __uint_as_float(
+            static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(rows, at, 0, 0)) << 16);
+      else
+        y = __uint_as_float(
+            static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rows, at, 0, 0)));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[t][r] = __builtin_fmaf(w[r], y, acc[t][r]);
+      for (int r = 0; r < 4; ++r) {
+        float f = static_cast<float>(w[r]);
+        if constexpr (sizeof(E) == 2) f = to_f32(from_f32<bf16>(f));  // the products' operand
+        if (w[r] != 0) acc[t][r] = __builtin_fmaf(f, y, acc[t][r]);
+      }
     }
   }
 }
@@ -785,17 +794,21 @@ __device__ __forceinline__ bool box_in(const BoxTaps<SLOTS>& tp, int i, int s) {
   return s < 0 || static_cast<uint32_t>(tp.at[i]) >> kAtBits == static_cast<uint32_t>(s);
 }
 
-// Adds the tap's weight v (fixed-point units) to its eight corners.
+// Adds the tap's weight v (fixed-point units) to its eight corners.  TOUCH: at
+// least one unit (2^-30) each, which marks the corners of zero weight too
+// (grid_sample reads those as well: 0 times a non-finite value is not 0).
+template <bool TOUCH = false>
 __device__ __forceinline__ void box_scatter(int* table, int at, int cx, int sz, float fx, float fy,
                                             float fz, float v) {
   int* const p = &table[at];
   int* const pz = p + sz;
   auto plane = [&](int* q, float w) {
     const float w1 = w * fy, w0 = w * (1.0f - fy), gx = 1.0f - fx;
-    atomicAdd(q, to_fix(w0 * gx));
-    atomicAdd(q + 1, to_fix(w0 * fx));
-    atomicAdd(q + cx, to_fix(w1 * gx));
-    atomicAdd(q + cx + 1, to_fix(w1 * fx));
+    auto fix = [](float x) { return TOUCH ? max(to_fix(x), 1) : to_fix(x); };
+    atomicAdd(q, fix(w0 * gx));
+    atomicAdd(q + 1, fix(w0 * fx));
+    atomicAdd(q + cx, fix(w1 * gx));
+    atomicAdd(q + cx + 1, fix(w1 * fx));
   };
   plane(p, v * (1.0f - fz));
   plane(pz, v * fz);

@@ -1,0 +1,314 @@
+// Matrix-core 3D-DSA forward for gfx950: bf16 or fp32 storage, fp32 accumulation.
+//
+// One workgroup = one (batch, head, frame, tile of 16 queries).  Instead of
+// gathering the 8 corner rows of K and V for each of a query's taps, it builds
+// dense tables on the matrix cores over the box of voxels that the tile's taps
+// reach (dsa3d_box.h: the whole box at once, or pieces of it):
+//   S[q][v] = q . K[v]  (MFMA, fp32 in LDS)  ->  per tap s = scale * sum_c w_c S[q][c]
+//   softmax over each query's taps in registers (wave reductions)
+//   A[q][v] = sum over taps/corners landing on v of p * w  (LDS integer adds)
+//   O[q] += A[q] . V  (MFMA, V transposed on the matrix cores)
+// This equals the reference's grid_sample + matmul + softmax + matmul
+// (infinity/video/attention.py:106-186) because trilinear sampling is linear in
+// the sampled rows.  Coordinates and corner choice round exactly as the fp32
+// reference does (div_rn, dsa3d_coords.h).
+//
+// Bound: the latency of the K and V rows' loads (half of a workgroup's time; the
+// box of a tile is about 1,000 rows of each, nine in ten from the L2) and VALU
+// issue (~1,450 instructions a wave).  Tables of the whole box against tables of
+// one plane at a time (tested by every tap on every plane, two or three barriers
+// each): 3.20 -> 2.86 ms at 65,536 tokens, 16 x 64, bf16; 6.5 -> 5.8 ms at 46,800
+// tokens, 16 x 96, offsets biased by up to 4 voxels; 2.04 -> 1.46 ms at 32,768
+// tokens, 8 x 64, fp32; 44 -> 30 us at 2,048 tokens, 4 x 64, fp32; unchanged
+// (12.3 -> 12.2 ms) at 131,072 tokens, 24 x 128.  Tried and slower: a persistent
+// grid with the next tile's offsets loaded ahead (registers spill), 8 or 10
+// blocks of K rows in flight per wave instead of 6.
+#pragma once
+
+#include <algorithm>
+#include <type_traits>
+
+#include "dsa3d_box.h"
+
+namespace msd {
+
+namespace {
+
+using namespace tiled;
+
+// Waves per SIMD: 4 (two workgroups per CU, 128 registers) except where the
+// fp32 operands of a wide head need more registers.
+template <int HD, typename E>
+constexpr int fwd_min_waves() {
+  return sizeof(E) == 4 && HD > 64 ? 2 : 4;
+}
+
+// S: storage, E: element type of the products.  XK: extra keys (a.G > 0).
+// RG: head_dim hd below HD (a multiple of 8), channels past it read as zero.
+// SAFE: the weighted sum by plain arithmetic.
+// Returns whether a sum was not finite.
+template <int HD, typename S, typename E, bool XK, bool RG, bool DROP, bool SAFE>
+__device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
+                                         float* __restrict__ lse, int hd_arg, unsigned tid,
+                                         int* s_tab, uint32_t* s_row, int* s_box,
+                                         float* s_qnan) {
+  float* const s_val = reinterpret_cast<float*>(s_tab);
+  const int hd = RG ? hd_arg : HD;
+
+  const Tile tl = box_tile(a, box_unit(a), tid);
+  RawOffsets<S, kSlots> raw;
+  box_load_offsets<S, kSlots>(a, tl, raw);
+  box_init(s_box);
+  __syncthreads();
+  // the tile's q rows load while the taps are set up
+  op_t<E> qx[HD / 32];
+  box_tile_rows<HD, S, E, RG>(a, tl, static_cast<const S*>(a.q), a.qs, hd, qx);
+  BoxTaps<kSlots> tp;
+  BoxPieces bx;
+  box_setup<S, kSlots, false, DROP>(a, tl, raw, tp, bx, s_box);
+
+  auto rows_of = [&](const void* base, int64_t stride) {
+    const S* p = static_cast<const S*>(base) + tl.sample0 * stride + static_cast<int64_t>(tl.head) * hd;
+    return box_rows(p, ((a.N - 1) * stride + hd) * static_cast<int64_t>(sizeof(S)));
+  };
+  auto set_rows = [&](int s, int64_t stride) {
+    box_row_offsets(a, tl, bx, box_seg(bx, s), static_cast<uint32_t>(stride * sizeof(S)), s_row);
+  };
+  auto row_off = [&](int v) { return s_row[v]; };
+  // extra keys: row g of the sample
+  const int G = XK ? a.G : 0, Gp = (G + 31) & ~31;
+  const int64_t D = static_cast<int64_t>(a.nh) * hd;
+  auto extra_rows = [&](const void* base) {
+    const S* p = static_cast<const S*>(base) + tl.b * static_cast<int64_t>(G) * D +
+                 static_cast<int64_t>(tl.head) * hd;
+    return box_rows(p, ((G - 1) * D + hd) * static_cast<int64_t>(sizeof(S)));
+  };
+  auto extra_off = [&](int g) {
+    return g < G ? static_cast<uint32_t>(g * static_cast<int>(D * sizeof(S))) : kNoRow;
+  };
+  constexpr int NB = box_score_blocks<HD, E>();
+
+  // ---- scores ---------------------------------------------------------------
+  float sc[kSlots];
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) sc[i] = 0.0f;
+  {
+    const __amdgpu_buffer_rsrc_t kr = rows_of(a.k, a.ks);
+#pragma nounroll
+    for (int s = 0; s < bx.n; ++s) {
+      set_rows(s, a.ks);
+      box_scores<HD, S, E, RG, NB>(tl, kr, row_off, bx.nv, hd, qx, s_val);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kSlots; ++i) {
+        if (kSubs * i >= a.K) continue;
+        if (!box_in(tp, i, bx.n > 1 ? s : -1)) continue;
+        const BoxTap t = box_tap(tp, i);
+        sc[i] = box_gather(s_val, t.at, bx.cx, bx.sz, t.fx, t.fy, t.fz);
+      }
+      __syncthreads();  // the next piece, the extra keys or the weights take the table
+    }
+  }
+
+  // ---- extra keys (attention.py:160-173): lane `sub` of a query takes keys
+  // sub + 32 j ------------------------------------------------------------------
+  constexpr int EPL = XK ? kMaxExtra / kSubs : 1;
+  float se[EPL];
+  if constexpr (XK) {
+    box_scores<HD, S, E, RG, NB>(tl, extra_rows(a.ek), extra_off, Gp, hd, qx, s_val);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const int g = tl.sub + kSubs * j;
+      se[j] = g < G ? s_val[tl.q * kBoxRow + g] * a.softmax_scale : -INFINITY;
+    }
+  }
+
+  // ---- softmax over each query's taps (32 lanes x kSlots) and extra keys ----
+  auto has_tap = [&](int i) { return tl.q_ok && tl.sub + kSubs * i < a.K; };
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) {
+    sc[i] = has_tap(i) ? sc[i] * a.softmax_scale : -INFINITY;
+    mx = fmaxf(mx, sc[i]);
+  }
+  if constexpr (XK) {
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) mx = fmaxf(mx, se[j]);
+  }
+  mx = half_reduce<true>(mx);
+  float den = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) {
+    sc[i] = has_tap(i) ? __expf(sc[i] - mx) : 0.0f;
+    den += sc[i];
+  }
+  if constexpr (XK) {
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      se[j] = tl.sub + kSubs * j < G ? __expf(se[j] - mx) : 0.0f;
+      den += se[j];
+    }
+  }
+  den = half_reduce<false>(den);
+  const float inv_den = 1.0f / den;
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) {
+    // p times its dropout factor, in fixed-point units
+    const float f = !DROP ? 1.0f : ((tp.flags >> (4 * i)) & 8u) ? 0.0f : a.drop.scale;
+    sc[i] *= inv_den * f * a.fix_a;
+  }
+  if (tl.sub == 0) {
+    s_qnan[tl.q] = den == den ? 1.0f : __builtin_nanf("");
+    if (lse != nullptr && tl.q_ok) lse[tl.qn * a.nh + tl.head] = mx + logf(den);
+  }
+  if constexpr (XK) {
+    // the keys' weights, in fixed-point units
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const int g = tl.sub + kSubs * j;
+      se[j] = g < G ? se[j] * inv_den * a.fix_a *
+                            (DROP ? dropout_factor(a.drop, tl.qn, tl.head, a.K + g) : 1.0f)
+                      : 0.0f;
+    }
+  }
+
+  // ---- weighted sum: the waves split the voxels, and their partial sums meet in
+  // the table's memory at the end ------------------------------------------------
+  const __amdgpu_buffer_rsrc_t vr = rows_of(a.v, a.vs);
+  f32x4_t acc[HD / 16];
+#pragma unroll
+  for (int t = 0; t < HD / 16; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto weighted = [&](__amdgpu_buffer_rsrc_t r, const auto& off, int n, BoxAhead<HD, E>& ah) {
+    if constexpr (SAFE)
+      box_weighted_safe<HD, S, E, RG>(tl, r, off, n, hd, s_tab, acc);
+    else
+      box_weighted<HD, S, E, RG, false>(tl, r, off, n, hd, s_tab, ah, acc);
+  };
+  if constexpr (XK) {
+    __syncthreads();  // every lane has read its extra keys' scores
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      if (tl.sub + kSubs * j < Gp)
+        s_tab[tl.q * kBoxRow + tl.sub + kSubs * j] =
+            SAFE && tl.sub + kSubs * j < G ? max(to_fix(se[j]), 1) : to_fix(se[j]);
+    __syncthreads();
+    BoxAhead<HD, E> ah;
+    box_weighted_begin<HD, S, E>(tl, extra_rows(a.ev), extra_off, Gp, ah);
+    weighted(extra_rows(a.ev), extra_off, Gp, ah);
+    __syncthreads();
+  }
+  auto piece = [&](int s) {
+    if (s >= 0 || a.vs != a.ks) set_rows(max(s, 0), a.vs);  // else as the scores left them
+    BoxAhead<HD, E> ah;
+    box_weighted_begin<HD, S, E>(tl, vr, row_off, bx.nv, ah);
+    box_zero(s_tab, ((bx.nv + 31) & ~31) >> 2);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      if (kSubs * i >= a.K) continue;
+      if (!box_in(tp, i, s)) continue;
+      const BoxTap t = box_tap(tp, i);
+      if (SAFE && !has_tap(i)) continue;  // (a copy of another lane's tap)
+      box_scatter<SAFE>(s_tab, t.at, bx.cx, bx.sz, t.fx, t.fy, t.fz, sc[i]);
+    }
+    __syncthreads();
+    weighted(vr, row_off, bx.nv, ah);
+    __syncthreads();  // the products have read the table
+  };
+  if (bx.n == 1) {  // the usual case apart: no tap stays live through its products
+    piece(-1);
+  } else {
+#pragma nounroll
+    for (int s = 0; s < bx.n; ++s) piece(s);
+  }
+  // partial O of wave w: [w][query][channel]
+  static_assert(kWaves * kTQ * HD <= kTQ * kBoxRow, "the partial sums fit the table");
+#pragma unroll
+  for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      s_val[(tl.wave * kTQ + 4 * (tl.lane >> 4) + r) * HD +
+            box_channel<HD, E>(t, tl.lane & 15)] = acc[t][r];
+  __syncthreads();
+  bool bad = false;
+#pragma unroll
+  for (int e0 = 0; e0 < kTQ * HD; e0 += kThreads) {
+    const int e = e0 + static_cast<int>(tid);
+    float o = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) o += s_val[w * kTQ * HD + e];
+    bad |= !__builtin_isfinite(o);
+    const int m = e / HD, ch = e - m * HD;
+    const int64_t n = tile_row(a, tl, m);
+    if (n >= 0 && (!RG || ch < hd))
+      out[n * D + tl.head * hd + ch] = from_f32<S>(o * a.fix_a_inv * s_qnan[m]);
+  }
+  return bad;
+}
+
+// A non-finite sum means that a V row of the tile's box holds a non-finite value,
+// which the products spread: to queries of the tile that do not sample the row
+// and (bf16) over its channels.  The tile is then done again with the sum by
+// plain arithmetic over what each query samples (from the start, so that nothing
+// is kept live for it).  Whole-head fp32 products (32, 64, 96, 128) go without.
+template <int HD, typename S, typename E, bool XK, bool RG, bool DROP>
+__global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_box_kernel(
+    Args a, S* __restrict__ out, float* __restrict__ lse, int hd) {
+  __shared__ __attribute__((aligned(16))) int s_tab[kTQ * kBoxRow];
+  __shared__ uint32_t s_row[kBoxCap];
+  __shared__ int s_box[8];
+  __shared__ int s_bad;
+  // per query: 1, or NaN when a score is not finite (its output is NaN then, as
+  // softmax makes it in the reference; the fixed-point weights alone would drop it)
+  __shared__ float s_qnan[kTQ];
+  if (box_unit(a) < 0) return;  // the grid is rounded up to the 8 XCDs
+  constexpr bool kCheck = sizeof(E) == 2 || RG;
+  if (kCheck && threadIdx.x == 0) s_bad = 0;
+  const bool bad = fwd_tile<HD, S, E, XK, RG, DROP, false>(a, out, lse, hd, threadIdx.x, s_tab,
+                                                            s_row, s_box, s_qnan);
+  if constexpr (kCheck) {
+    if (__builtin_amdgcn_ballot_w64(bad) != 0 && (threadIdx.x & 63) == 0) s_bad = 1;
+    __syncthreads();
+    if (s_bad == 0) return;
+    // nothing of the first pass is kept for the second, the arguments included
+    struct KernArgs {
+      Args a;
+      S* out;
+      float* lse;
+      int hd;
+    };
+    unsigned tid = threadIdx.x;
+    auto kp = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+v"(tid), "+s"(kp));
+    KernArgs k;
+    __builtin_memcpy(&k, (const void*)kp, sizeof(k));
+    fwd_tile<HD, S, E, XK, RG, DROP, true>(k.a, k.out, k.lse, k.hd, tid, s_tab, s_row, s_box,
+                                           s_qnan);
+  }
+}
+
+template <typename S, typename E, bool RG>
+hipError_t fwd_typed(const msd_dsa3d_desc& d, const Args& a, void* out, float* lse, hipStream_t s) {
+  const dim3 grid(box_grid(d.B, d.T, d.H, d.W, d.num_heads));
+  const dim3 block(kThreads);
+  S* const o = static_cast<S*>(out);
+  auto go = [&]<int HD>() {
+    auto run = [&]<bool XK, bool DROP>() {
+      hipLaunchKernelGGL((dsa3d_fwd_box_kernel<HD, S, E, XK, RG, DROP>), grid, block, 0, s, a, o,
+                         lse, d.head_dim);
+    };
+    const bool drop = a.drop.threshold != 0;
+    if (a.G > 0) drop ? run.template operator()<true, true>() : run.template operator()<true, false>();
+    else drop ? run.template operator()<false, true>() : run.template operator()<false, false>();
+  };
+  if (d.head_dim <= 32) go.template operator()<32>();
+  else if (d.head_dim <= 64) go.template operator()<64>();
+  else if (d.head_dim <= 96) go.template operator()<96>();
+  else go.template operator()<128>();
+  return hipGetLastError();
+}
+
+}  // namespace
+
+}  // namespace msd

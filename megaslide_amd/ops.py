@@ -194,7 +194,7 @@ def _core_bwd_op(q: Tensor, k: Tensor, v: Tensor, offsets: Tensor, extra_k: Opti
     dek = torch.empty_like(call.ek) if has_extra else q.new_empty((0,))
     dev_ = torch.empty_like(call.ev) if has_extra else q.new_empty((0,))
     lib = _lib.load()
-    ws_bytes = lib.msd_dsa3d_bwd_workspace_size(ctypes.byref(desc))
+    ws_bytes = lib.msd_dsa3d_bwd_best_workspace_size(ctypes.byref(desc))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
         _lib.check(lib.msd_dsa3d_bwd(
