@@ -24,7 +24,7 @@ LIB_NAME = "libmegaslide_dsa3d.so"
 OBJ_DIR = os.path.join(ROOT, "_build", "obj")
 
 SOURCES = ["abi.hip", "dsa3d_direct.hip", "dsa3d_fwd.hip", "dsa3d_ragged.hip",
-           "dsa3d_tiled.hip", "dwconv3d.hip"]
+           "dsa3d_bwd1.hip", "dsa3d_tiled.hip", "dwconv3d.hip"]
 
 ARCH = os.environ.get("MSD_OFFLOAD_ARCH", "gfx950")
 

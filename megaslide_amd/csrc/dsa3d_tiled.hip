@@ -1,21 +1,14 @@
-// Matrix-core (tiled) 3D-DSA forward and backward for gfx950: bf16 or fp32
-// storage, fp32 accumulation, head_dim 32, 64, 96 or 128.
-//
-// One workgroup = one (batch, head, tile of 16 queries).  Instead of gathering
-// the 8 corner rows of K and V for each of a query's taps, it builds dense
-// tables on the matrix cores over the bounding box of the tile's corners, one
-// z-plane (and 16x16 chunk) at a time:
-//   pass 1:  S[q][v] = q . K[v]  (MFMA)  ->  per tap s = scale * sum_c w_c S[q][c]
-//   softmax over each query's taps in registers (wave reductions)
-//   pass 2:  A[q][v] = sum over taps/corners landing on v of p * w  (LDS atomics)
-//            O[q] += A[q] . V  (MFMA, V chunk staged transposed in LDS)
-// This equals the reference's grid_sample + matmul + softmax + matmul
-// (infinity/video/attention.py:106-186) because trilinear sampling is linear in
-// the sampled rows.  Coordinates and corner choice round exactly as the fp32
-// reference does (div_rn, dsa3d_coords.h).
+// Matrix-core (tiled) 3D-DSA backward for gfx950: dq, dK and dV (and the extra
+// keys' gradients) after the first kernel (dsa3d_bwd1.hip), and the launches of
+// the whole backward; bf16 or fp32 storage, fp32 accumulation, head_dim 32, 64,
+// 96 or 128.
+//   dq[q] = sum_v B[q][v] K[v],  dK[v] = sum_q B[q][v] q,  dV[v] = sum_q A[q][v] dO[q]
+// with A = p * w and B = ds * scale * w scattered into LDS tables (integer adds)
+// per plane of the corner box, the products on the matrix cores.
 #include <algorithm>
 #include <type_traits>
 
+#include "dsa3d_bwd1.h"
 #include "dsa3d_tiled_common.h"
 
 namespace msd {
@@ -32,432 +25,6 @@ template <typename E>
 __device__ __forceinline__ op_t<E> table_t_rows(const int* table_t, int row, int col0, int vb,
                                                 int lane) {
   return fix_to_op<E>(&table_t[(32 * vb + (lane & 31)) * row + col0 + 8 * (lane >> 5)]);
-}
-
-// Zero block after each first-backward table: covers a slot's largest corner
-// index dy + dx = 32 (floats; a multiple of 4 keeps the next table 16-byte
-// aligned).
-constexpr int kP1Zero = 36;
-constexpr int kP1Tab = kTQ * kSRow + kP1Zero;
-
-// First backward kernel (one frame, 16 queries): pass 1 of the backward.  It
-// rebuilds S and dP = dO V^T per plane, accumulates per tap s, dp and their
-// coordinate derivatives, then writes the offset gradients and, for the second
-// kernel, p times its dropout factor and ds * softmax_scale of every tap (fp32,
-// [token][head][tap]).
-// Waves per SIMD of the first backward kernel.  bf16 fits 128 registers, so
-// two workgroups share a CU and each hides the other's latencies (barriers,
-// table loads): q and dO then stay in LDS and K/V rows are loaded at the step
-// (at head_dim 128 in two 64-channel halves per table block).  fp32 keeps q/dO
-// in registers and prefetches the next step's rows, at one workgroup per CU.
-template <int HD, typename E>
-constexpr int p1_min_waves() {
-  return sizeof(E) == 2 || HD == 64 ? 4 : 2;
-}
-
-// AE: bytes of one dK / dV accumulator element (4 = fp32 rows, 2 = scaled fp16).
-// REC: also write the tap records, tile header and transposed q / dO of the
-// column-streaming kernel (bf16 storage).
-template <int HD, typename E, int AE, bool REC = false>
-__global__ __launch_bounds__(kThreads, (p1_min_waves<HD, E>())) void dsa3d_bwd_p1_kernel(
-    Args a, const E* __restrict__ out, const E* __restrict__ dout,
-    const float* __restrict__ lse, const float* __restrict__ dlse, E* __restrict__ doff,
-    float* __restrict__ p_ws, float* __restrict__ b_ws, void* __restrict__ dk_acc,
-    void* __restrict__ dv_acc, int64_t acc_ks, int64_t acc_vs, RecArgs rc) {
-  static_assert(!REC || (sizeof(E) == 2 && p1_min_waves<HD, E>() == 4),
-                "records come from the bf16 kernel that stages q and dO in LDS");
-  // S and dP tables, double-buffered (one barrier per plane).  A buffer is
-  // [S rows | zeros | dP rows | zeros]: a slot that misses the step reads the
-  // zero block instead of its corners, so its values are 0 with no select, and
-  // dP sits a constant kP1Tab floats past S (immediate offsets on the reads).
-  __shared__ __attribute__((aligned(16))) float s_tb[2][2 * kP1Tab];
-  __shared__ int s_red[kWaves][6];
-  // record bins (REC): counts, then starts
-  __shared__ int s_bin[REC ? 2 * kRecBins : 1];
-  if (REC && threadIdx.x < kRecBins) s_bin[threadIdx.x] = 0;  // ordered by the setup's barrier
-  constexpr bool kTwoWg = p1_min_waves<HD, E>() == 4;
-  // [query][channel] row of the staged q and dO (elements): HD / 2 + 8 words makes
-  // the MFMA operand reads (lane l: query l % 16, 8 channels from 8 (l / 16))
-  // bank-conflict-free on gfx950 (64 banks, 16-lane passes for 16-byte reads)
-  constexpr int XR = HD + 16;
-  __shared__ __attribute__((aligned(16))) word_t<E> s_x[kTwoWg ? 2 * kTQ * XR : 1];
-
-  const Tile tl = make_tile<1, kSubs>(a);
-  const int D = a.nh * HD;
-  // The tile's q and dO rows (staged in LDS, or held as MFMA operands) are
-  // loaded first, so that the slot setup's arithmetic covers their latency.
-  constexpr int XCPR = HD * static_cast<int>(sizeof(E)) / 16;  // 16-byte pieces of a row
-  constexpr int kXItems = 2 * kTQ * XCPR, kXIPT = kTwoWg ? (kXItems + kThreads - 1) / kThreads : 1;
-  uint4 xst[kXIPT];
-  op_t<E> qx[HD / 32], gx[HD / 32];
-  if constexpr (kTwoWg) {
-    // item e: q (t = 0) or dO (t = 1) row m, 16 bytes from channel ch
-#pragma unroll
-    for (int j = 0; j < kXIPT; ++j) {
-      const int e = threadIdx.x + kThreads * j;
-      const int t = e / (kTQ * XCPR), m = (e / XCPR) % kTQ, ch = (e % XCPR) * (16 / sizeof(E));
-      const int64_t row = e < kXItems ? tile_row(a, tl, m) : -1;
-      xst[j] = uint4{0u, 0u, 0u, 0u};
-      if (row >= 0) {
-        const E* src = t == 0 ? static_cast<const E*>(a.q) + row * a.qs : dout + row * D;
-        xst[j] = *reinterpret_cast<const uint4*>(src + tl.head * HD + ch);
-      }
-    }
-  } else {
-    load_rows_operand<HD, E>(a, tl, static_cast<const E*>(a.q), a.qs, qx);
-    load_rows_operand<HD, E>(a, tl, dout, D, gx);
-  }
-  Slot sl[kSlots];
-  Box box;
-  setup_slots<E, kSubs, kSlots>(a, tl, sl, box, s_red, true);
-  const int nchunks = box.ncy * box.ncx;
-  const int nit = (box.zhi - box.zlo + 1) * nchunks;
-  const E* const kp = static_cast<const E*>(a.k);
-  const E* const vp = static_cast<const E*>(a.v);
-  for (int e = threadIdx.x; e < 2 * 2 * kP1Zero; e += kThreads)
-    s_tb[e / (2 * kP1Zero)][((e / kP1Zero) & 1) * kP1Tab + kTQ * kSRow + e % kP1Zero] = 0.0f;
-  {
-    // The second kernel adds dK and dV into accumulator rows (the fp32 outputs
-    // for fp32 storage, fp32 or scaled fp16 rows for bf16): zero this tile's
-    // rows of the head first (the tiles of a launch partition the (token, head)
-    // pairs, and the second kernel starts after this one ends), 16 bytes a thread.
-    constexpr int CPR = HD * AE / 16;
-    for (int e = threadIdx.x; e < 2 * kTQ * CPR; e += kThreads) {
-      const int t = e / (kTQ * CPR), m = (e / CPR) % kTQ, ch = (e % CPR) * (16 / AE);
-      const int64_t row = tile_row(a, tl, m);
-      if (row < 0) continue;
-      const int64_t el = row * (t == 0 ? acc_ks : acc_vs) + tl.head * HD + ch;
-      char* dst = static_cast<char*>(t == 0 ? dk_acc : dv_acc) + el * AE;
-      *reinterpret_cast<uint4*>(dst) = uint4{0u, 0u, 0u, 0u};
-    }
-  }
-
-  if constexpr (kTwoWg) {
-#pragma unroll
-    for (int j = 0; j < kXIPT; ++j) {
-      const int e = threadIdx.x + kThreads * j;
-      if (e >= kXItems) continue;
-      const int t = e / (kTQ * XCPR), m = (e / XCPR) % kTQ, ch = (e % XCPR) * (16 / sizeof(E));
-      *reinterpret_cast<uint4*>(&s_x[(t * kTQ + m) * XR + ch]) = xst[j];
-    }
-    __syncthreads();
-  }
-  // MFMA A operand of staged row block t (q or dO): lane l holds channels
-  // 32 c + 8 (l / 16) + [0, 8) of query l % 16
-  auto staged_x = [&](int t, op_t<E> (&x)[HD / 32]) {
-#pragma unroll
-    for (int cc = 0; cc < HD / 32; ++cc)
-      x[cc] = load_op<E>(&s_x[(t * kTQ + (tl.lane & 15)) * XR + 32 * cc + 8 * (tl.lane >> 4)]);
-  };
-
-  // Delta = dO . O - dlse and lse for this lane's query.  dO . O = sum_k p_k f_k
-  // dP_k over the query's taps (formed in fp32 after the plane walk) plus, with
-  // extra keys, the same sum over the keys (formed by their kernel before this
-  // one): neither sees the rounding of the stored output (bf16 storage), which
-  // a peaked softmax would otherwise turn into ds errors as large as ds itself.
-  float delta = 0.0f, lse_q = 0.0f;
-  if (tl.q_ok) {
-    // with extra keys: their sum of p f dP (their kernel ran first)
-    if (a.G > 0) delta = a.dlt[tl.qn * a.nh + tl.head];
-    lse_q = lse[tl.qn * a.nh + tl.head];
-  }
-  if (dlse != nullptr && tl.q_ok) delta -= dlse[tl.qn * a.nh + tl.head];
-  // kept in LDS across the plane loop (registers are the limit there)
-  __shared__ float s_dl[kTQ][2];
-  if (tl.sub == 0) {
-    s_dl[tl.q][0] = delta;
-    s_dl[tl.q][1] = lse_q;
-  }
-
-  // ---- pass 1: per tap, the interpolated S and dP and their coordinate
-  // derivatives (x, y within a plane; z across planes) -------------------------
-  float s_[kSlots], dp_[kSlots], gxs[kSlots], gxd[kSlots], gys[kSlots], gyd[kSlots], gzs[kSlots],
-      gzd[kSlots];
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i)
-    s_[i] = dp_[i] = gxs[i] = gxd[i] = gys[i] = gyd[i] = gzs[i] = gzd[i] = 0.0f;
-  // K and V rows of the next (plane, chunk) are loaded while the current one is
-  // used.  fp32 rows beyond head_dim 64 would spill that way: they are loaded
-  // at the step, one 16-voxel block at a time.
-  constexpr bool kPrefetch = !kTwoWg && (sizeof(E) == 2 || HD == 64);
-  TableRows<HD, E> rk, rv;
-  Walk w = walk_begin(box);
-  if (kPrefetch && nit > 0) {
-    load_table_rows<HD, E>(a, tl, w.c, w.z, kp, a.ks, rk);
-    load_table_rows<HD, E>(a, tl, w.c, w.z, vp, a.vs, rv);
-  }
-  for (int it = 0; it < nit; ++it) {
-    const Walk wn = walk_next(box, w);
-    const Chunk& c = w.c;
-    const int z = w.z;
-    // buffer it & 1 was last read for step it - 2, before the previous barrier
-    float* const tb = s_tb[it & 1];
-    if constexpr (kPrefetch) {
-      store_table<HD, E>(tl, c, qx, rk, tb);
-      store_table<HD, E>(tl, c, gx, rv, tb + kP1Tab);
-      if (it + 1 < nit) {
-        load_table_rows<HD, E>(a, tl, wn.c, wn.z, kp, a.ks, rk);
-        load_table_rows<HD, E>(a, tl, wn.c, wn.z, vp, a.vs, rv);
-      }
-    } else {
-      const char* ko = head_origin<HD, E>(a, tl, c, z, kp, a.ks);
-      const char* vo = head_origin<HD, E>(a, tl, c, z, vp, a.vs);
-#pragma nounroll
-      for (int j = 0; j < 2; ++j) {
-        if constexpr (kTwoWg && HD * sizeof(E) == 256) {
-          // S and dP of block j over two channel halves (bf16 head_dim 128,
-          // fp32 64): a half's K/V rows and q/dO operands are HD / 64
-          // operands each (registers are the limit)
-          constexpr int OPH = HD / 64, CH = HD / 2;
-          const int blk = tl.wave + kWaves * j;
-          if (blk * 16 >= c.nv) continue;  // wave-uniform: no voxel of the block
-          const int vi = blk * 16 + (tl.lane & 15);
-          const bool v_ok = vi < c.nv;
-          const int lc = 8 * (tl.lane >> 4);
-          const E* const pk = chunk_voxel<E>(ko, a, c, a.ks, lc, v_ok ? vi : 0);
-          const E* const pv = chunk_voxel<E>(vo, a, c, a.vs, lc, v_ok ? vi : 0);
-          f32x4_t as = {0.0f, 0.0f, 0.0f, 0.0f}, ad = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            op_t<E> yk[OPH], yv[OPH];
-#pragma unroll
-            for (int cc = 0; cc < OPH; ++cc) {
-              yk[cc] = yv[cc] = zero_op<E>();
-              if (v_ok) {
-                yk[cc] = load_op<E>(pk + CH * h + 32 * cc);
-                yv[cc] = load_op<E>(pv + CH * h + 32 * cc);
-              }
-            }
-            const word_t<E>* const xq = &s_x[(tl.lane & 15) * XR + CH * h + lc];
-            const word_t<E>* const xo = xq + kTQ * XR;
-#pragma unroll
-            for (int cc = 0; cc < OPH; ++cc) {
-              as = mma16(load_op<E>(xq + 32 * cc), yk[cc], as);
-              ad = mma16(load_op<E>(xo + 32 * cc), yv[cc], ad);
-            }
-          }
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            tb[(4 * (tl.lane >> 4) + rr) * kSRow + vi] = as[rr];
-            tb[kP1Tab + (4 * (tl.lane >> 4) + rr) * kSRow + vi] = ad[rr];
-          }
-          continue;
-        }
-        load_block_rows<HD, E>(a, tl, c, ko, a.ks, j, rk.y[0]);
-        load_block_rows<HD, E>(a, tl, c, vo, a.vs, j, rv.y[0]);
-        if constexpr (kTwoWg) {
-          op_t<E> x[HD / 32];
-          staged_x(0, x);
-          store_table_block<HD, E>(tl, c, x, rk.y[0], j, tb);
-          staged_x(1, x);
-          store_table_block<HD, E>(tl, c, x, rv.y[0], j, tb + kP1Tab);
-        } else {
-          store_table_block<HD, E>(tl, c, qx, rk.y[0], j, tb);
-          store_table_block<HD, E>(tl, c, gx, rv.y[0], j, tb + kP1Tab);
-        }
-      }
-    }
-    __syncthreads();
-    // a hit reads its 4 corners in both tables; a miss reads the zero block
-    // (never stale entries, which may be non-finite) and has wz = dwz = 0.  A
-    // slot that no lane of the wave hits (about a third of them) is skipped.
-    const float* const r0 = &tb[tl.q * kSRow];
-    const float* const zr = &tb[kTQ * kSRow];
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      float wz, dwz;
-      const bool hit = slot_weight(sl[i], step_key(c.id, z), wz, dwz);
-      if (__builtin_amdgcn_ballot_w64(hit) == 0) continue;
-      const int base = sl[i].idx & 0x1ff, dy = (sl[i].idx >> 9) & 0x1f, dx = (sl[i].idx >> 14) & 1;
-      const float* const ps = hit ? r0 + base : zr;
-      const float* const pd = ps + kP1Tab;
-      const Bilerp bs = bilerp(sl[i], ps[0], ps[dx], ps[dy], ps[dy + dx]);
-      const Bilerp bd = bilerp(sl[i], pd[0], pd[dx], pd[dy], pd[dy + dx]);
-      s_[i] = __builtin_fmaf(wz, bs.val, s_[i]);
-      gxs[i] = __builtin_fmaf(wz, bs.dx, gxs[i]);
-      gys[i] = __builtin_fmaf(wz, bs.dy, gys[i]);
-      gzs[i] = __builtin_fmaf(dwz, bs.val, gzs[i]);
-      dp_[i] = __builtin_fmaf(wz, bd.val, dp_[i]);
-      gxd[i] = __builtin_fmaf(wz, bd.dx, gxd[i]);
-      gyd[i] = __builtin_fmaf(wz, bd.dy, gyd[i]);
-      gzd[i] = __builtin_fmaf(dwz, bd.val, gzd[i]);
-    }
-    w = wn;
-  }
-
-  // p = exp(scale * s - lse), ds = p (dp - Delta).  The coordinate gradient of
-  // a tap is ds*scale*dS/du + p*dP/du; chain it through the clamp mask, the
-  // unnormalisation (S/2), the slot divisor and offset_scale into d offsets.
-  const float cxs = a.gsx, cys = a.gsy, czs = a.gsz;
-  // the query's token row and the taps' offsets are recomputed here from the
-  // wave (a scalar) and the lane id: kept from before the plane loop, they
-  // spill (as does the thread index register)
-  const int tid = 64 * __builtin_amdgcn_readfirstlane(tl.wave) +
-                  static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
-  const int sub = tid % kSubs;
-  const int64_t qn = tile_row(a, tl, tid / kSubs);
-  const int64_t tap0 = (qn * a.nh + tl.head) * a.K;
-  delta = s_dl[tid / kSubs][0];  // written before the loop's first barrier
-  lse_q = s_dl[tid / kSubs][1];
-  // p of every tap (0 for empty slots) in place of s.  Dropout: o sums
-  // pd * v_s with pd = p * factor, so dp and the V-side coordinate gradient
-  // see the factor.
-  float pdp = 0.0f;  // sum_k p_k f_k dP_k over this lane's taps
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) {
-    const bool ok = slot_z0(sl[i]) >= 0;
-    s_[i] = ok ? __expf(s_[i] * a.softmax_scale - lse_q) : 0.0f;
-    pdp = __builtin_fmaf(s_[i] * slot_dropout(sl[i], a.drop), dp_[i], pdp);
-  }
-#pragma unroll
-  for (int m = 1; m < kSubs; m <<= 1) pdp += __shfl_xor(pdp, m);
-  delta += pdp;
-  // the whole Delta for the extra keys' kernel that runs next (each query's
-  // entry is read above and written here by this workgroup only)
-  if (a.G > 0 && sub == 0 && qn >= 0) a.dlt[qn * a.nh + tl.head] = delta;
-  // p * factor in place of p, ds * scale = p (f dP - Delta) scale in place of dp
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) {
-    const float dfac = slot_dropout(sl[i], a.drop);
-    dp_[i] = s_[i] * (dfac * dp_[i] - delta) * a.softmax_scale;
-    s_[i] *= dfac;
-  }
-  // bf16 storage keeps one word per tap: fp16 p * factor and ds * scale / l1,
-  // with l1 = sum over the query's taps of |ds * scale| kept per token and head
-  // (the normalised values lie in [-1, 1], where fp16 keeps 11 bits)
-  float rl1 = 1.0f, l1q = 0.0f;
-  if constexpr (sizeof(E) == 2) {
-    float l1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) l1 += fabsf(dp_[i]);
-#pragma unroll
-    for (int m = 1; m < kSubs; m <<= 1) l1 += __shfl_xor(l1, m);
-    rl1 = l1 > 1e-30f ? 1.0f / l1 : 0.0f;
-    l1q = l1;
-    if (sub == 0 && qn >= 0) b_ws[qn * a.nh + tl.head] = l1;
-  }
-  // Records for the column-streaming kernel (REC), counting-sorted by z0: the
-  // bins' counts by LDS atomics (their return values place each record in its
-  // bin), then one thread's prefix sum.  Within a bin the order is the
-  // atomics' order, which no result depends on (the consumer sums integers).
-  int pos[kSlots];
-  const bool rec_wide = REC && !(box.zhi < box.zlo) && box.zhi - box.zlo + 1 > kRecBins;
-  if constexpr (REC) {
-    const int64_t trec = static_cast<int64_t>(tl.head) * rc.tiles +
-                         rec_tile(a, tl.b, tl.t0, tl.h0 / kTileH, tl.w0 / kTileW);
-    // the column list's count and, after the list, the 8 work counters of the
-    // column-streaming kernel
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 9)
-      rc.collist[threadIdx.x == 0 ? 0 : a.nh * a.B * a.tiles_h * a.tiles_w + threadIdx.x] = 0;
-    const int nb = box.zhi < box.zlo ? 0 : box.zhi - box.zlo + 1;
-    if (sub == 0) s_dl[tid / kSubs][0] = l1q;  // this query's l1 (delta was read above)
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      pos[i] = 0;
-      if (!rec_wide && slot_z0(sl[i]) >= 0)
-        pos[i] = atomicAdd(&s_bin[slot_z0(sl[i]) - box.zlo], 1);
-    }
-    __syncthreads();
-    // exclusive prefix of the 16 counts in wave 0 (lane bb holds bin bb)
-    if (threadIdx.x < 64) {
-      const int bb = threadIdx.x & (kRecBins - 1);
-      const int cnt = threadIdx.x < kRecBins ? s_bin[bb] : 0;
-      int inc = cnt;
-#pragma unroll
-      for (int m = 1; m < kRecBins; m <<= 1) {
-        const int o = __shfl_up(inc, m, kRecBins);
-        if (bb >= m) inc += o;
-      }
-      int* const hdr = rc.hdr + trec * kRecHdr;
-      if (threadIdx.x < kRecBins) {
-        s_bin[kRecBins + bb] = inc - cnt;
-        hdr[8 + bb] = inc - cnt;
-        if (bb == kRecBins - 1) hdr[8 + kRecBins] = inc;
-      }
-      if (threadIdx.x == 0) {
-        hdr[0] = box.zlo;
-        hdr[1] = box.zhi;
-        hdr[2] = box.ylo;
-        hdr[3] = box.yhi;
-        hdr[4] = box.xlo;
-        hdr[5] = box.xhi;
-        hdr[6] = rec_wide ? -1 : nb;
-      }
-    }
-    __syncthreads();
-  }
-  // a record's corner (y0, x0) from the tap's table index in its chunk of
-  // the box; one chunk column (the usual case): the box's x origin and width
-  const bool one_cx = box.ncx == 1;
-  const int nx1 = min(kChunk, box.xhi - box.xlo + 1);
-  const float rnx1 = __builtin_amdgcn_rcpf(static_cast<float>(nx1));
-  u32x4_t* const rec = REC ? rc.rec + (static_cast<int64_t>(tl.head) * rc.tiles +
-                                       rec_tile(a, tl.b, tl.t0, tl.h0 / kTileH, tl.w0 / kTileW)) *
-                                          (static_cast<int64_t>(a.K) * kTQ)
-                           : nullptr;
-#pragma unroll
-  for (int i = 0; i < kSlots; ++i) {
-    if (slot_z0(sl[i]) < 0) continue;
-    const float pd = s_[i], dss = dp_[i];
-    const int kap = sub + kSubs * i;
-    uint32_t pair = 0;
-    if constexpr (sizeof(E) == 4) {
-      p_ws[tap0 + kap] = pd;
-      b_ws[tap0 + kap] = dss;
-    } else {
-      pair = pack_h2(pd, dss * rl1);
-      reinterpret_cast<uint32_t*>(p_ws)[tap0 + kap] = pair;
-    }
-    E* dp = doff + qn * a.C + (static_cast<int64_t>(tl.head) * a.K + kap) * 3;
-    const int m = sl[i].zc >> 17;
-    dp[0] = from_f32<E>((m & 1) ? (dss * gxs[i] + pd * gxd[i]) * cxs : 0.0f);
-    dp[1] = from_f32<E>((m & 2) ? (dss * gys[i] + pd * gyd[i]) * cys : 0.0f);
-    dp[2] = from_f32<E>((m & 4) ? (dss * gzs[i] + pd * gzd[i]) * czs : 0.0f);
-    if constexpr (REC) {
-      if (rec_wide) continue;
-      const int idx = sl[i].idx;
-      const int base = idx & 0x1ff, ch = static_cast<int>(static_cast<uint32_t>(idx) >> 16);
-      int cy = ch, cx0 = box.xlo, nx = nx1;
-      float rnx = rnx1;
-      if (!one_cx) {
-        cy = ch / box.ncx;
-        cx0 = box.xlo + kChunkStep * (ch - cy * box.ncx);
-        nx = min(kChunk, box.xhi - cx0 + 1);
-        rnx = __builtin_amdgcn_rcpf(static_cast<float>(nx));
-      }
-      const int vy = static_cast<int>((static_cast<float>(base) + 0.5f) * rnx);
-      const int y0 = box.ylo + kChunkStep * cy + vy, x0 = cx0 + base - vy * nx;
-      const uint32_t ux = min(65535u, static_cast<uint32_t>(sl[i].fx * 65536.0f + 0.5f));
-      const uint32_t uy = min(65535u, static_cast<uint32_t>(sl[i].fy * 65536.0f + 0.5f));
-      u32x4_t r;
-      r[0] = static_cast<uint32_t>(y0) | (static_cast<uint32_t>(x0) << 14) |
-             (static_cast<uint32_t>(tid / kSubs) << 28);
-      r[1] = ux | (uy << 16);
-      r[2] = __float_as_uint(sl[i].fz);
-      r[3] = pair;
-      rec[s_bin[kRecBins + slot_z0(sl[i]) - box.zlo] + pos[i]] = r;
-    }
-  }
-  if constexpr (REC) {
-    const int64_t trec = static_cast<int64_t>(tl.head) * rc.tiles +
-                         rec_tile(a, tl.b, tl.t0, tl.h0 / kTileH, tl.w0 / kTileW);
-    // q and dO of the tile transposed, with the fixed-point scales of the B
-    // (l1 / 2^30, per query) and A (1 / fix_a) tables: item e = (tensor,
-    // channel, query half) writes 8 queries (16 bytes)
-    E* const qt = static_cast<E*>(rc.qt) + trec * (2 * HD * kTQ);
-    for (int e = threadIdx.x; e < 2 * HD * 2; e += kThreads) {
-      const int t = e / (2 * HD), chn = (e / 2) % HD, h8 = 8 * (e & 1);
-      uint16_t v8[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int m = h8 + j;
-        const float sc = t == 0 ? s_dl[m][0] * kFixAInv : a.fix_a_inv;
-        const uint16_t raw = s_x[(t * kTQ + m) * XR + chn];
-        v8[j] = from_f32<E>(__uint_as_float(static_cast<uint32_t>(raw) << 16) * sc).bits;
-      }
-      __builtin_memcpy(&qt[(t * HD + chn) * kTQ + h8], v8, sizeof(v8));
-    }
-  }
 }
 
 // Second backward kernel: dq, dK and dV for tiles of FR consecutive frames
@@ -2124,14 +1691,13 @@ struct BwdBufs {
 
 template <int HD, typename E>
 void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,
-                     const void* off, const void* ek, const void* ev, const E* o, const E* go,
+                     const void* off, const void* ek, const void* ev, const E* go,
                      const float* lse, const float* dlse, E* gq, E* goff, const BwdBufs<E>& w,
                      hipStream_t s) {
   constexpr int CW = p2_window<HD, E>(), FR = p2_frames<HD, E>();
   tiled::Args a1 = make_tiled_args(d, q, k, v, off, tiled_tiles<1>(d), ek, ev);
   a1.dlt = w.dlt;
   const tiled::Args a2 = make_tiled_args(d, q, k, v, off, tiled_tiles<FR>(d), ek, ev);
-  const dim3 g1 = tiled_grid<1>(d);
   dim3 g2 = tiled_grid<FR>(d);
   g2.z = HD / CW;
   float* const p_ws = w.p_ws;
@@ -2146,9 +1712,8 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
   // and the tile kernel the columns it flags
   if constexpr (sizeof(E) == 2) {
     if (!h16 && w.rec.rec != nullptr) {
-      hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, 4, true>), g1, dim3(tiled::kThreads), 0, s,
-                         a1, o, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs,
-                         w.rec);
+      launch_bwd_p1<HD, E, 4, true>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
+                                    acc_vs, w.rec, s);
       // persistent: one workgroup per CU (each takes a CU's LDS)
       hipLaunchKernelGGL((dsa3d_bwd_p2s_kernel<HD, E>), dim3(device_cus()), dim3(kS2Threads), 0,
                          s, a1, w.rec, b_ws, gq, static_cast<float*>(dk_acc),
@@ -2165,12 +1730,12 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
                        w.dqx, w.ds_e, w.pf_e);
   if constexpr (sizeof(E) == 2) {
     if (h16)
-      hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, 2>), g1, dim3(tiled::kThreads), 0, s, a1, o,
-                         go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, RecArgs{});
+      launch_bwd_p1<HD, E, 2, false>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
+                                     acc_vs, RecArgs{}, s);
   }
   if (!h16)
-    hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, 4>), g1, dim3(tiled::kThreads), 0, s, a1, o,
-                       go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, RecArgs{});
+    launch_bwd_p1<HD, E, 4, false>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
+                                   acc_vs, RecArgs{}, s);
   if (d.extra_g > 0)
     hipLaunchKernelGGL((dsa3d_bwd_extra_kernel<HD, E, false>), gx, dim3(256), 0, s, a1, go, lse,
                        w.dqx, w.ds_e, w.pf_e);
@@ -2320,7 +1885,6 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
   const int64_t rows = static_cast<int64_t>(d.B) * d.T * d.H * d.W;
   const int D = d.num_heads * d.head_dim;
   const int64_t erows = static_cast<int64_t>(d.B) * d.extra_g;
-  const auto* o = static_cast<const E*>(out);
   const auto* go = static_cast<const E*>(dout);
   auto* gq = static_cast<E*>(dq);
   auto* goff = static_cast<E*>(doff);
@@ -2365,10 +1929,10 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
                        erows * D);
   }
   switch (d.head_dim) {
-    case 32: launch_bwd_pair<32, E>(d, q, k, v, off, ek, ev, o, go, lse, dlse, gq, goff, w, s); break;
-    case 64: launch_bwd_pair<64, E>(d, q, k, v, off, ek, ev, o, go, lse, dlse, gq, goff, w, s); break;
-    case 96: launch_bwd_pair<96, E>(d, q, k, v, off, ek, ev, o, go, lse, dlse, gq, goff, w, s); break;
-    case 128: launch_bwd_pair<128, E>(d, q, k, v, off, ek, ev, o, go, lse, dlse, gq, goff, w, s); break;
+    case 32: launch_bwd_pair<32, E>(d, q, k, v, off, ek, ev, go, lse, dlse, gq, goff, w, s); break;
+    case 64: launch_bwd_pair<64, E>(d, q, k, v, off, ek, ev, go, lse, dlse, gq, goff, w, s); break;
+    case 96: launch_bwd_pair<96, E>(d, q, k, v, off, ek, ev, go, lse, dlse, gq, goff, w, s); break;
+    case 128: launch_bwd_pair<128, E>(d, q, k, v, off, ek, ev, go, lse, dlse, gq, goff, w, s); break;
     default: return hipErrorInvalidValue;
   }
   if constexpr (!kInPlace) {

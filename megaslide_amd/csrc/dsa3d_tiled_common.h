@@ -1,16 +1,13 @@
 // Shared building blocks of the matrix-core (tiled) 3D-DSA kernels.
 //
-// A workgroup of 8 waves owns one (batch, head, tile of FRAMES consecutive
-// frames x 4 rows x 4 columns of queries).  Thread i serves group query
-// q = i / SUBS (frame q / 16 of the tile, position q % 16) and the taps
-// kappa = (i % SUBS) + SUBS * j, j < SLOTS.  The forward and the first backward
-// kernel use FRAMES = 1, SUBS = 32, SLOTS = 5; the dK/dV/dq kernel FRAMES = 2,
-// SUBS = 16, SLOTS = 10.  Every tap's 2x2 (y, x) corner
-// footprint is resolved against per-plane score tables
-//   S[q][v] = X[q] . Y[v]   (X = q or dO rows, Y = K or V rows; MFMA, fp32 in LDS)
-// built over the (y, x) bounding box of all corners of the tile, cut into
-// 16 x 16 chunks whose starts are 15 voxels apart: two adjacent voxels always
-// share a chunk, so each tap is assigned to exactly one chunk.
+// A workgroup owns one (batch, head, tile of FRAMES consecutive frames x 4 rows x
+// 4 columns of queries).  Thread i serves group query q = i / SUBS (frame q / 16
+// of the tile, position q % 16) and the taps kappa = (i % SUBS) + SUBS * j, j <
+// SLOTS.  The forward and the first backward kernel (dsa3d_box.h: tables of a
+// tile's whole corner box) use FRAMES = 1, SUBS = 32, SLOTS = 5; the dK/dV/dq
+// tile kernel FRAMES = 2 or 3, SUBS = 16, SLOTS = 10 and one table per plane and
+// 16 x 16 chunk of the box: chunk starts are 15 voxels apart, so two adjacent
+// voxels always share a chunk and each tap's 2 x 2 footprint lies in exactly one.
 #pragma once
 
 #include "common.h"
@@ -80,30 +77,6 @@ __device__ __forceinline__ op_t<E> zero_op() {
     const f32x8_t z = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     return z;
   }
-}
-
-// Bytes of one dK / dV accumulator element of the tiled backward: fp16 for
-// bf16 storage (scaled per call, packed-pair atomics), fp32 otherwise.
-template <typename E>
-constexpr int acc_bytes() {
-  return sizeof(E) == 2 ? 2 : 4;
-}
-
-// Largest |x| of an 8-element operand (a NaN element is passed over).
-template <typename E>
-__device__ __forceinline__ float max_abs_op(const op_t<E>& x) {
-  float m = 0.0f;
-  if constexpr (sizeof(E) == 2) {
-    const u32x4_t b = __builtin_bit_cast(u32x4_t, x);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      m = fmaxf(m, fmaxf(fabsf(__uint_as_float(b[i] << 16)),
-                         fabsf(__uint_as_float(b[i] & 0xffff0000u))));
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(x[j]));
-  }
-  return m;
 }
 
 // 8 consecutive elements (16 or 32 bytes) from global memory or LDS.
@@ -203,32 +176,14 @@ __device__ __forceinline__ int64_t rec_tile(const Args& a, int b, int t, int th,
 
 // Geometry of one tap, kept in registers between the passes.
 struct Slot {
-  int zc;    // z0 (bits 0-15, -1 = empty) | hz << 16 | clamp-gradient mask x,y,z << 17..19
-             // | dropped by attention dropout << 20
+  int zc;    // z0 (bits 0-15, -1 = empty) | hz << 16
   int idx;   // table index of corner (y0, x0) | dy_off << 9 | dx_off << 14 | chunk << 16
   float fz;  // weight of the upper z corner
   float fx, fy;  // weights of the upper x / y corners (0 when that corner is outside)
 };
 
-// The slot's words as opaque values at this point: keeps the compiler from
-// hoisting what it derives from them (keys, corner weights and addresses) out
-// of a plane loop, where registers are the limit.  Costs no instruction.
-__device__ __forceinline__ Slot opaque(const Slot& s) {
-  Slot r = s;
-  asm volatile("" : "+v"(r.zc), "+v"(r.idx), "+v"(r.fz), "+v"(r.fx), "+v"(r.fy));
-  return r;
-}
-
 __device__ __forceinline__ int slot_z0(const Slot& s) { return static_cast<int16_t>(s.zc & 0xffff); }
 __device__ __forceinline__ bool slot_hz(const Slot& s) { return (s.zc >> 16) & 1; }
-__device__ __forceinline__ int slot_chunk(const Slot& s) {
-  return static_cast<int>(static_cast<uint32_t>(s.idx) >> 16);
-}
-// Dropout factor of the slot's softmax weight: 1 (off), 0 (dropped) or 1/(1-p).
-__device__ __forceinline__ float slot_dropout(const Slot& s, const DropoutArgs& d) {
-  return d.threshold == 0 ? 1.0f : (((s.zc >> 20) & 1) ? 0.0f : d.scale);
-}
-
 struct Tile {
   int b, head, t0, t, h0, w0;  // t0: first frame of the tile; t: this lane's frame
   int64_t sample0;
@@ -278,11 +233,6 @@ __device__ __forceinline__ Tile make_tile_at(const Args& a, int tile) {
   return t;
 }
 
-template <int FRAMES, int SUBS>
-__device__ __forceinline__ Tile make_tile(const Args& a) {
-  return make_tile_at<FRAMES, SUBS>(a, blockIdx.x);
-}
-
 // Token row of group query m (frame m / 16, position m % 16), or -1 outside the grid.
 __device__ __forceinline__ int64_t tile_row(const Args& a, const Tile& t, int m) {
   const int tt = t.t0 + m / kTQ, s = m % kTQ;
@@ -322,10 +272,9 @@ __device__ __forceinline__ float grid_coord_rn(float base, float o, float div, f
 
 // Tap geometry for all SLOTS slots of this lane (coordinates exactly as the
 // reference rounds them) and the block-wide bounding box of every corner.
-// With `dropout`, each tap's keep decision is drawn here once (bit 20 of zc).
 template <typename E, int SUBS, int SLOTS, int NW = kWaves>
 __device__ __forceinline__ void setup_slots(const Args& a, const Tile& tl, Slot* sl, Box& box,
-                                            int (*s_red)[6], bool dropout = false) {
+                                            int (*s_red)[6]) {
   int zlo = 1 << 30, zhi = -1, ylo = 1 << 30, yhi = -1, xlo = 1 << 30, xhi = -1;
   int y0s[SLOTS], x0s[SLOTS];
   const int qh = tl.qh, qw = tl.qw;
@@ -355,13 +304,7 @@ __device__ __forceinline__ void setup_slots(const Args& a, const Tile& tl, Slot*
                                               a.div_y, a.rdiv_y), a.H);
     const Axis az = axis_sample(grid_coord_rn(base_coord_rn(tl.t, ci, a.bdiv_z, a.rbdiv_z), o2,
                                               a.div_z, a.rdiv_z), a.T);
-    // clamp-gradient masks: zero where u <= 0 or u >= S-1 (grid_sample border padding)
-    const int mx = (ax.u > 0.0f && ax.u < static_cast<float>(a.W - 1)) ? 1 : 0;
-    const int my = (ay.u > 0.0f && ay.u < static_cast<float>(a.H - 1)) ? 1 : 0;
-    const int mz = (az.u > 0.0f && az.u < static_cast<float>(a.T - 1)) ? 1 : 0;
-    sl[i].zc = az.i0 | (az.hi_ok << 16) | (mx << 17) | (my << 18) | (mz << 19);
-    if (dropout && a.drop.threshold != 0 && dropout_factor(a.drop, tl.qn, tl.head, kap) == 0.0f)
-      sl[i].zc |= 1 << 20;
+    sl[i].zc = az.i0 | (az.hi_ok << 16);
     // an upper corner outside the volume only occurs with weight 0 (the
     // coordinate is clamped to S-1), so fx/fy/fz are 0 there
     sl[i].fx = ax.f;
@@ -529,95 +472,13 @@ __device__ __forceinline__ u32x4_t load16(const void* p) {
   return r;
 }
 
-// Rows of the tile (queries m = lane % 16) as MFMA A operands: x[c] holds
-// channels 32*c + 8*(lane/16) + [0, 8), c < HD/32.
-template <int HD, typename E>
-__device__ __forceinline__ void load_rows_operand(const Args& a, const Tile& tl, const E* base,
-                                                  int64_t stride, op_t<E> (&x)[HD / 32]) {
-#pragma unroll
-  for (int c = 0; c < HD / 32; ++c) x[c] = zero_op<E>();
-  const int64_t row = tile_row(a, tl, tl.lane & 15);
-  if (row < 0) return;
-  const E* p = base + row * stride + tl.head * HD + 8 * (tl.lane >> 4);
-#pragma unroll
-  for (int c = 0; c < HD / 32; ++c) x[c] = load_op<E>(p + 32 * c);
-}
-
-// Y rows of 16-voxel block j (< 2) of this wave (block w + 8 j; a chunk has at
-// most 16 blocks) as MFMA B operands: y[c] holds channels 32*c + 8*(lane/16)
-// + [0, 8) of voxel 16*block + lane % 16.
-template <int HD, typename E>
-__device__ __forceinline__ void load_block_rows(const Args& a, const Tile& tl, const Chunk& c,
-                                                const char* origin, int64_t ystride, int j,
-                                                op_t<E> (&y)[HD / 32]) {
-  const int vi = (tl.wave + kWaves * j) * 16 + (tl.lane & 15);
-#pragma unroll
-  for (int cc = 0; cc < HD / 32; ++cc) y[cc] = zero_op<E>();
-  if (vi < c.nv) {
-    const E* p = chunk_voxel<E>(origin, a, c, ystride, 8 * (tl.lane >> 4), vi);
-#pragma unroll
-    for (int cc = 0; cc < HD / 32; ++cc) y[cc] = load_op<E>(p + 32 * cc);
-  }
-}
-
-// The chunk's rows of head tl.head in plane z (wave-uniform origin).
-template <int HD, typename E>
-__device__ __forceinline__ const char* head_origin(const Args& a, const Tile& tl, const Chunk& c,
-                                                   int z, const E* ybase, int64_t ystride) {
-  return chunk_origin(a, tl, c, z, ybase, ystride, tl.head * HD);
-}
-
-// table[m][vi] = X[m] . Y[vi] for the voxels vi of block j of this wave.
-template <int HD, typename E>
-__device__ __forceinline__ void store_table_block(const Tile& tl, const Chunk& c,
-                                                  const op_t<E> (&x)[HD / 32],
-                                                  const op_t<E> (&y)[HD / 32], int j,
-                                                  float* table) {
-  const int blk = tl.wave + kWaves * j;
-  if (blk * 16 >= c.nv) return;
-  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int cc = 0; cc < HD / 32; ++cc) acc = mma16(x[cc], y[cc], acc);
-  const int vi = blk * 16 + (tl.lane & 15);
-#pragma unroll
-  for (int rr = 0; rr < 4; ++rr) table[(4 * (tl.lane >> 4) + rr) * kSRow + vi] = acc[rr];
-}
-
-// Both blocks of the wave, loaded together: all loads are issued before any
-// is used.
-template <int HD, typename E>
-struct TableRows {
-  op_t<E> y[2][HD / 32];  // [block][channels 32*c + kq]
-};
-
-template <int HD, typename E>
-__device__ __forceinline__ void load_table_rows(const Args& a, const Tile& tl, const Chunk& c,
-                                                int z, const E* ybase, int64_t ystride,
-                                                TableRows<HD, E>& r) {
-  const char* origin = head_origin<HD, E>(a, tl, c, z, ybase, ystride);
-#pragma unroll
-  for (int j = 0; j < 2; ++j) load_block_rows<HD, E>(a, tl, c, origin, ystride, j, r.y[j]);
-}
-
-template <int HD, typename E>
-__device__ __forceinline__ void store_table(const Tile& tl, const Chunk& c,
-                                            const op_t<E> (&x)[HD / 32], const TableRows<HD, E>& r,
-                                            float* table) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j) store_table_block<HD, E>(tl, c, x, r.y[j], j, table);
-}
-
 // Chunk rows of Y (plane z), channels col0 + [0, CW), transposed into LDS:
 // yt[channel][voxel] (row stride ElemT<E>::kRow), padded up to nvp voxels
-// with zeros or, with kPadCopies, copies of voxel nv - 1 (loads of every
-// lane, no zeroing; the tables hold 0 for those voxels: 3% faster in the
-// forward, 2-3% slower in the dq/dK/dV kernel), by the first NT = 512 threads
-// of the workgroup.  Thread t moves
+// with zeros, by the first NT = 512 threads of the workgroup.  Thread t moves
 // voxels 2 p + {0, 1} of channel groups q0 + 4 g (8 channels each, g < CW /
 // 32), p = 16 (t >> 6) + (t & 15), q0 = (t >> 4) & 3: a wave's lanes cover 4
 // adjacent channel groups of 16 voxel pairs, so a load touches 16 rows, 32
-// channels of each (64 rows of 8 channels took 4% longer in the forward, 32
-// rows of 16 channels 1.5%).  Its loads are issued first.
+// channels of each.  Its loads are issued first.
 //
 // LDS banks, as measured on gfx950: a 4-byte access is served per half-wave
 // over 32 banks of 4 bytes; a 16-byte read over 64 banks in four passes of 16
@@ -653,35 +514,22 @@ __device__ __forceinline__ int stage_group0() {
   return (stage_tid() >> 4) & 3;
 }
 
-template <int NT, int CW, typename E, bool kPadCopies = false>
+template <int NT, int CW, typename E>
 __device__ __forceinline__ void load_stage_rows(const Args& a, const Tile& tl, const Chunk& c,
                                                 int z, const E* ybase, int64_t ystride,
                                                 int col0, StageRows<NT, CW, E>& r) {
   constexpr int G = StageRows<NT, CW, E>::G;
   const int q0 = stage_group0(), v0 = 2 * stage_pair();
-  if constexpr (kPadCopies) {
-    // threads past NT (a larger workgroup) or past the padded chunk do not
-    // stage (store_stage skips them too)
-    if (threadIdx.x >= NT || v0 >= c.nvp) return;
-    const char* origin = chunk_origin(a, tl, c, z, ybase, ystride, col0);
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const E* p = chunk_voxel<E>(origin, a, c, ystride, 8 * q0, min(v0 + e, c.nv - 1));
+  for (int g = 0; g < G; ++g) r.x[g][0] = r.x[g][1] = zero_op<E>();
+  if (threadIdx.x >= NT) return;  // a larger workgroup: the other threads do not stage
+  const char* origin = chunk_origin(a, tl, c, z, ybase, ystride, col0);
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    if (v0 + e < c.nv) {
+      const E* p = chunk_voxel<E>(origin, a, c, ystride, 8 * q0, v0 + e);
 #pragma unroll
       for (int g = 0; g < G; ++g) r.x[g][e] = load_op<E>(p + 32 * g);
-    }
-  } else {
-#pragma unroll
-    for (int g = 0; g < G; ++g) r.x[g][0] = r.x[g][1] = zero_op<E>();
-    if (threadIdx.x >= NT) return;  // a larger workgroup: the other threads do not stage
-    const char* origin = chunk_origin(a, tl, c, z, ybase, ystride, col0);
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      if (v0 + e < c.nv) {
-        const E* p = chunk_voxel<E>(origin, a, c, ystride, 8 * q0, v0 + e);
-#pragma unroll
-        for (int g = 0; g < G; ++g) r.x[g][e] = load_op<E>(p + 32 * g);
-      }
     }
   }
 }
@@ -728,17 +576,6 @@ __device__ __forceinline__ void store_stage(const Chunk& c, const StageRows<NT, 
   }
 }
 
-// Zero a [16][nvp] fp32 table.
-__device__ __forceinline__ void zero_table(float* table, int nvp) {
-  for (int task = threadIdx.x; task < kTQ * (kChunkNV / 4); task += kThreads) {
-    const int row = task >> 6, c4 = (task & 63) * 4;
-    if (c4 < nvp) {
-      const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-      __builtin_memcpy(&table[row * kSRow + c4], &z, sizeof(z));
-    }
-  }
-}
-
 // Step key of (chunk, plane z): chunk << 16 | z.  A slot's key is that of its
 // lower plane z0 (an empty slot's z0 field 0xffff matches no plane), so the
 // distance d = step key - slot key is 0 on the lower plane and 1 on the upper
@@ -760,61 +597,21 @@ __device__ __forceinline__ bool slot_hits(const Slot& s, uint32_t key, float& wz
   return true;
 }
 
-// Branch-free form of slot_hits: the z weight (0 when the slot has no corners
-// on the step's plane), its z derivative sign (0 likewise) and the hit flag.
-__device__ __forceinline__ bool slot_weight(const Slot& s, uint32_t key, float& wz, float& dwz) {
-  const uint32_t d = key - slot_key(s);
-  const bool hit = d <= static_cast<uint32_t>(slot_hz(s));
-  wz = hit ? (d == 0 ? 1.0f - s.fz : s.fz) : 0.0f;
-  dwz = hit ? (d == 0 ? -1.0f : 1.0f) : 0.0f;
-  return hit;
-}
-
-// Table values at the slot's 4 (y, x) corners of the current plane.  An upper
-// corner row outside the volume (dy = 0, weight fy = 0) reads the lower row
-// again.  Each row's two x corners are one paired read of entries base and
-// base + 1; for an upper x corner outside the volume (weight fx = 0) entry
-// base + 1 belongs to another voxel, so its value is replaced by 0 (one
-// select): grid_sample skips out-of-volume corners, and a non-finite score of
-// that other voxel must not reach this tap as 0 * inf.  Every index is at most
-// kChunkNV, inside a table row even for a slot of another chunk (whose values
-// are then discarded).
-__device__ __forceinline__ void corners4(const Slot& s, const float* row, float& t00, float& t01,
-                                         float& t10, float& t11) {
-  const int base = s.idx & 0x1ff, dy = (s.idx >> 9) & 0x1f;
-  const bool hx = (s.idx >> 14) & 1;
-  t00 = row[base];
-  const float r01 = row[base + 1];
-  t10 = row[base + dy];
-  const float r11 = row[base + dy + 1];
-  t01 = hx ? r01 : 0.0f;
-  t11 = hx ? r11 : 0.0f;
-}
-
-// Zeroes NB whole tables (pad columns included).
-template <int NB>
-__device__ __forceinline__ void zero_tables_all(float* tables) {
-  constexpr int n4 = NB * kTQ * kSRow / 4;
-  for (int e = threadIdx.x; e < n4; e += blockDim.x) {
-    const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-    __builtin_memcpy(&tables[4 * e], &z, sizeof(z));
-  }
-}
-
 // Bilinear (y, x) interpolation of 4 corner values and its two partial
 // derivatives: val = lerp_y(top, bot), d/dfx and d/dfy.
 struct Bilerp {
   float val, dx, dy;
 };
 
-__device__ __forceinline__ Bilerp bilerp(const Slot& s, float t00, float t01, float t10, float t11) {
+__device__ __forceinline__ Bilerp bilerp(float fx, float fy, float t00, float t01, float t10,
+                                         float t11) {
   const float dtop = t01 - t00, dbot = t11 - t10;
-  const float top = __builtin_fmaf(s.fx, dtop, t00);
-  const float bot = __builtin_fmaf(s.fx, dbot, t10);
+  const float top = __builtin_fmaf(fx, dtop, t00);
+  const float bot = __builtin_fmaf(fx, dbot, t10);
   Bilerp r;
   r.dy = bot - top;
-  r.val = __builtin_fmaf(s.fy, r.dy, top);
-  r.dx = __builtin_fmaf(s.fy, dbot - dtop, dtop);
+  r.val = __builtin_fmaf(fy, r.dy, top);
+  r.dx = __builtin_fmaf(fy, dbot - dtop, dtop);
   return r;
 }
 
@@ -861,67 +658,6 @@ __device__ __forceinline__ op_t<E> fix_to_op(const int* p) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) r[i] = static_cast<float>(p[i]);
     return r;
-  }
-}
-
-// 8 floats -> MFMA operand (rounded to bf16 for bf16 storage).
-template <typename E>
-__device__ __forceinline__ op_t<E> f32_to_op(const float* p) {
-  if constexpr (sizeof(E) == 2) {
-    u32x4_t r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const f32x2_t f = {p[2 * i], p[2 * i + 1]};
-      r[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
-    }
-    return __builtin_bit_cast(bf16x8_t, r);
-  } else {
-    f32x8_t r;
-    __builtin_memcpy(&r, p, sizeof(r));
-    return r;
-  }
-}
-
-// MFMA B operands of 16 extra-key rows (block eb of 16): y[c] holds channels
-// 32 c + 8 (lane / 16) + [0, 8) of extra key 16 eb + lane % 16 of the tile's
-// sample and head; rows past G are zero.
-template <int HD, typename E>
-__device__ __forceinline__ void load_extra_rows(const Args& a, const Tile& tl, const void* base,
-                                                int eb, op_t<E> (&y)[HD / 32]) {
-#pragma unroll
-  for (int c = 0; c < HD / 32; ++c) y[c] = zero_op<E>();
-  const int g = 16 * eb + (tl.lane & 15);
-  if (g >= a.G) return;
-  const int D = a.nh * HD;
-  const E* p = static_cast<const E*>(base) + (static_cast<int64_t>(tl.b) * a.G + g) * D +
-               tl.head * HD + 8 * (tl.lane >> 4);
-#pragma unroll
-  for (int c = 0; c < HD / 32; ++c) y[c] = load_op<E>(p + 32 * c);
-}
-
-// Extra-key rows (key or value) of the tile's head, channels [0, HD), keys
-// g0 + [0, ng) transposed into yt[channel][g - g0] (row stride `row`
-// elements), zero for keys past G: thread item e moves 8 channels of one key.
-template <int HD, typename E>
-__device__ __forceinline__ void stage_extra_t(const Args& a, const Tile& tl, const void* base,
-                                              int g0, int ng, int row, word_t<E>* yt, int nthreads) {
-  const int D = a.nh * HD;
-  for (int e = threadIdx.x; e < ng * (HD / 8); e += nthreads) {
-    const int gi = e / (HD / 8), cg = e % (HD / 8), g = g0 + gi;
-    op_t<E> x = zero_op<E>();
-    if (g < a.G)
-      x = load_op<E>(static_cast<const E*>(base) + (static_cast<int64_t>(tl.b) * a.G + g) * D +
-                     tl.head * HD + 8 * cg);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if constexpr (sizeof(E) == 2) {
-        const u32x4_t xb = __builtin_bit_cast(u32x4_t, x);
-        yt[(8 * cg + i) * row + gi] =
-            static_cast<uint16_t>((i & 1) ? (xb[i / 2] >> 16) : (xb[i / 2] & 0xffffu));
-      } else {
-        yt[(8 * cg + i) * row + gi] = x[i];
-      }
-    }
   }
 }
 

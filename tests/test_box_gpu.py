@@ -102,3 +102,23 @@ def test_other_head_sizes_match_direct(hd, G, p, dt):
     for x, y in zip(a, b):
         tol = 2e-5 if dt == torch.float32 else 2.0 ** -8
         assert (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
+
+
+@pytest.mark.parametrize("hd,dt", [(32, torch.float32), (64, torch.bfloat16), (96, torch.float32),
+                                   (128, torch.bfloat16)])
+@pytest.mark.parametrize("p", [0.0, 0.4])
+@pytest.mark.parametrize("case", CASES)
+def test_box_backward_matches_direct(case, p, hd, dt):
+    """The first backward kernel's tables, pieces and records: every gradient against the direct
+    kernels (fp32: fixed-point tables of 2^-30 per corner; bf16: operands of 2^-9).  A one-tap
+    window's dq and dk vanish identically: 1e-4 of the unit-variance inputs."""
+    print(f"[box backward] {case} {hd} {dt} {p}", flush=True)
+    T, H, W, nh, win, _ = case
+    ins = _inputs(case, hd, dt)
+    kw = dict(dropout_p=p, dropout_seed=3)
+    a = _grads(ins, [], (T, H, W), nh, win, algo="tiled", **kw)
+    b = _grads(ins, [], (T, H, W), nh, win, algo="direct", **kw)
+    for x, y in zip(a, b):
+        tol = 2e-5 if dt == torch.float32 else 2e-2
+        bound = max(tol * y.float().abs().max().item(), 1e-4)
+        assert (x.float() - y.float()).abs().max().item() <= bound
