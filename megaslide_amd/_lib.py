@@ -30,6 +30,7 @@ EXPORTS = (
     "msd_last_error",
     "msd_dsa3d_fwd",
     "msd_dsa3d_bwd_workspace_size",
+    "msd_dsa3d_bwd_best_workspace_size",
     "msd_dsa3d_bwd",
     "msd_dsa3d_bwd_noalloc",
     "msd_dwconv3d_fwd",
