@@ -139,13 +139,18 @@ __device__ __forceinline__ AxisTap axis_tap(float pos2, float o, float bdiv, flo
 // One workgroup per unit (head, tile).  Workgroups are dispatched round-robin
 // over the 8 XCDs; each XCD has a contiguous run of units, so that neighbouring
 // tiles (frames vary fastest: they read nearly the same K/V planes) share its L2.
-inline unsigned box_grid(int B, int T, int H, int W, int heads) {
+// A launch takes at most 2^32 - 1 threads along x, which 2^23 workgroups reach: more
+// of them go on along y.
+inline dim3 box_grid(int B, int T, int H, int W, int heads) {
+  constexpr int64_t kMaxX = 1 << 22;
   const int64_t units = tile_count<1>(B, T, H, W) * heads;
-  return static_cast<unsigned>((units + 7) / 8 * 8);
+  if (units <= kMaxX) return dim3(static_cast<unsigned>((units + 7) / 8 * 8));
+  return dim3(static_cast<unsigned>(kMaxX), static_cast<unsigned>((units + kMaxX - 1) / kMaxX));
 }
 // This workgroup's unit, -1 past the last.
 __device__ __forceinline__ int box_unit(const Args& a) {
-  const unsigned u = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const unsigned i = blockIdx.y * gridDim.x + blockIdx.x;  // x is a multiple of 8
+  const unsigned u = (i & 7) * ((gridDim.x >> 3) * gridDim.y) + (i >> 3);
   const unsigned n = static_cast<unsigned>(a.nh * a.B * a.T) * (a.tiles_h * a.tiles_w);
   return u < n ? static_cast<int>(u) : -1;
 }
@@ -368,9 +373,6 @@ __device__ __forceinline__ BoxSeg box_seg(const BoxPieces& bx, int s) {
 
 // Rows of one sample and head behind a buffer resource: 32-bit byte offsets,
 // rows outside the volume or the box at an offset past the end read as zero.
-// (The host admits a sample of less than 2^32 - 2048 bytes; lane and immediate
-// offsets added to kNoRow stay below that.)
-constexpr uint32_t kNoRow = 0xfffff800u;
 constexpr int kBufWord3 = 0x00020000;  // raw 32-bit dwords, no swizzle (gfx9)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t box_rows(const void* base, int64_t bytes) {
   // wave-uniform by construction; said so, the resource stays in scalar registers

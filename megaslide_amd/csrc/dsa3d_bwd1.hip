@@ -316,7 +316,7 @@ template <int HD, typename E, int AE, bool REC>
 void launch_bwd_p1(const Args& a, const E* dout, const float* lse, const float* dlse, E* doff,
                    float* p_ws, float* b_ws, void* dk_acc, void* dv_acc, int64_t acc_ks,
                    int64_t acc_vs, const RecArgs& rc, hipStream_t s) {
-  const dim3 grid(box_grid(a.B, a.T, a.H, a.W, a.nh)), block(kThreads);
+  const dim3 grid = box_grid(a.B, a.T, a.H, a.W, a.nh), block(kThreads);
   if (a.drop.threshold != 0)
     hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, AE, REC, true>), grid, block, 0, s, a, dout, lse,
                        dlse, doff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, rc);

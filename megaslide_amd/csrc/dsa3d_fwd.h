@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_
 
 template <typename S, typename E, bool RG>
 hipError_t fwd_typed(const msd_dsa3d_desc& d, const Args& a, void* out, float* lse, hipStream_t s) {
-  const dim3 grid(box_grid(d.B, d.T, d.H, d.W, d.num_heads));
+  const dim3 grid = box_grid(d.B, d.T, d.H, d.W, d.num_heads);
   const dim3 block(kThreads);
   S* const o = static_cast<S*>(out);
   auto go = [&]<int HD>() {

@@ -196,12 +196,11 @@ bool dsa3d_ragged_supported(const msd_dsa3d_desc& d, const void* q, const void* 
     if (reinterpret_cast<uintptr_t>(p) % 16) return false;
   // the forward addresses a sample's rows with 32-bit byte offsets, and packs a
   // tap's piece of a cut box into 17 bits (a sample of less than 2^25 voxels)
-  const int64_t n = static_cast<int64_t>(d.T) * d.H * d.W;
-  const int64_t eb = d.dtype == MSD_BF16 ? 2 : 4;
-  if (n >= int64_t{1} << 25 ||
-      n * std::max(d.k_stride, d.v_stride) * eb >= static_cast<int64_t>(kNoRow))
+  const msd_dsa3d_desc p = padded_desc(d);
+  if (static_cast<int64_t>(d.T) * d.H * d.W >= int64_t{1} << 25 || !rows_below_limit(d) ||
+      !rows_below_limit(p))
     return false;
-  return dsa3d_tiled_supported(padded_desc(d), nullptr, nullptr, nullptr);
+  return dsa3d_tiled_supported(p, nullptr, nullptr, nullptr);
 }
 
 hipError_t launch_dsa3d_fwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,

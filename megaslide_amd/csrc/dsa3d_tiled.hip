@@ -1983,6 +1983,9 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
                                   void* dek, void* dev, void* ws, hipStream_t s) {
+  if (!tiled::rows_below_limit(d))
+    return launch_dsa3d_bwd_direct(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
+                                   dek, dev, ws, s);
   if (d.dtype == MSD_BF16)
     return bwd_tiled_typed<bf16>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
                                  dek, dev, ws, s);

@@ -42,6 +42,17 @@ constexpr int kMaxChunks = 1 << 16;     // chunk ids are kept in 16 bits
 // lane; 64 banks in four 16-lane passes) are 2-way conflicted in each pass, and
 // no stride or row order avoids that without conflicting the result writes.
 constexpr int kSRow = kChunkNV + 4;
+// Byte offset that stands for a row outside the volume or the box (dsa3d_box.h):
+// past the end of a sample's rows, and no lane or immediate offset added to it
+// wraps.  Samples that reach it (or extra keys whose signed offsets overflow)
+// take the direct kernels.
+constexpr uint32_t kNoRow = 0xfffff800u;
+inline bool rows_below_limit(const msd_dsa3d_desc& d) {
+  const int64_t st = d.k_stride > d.v_stride ? d.k_stride : d.v_stride;
+  const int64_t eb = d.dtype == MSD_BF16 ? 2 : 4;
+  return static_cast<int64_t>(d.T) * d.H * d.W * st * eb < static_cast<int64_t>(kNoRow) &&
+         int64_t{d.extra_g} * d.num_heads * d.head_dim * eb < int64_t{1} << 31;
+}
 constexpr int kVRow = kChunkNV + 8;     // bf16 row stride of a transposed K/V chunk
 
 // Matrix-core operands per element type.  A lane's operand of one k block is

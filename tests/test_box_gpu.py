@@ -122,3 +122,22 @@ def test_box_backward_matches_direct(case, p, hd, dt):
         tol = 2e-5 if dt == torch.float32 else 2e-2
         bound = max(tol * y.float().abs().max().item(), 1e-4)
         assert (x.float() - y.float()).abs().max().item() <= bound
+
+
+def test_more_workgroups_than_one_launch_axis_takes():
+    """8.5 million tiles of one query: more workgroups of 512 threads than an axis of a launch
+    holds.  One tap per query: the output is that tap's V sample, and dq, dk vanish."""
+    from megaslide_amd import dsa3d_core
+
+    B, T, nh, hd = 32, 4096, 65, 32
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q, v, dout = (torch.randn(B, T, nh * hd, generator=g, device="cuda", dtype=torch.bfloat16)
+                  for _ in range(3))
+    off = torch.zeros(B, T, nh * 3, device="cuda", dtype=torch.bfloat16)
+    res = []
+    for algo in ("tiled", "direct"):
+        vv = v.detach().requires_grad_(True)
+        out = dsa3d_core(q, q, vv, off, (T, 1, 1), nh, (1, 1, 1), algo=algo)
+        res.append((out.detach(), *torch.autograd.grad(out, vv, dout)))
+    for x, y in zip(*res):
+        assert (x - y).abs().max() <= 2e-2 * y.abs().max()
