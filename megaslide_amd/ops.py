@@ -195,7 +195,15 @@ def _core_bwd_op(q: Tensor, k: Tensor, v: Tensor, offsets: Tensor, extra_k: Opti
     dev_ = torch.empty_like(call.ev) if has_extra else q.new_empty((0,))
     lib = _lib.load()
     ws_bytes = lib.msd_dsa3d_bwd_best_workspace_size(ctypes.byref(desc))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+    need = lib.msd_dsa3d_bwd_workspace_size(ctypes.byref(desc))
+    try:
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        if need == ws_bytes:
+            raise
+        # the padded copies do not fit: the kernels that do without them
+        ws_bytes = need
+        ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
         _lib.check(lib.msd_dsa3d_bwd(
             ctypes.byref(desc), qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), call.off.data_ptr(),

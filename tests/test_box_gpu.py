@@ -141,3 +141,24 @@ def test_more_workgroups_than_one_launch_axis_takes():
         res.append((out.detach(), *torch.autograd.grad(out, vv, dout)))
     for x, y in zip(*res):
         assert (x - y).abs().max() <= 2e-2 * y.abs().max()
+
+
+def test_padded_backward_does_without_its_copies(monkeypatch):
+    """Where the padded copies' workspace does not fit the device, the backward takes the kernels
+    that need none (the direct ones: equal up to the atomics' order, 2e-5 as above)."""
+    case = (4, 9, 10, 3, (3, 5, 5), 1.0)
+    ins = _inputs(case, 40, torch.float32)
+    ref = _grads(ins, [], case[:3], 3, case[4], algo="direct")
+    empty, failed = torch.empty, []
+
+    def scarce(*args, **kw):
+        if kw.get("dtype") == torch.uint8 and not failed:
+            failed.append(args)
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", scarce)
+    got = _grads(ins, [], case[:3], 3, case[4])
+    assert failed
+    for x, y in zip(got, ref):
+        assert (x - y).abs().max() <= 2e-5 * y.abs().max()
