@@ -1707,7 +1707,7 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
   const int64_t acc_ks = w.acc_ks, acc_vs = w.acc_vs;
   // scaled fp16 accumulation: bf16 storage with MSD_ACCUM_F16 only
   const bool h16 = sizeof(E) == 2 && w.h16;
-  // bf16 with fp32 accumulation and no extra keys: the first kernel also
+  // bf16 with fp32 accumulation, no extra keys and enough columns: the first kernel also
   // writes tap records, the column-streaming kernel takes every column it can
   // and the tile kernel the columns it flags
   if constexpr (sizeof(E) == 2) {
@@ -1833,10 +1833,31 @@ struct TiledWs {
   size_t acc, xacc, p, ds, dse, pfe, dqx, dlt, stats, scales, rec, hdr, qt, collist, bytes;
 };
 
-// Calls that take the column-streaming dq/dK/dV kernel: bf16 storage with fp32
+// Calls that the column-streaming dq/dK/dV kernel can take: bf16 storage with fp32
 // dK/dV accumulation and no extra keys.
 bool tiled_streams(const msd_dsa3d_desc& d) {
   return d.dtype == MSD_BF16 && d.dkv_accum == MSD_ACCUM_F32 && d.extra_g == 0;
+}
+
+// Whether such a call has the columns to keep the streaming kernel's one workgroup
+// per CU busy; the tile kernel, which splits a column into tiles of two or three
+// frames, takes it otherwise (the workspace is the same, so that its size does not
+// depend on the device).  The streaming kernel walks a unit (two neighbouring
+// columns of a head) serially on one CU and spends about 2/3 of the tile kernel's
+// time per unit, so a launch of few units ends when its longest column does.
+// Backward in us, streaming -> tile, of 256 CUs: 32 units (32 frames of 8 x 8, 16
+// heads of 64, window 3x5x5) 381 -> 281; 48 units (32 of 12 x 16, 8 x 64, 3x7x7)
+// 1,237 -> 485; 128 units (16 of 16 x 16, 16 x 64) 809 -> 549; 192 units (32 of
+// 16 x 16, 24 x 64) 1,865 -> 1,975, with other depths 7 % either way.  The tile kernel
+// costs more at head_dim 128 (two channel windows) and 32 (two frames a tile): with
+// boxes of offsets of many voxels up to 5 and 14 % slower at 120 units, 1.2 to 3.4
+// times faster at up to 80.
+bool enough_columns(const msd_dsa3d_desc& d) {
+  const int64_t units = static_cast<int64_t>(d.B) * d.num_heads *
+                        ((d.H + tiled::kTileH - 1) / tiled::kTileH) *
+                        ((d.W + 2 * tiled::kTileW - 1) / (2 * tiled::kTileW));
+  const int64_t cus = device_cus();
+  return d.head_dim == 64 || d.head_dim == 96 ? 2 * units > cus : 5 * units > 2 * cus;
 }
 
 TiledWs tiled_ws(const msd_dsa3d_desc& d) {
@@ -1915,7 +1936,7 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
   w.dqx = erows > 0 ? reinterpret_cast<float*>(base + L.dqx) : nullptr;
   w.dlt = erows > 0 ? reinterpret_cast<float*>(base + L.dlt) : nullptr;
   w.rec = RecArgs{};
-  if (tiled_streams(d)) {
+  if (tiled_streams(d) && enough_columns(d)) {
     w.rec.rec = reinterpret_cast<tiled::u32x4_t*>(base + L.rec);
     w.rec.hdr = reinterpret_cast<int*>(base + L.hdr);
     w.rec.qt = base + L.qt;

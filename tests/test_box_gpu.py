@@ -162,3 +162,28 @@ def test_padded_backward_does_without_its_copies(monkeypatch):
     assert failed
     for x, y in zip(got, ref):
         assert (x - y).abs().max() <= 2e-5 * y.abs().max()
+
+
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("case", [
+    # units (pairs of 4 x 4 columns of a head) on both sides of the lines of 256 CUs
+    (6, 4, 4, 102, (3, 5, 5), 0.5),
+    (6, 4, 4, 103, (3, 5, 5), 0.5),
+    (6, 4, 4, 128, (3, 5, 5), 0.5),
+    (6, 4, 4, 129, (3, 5, 5), 0.5),
+    # the streaming kernel's walks: its ring of frames, wide boxes, more than 256 frames
+    (40, 4, 4, 136, (3, 7, 7), 0.5),
+    (20, 8, 24, 24, (3, 3, 3), 4.0),
+    (5, 13, 21, 12, (3, 7, 7), 1.5),
+    (300, 4, 4, 130, (1, 3, 3), 0.5),
+])
+def test_both_second_backward_kernels_match_direct(case, hd):
+    """bf16 gradients through the tile kernel (few columns) and the column-streaming one (many):
+    operands of 2^-9 as above."""
+    print(f"[second backward kernel] {case} {hd}", flush=True)
+    T, H, W, nh, win, _ = case
+    ins = _inputs(case, hd, torch.bfloat16)
+    a = _grads(ins, [], (T, H, W), nh, win, algo="tiled")
+    b = _grads(ins, [], (T, H, W), nh, win, algo="direct")
+    for x, y in zip(a, b):
+        assert (x.float() - y.float()).abs().max() <= 2e-2 * y.float().abs().max()
