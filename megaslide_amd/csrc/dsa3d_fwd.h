@@ -20,7 +20,8 @@
 // each): 3.20 -> 2.86 ms at 65,536 tokens, 16 x 64, bf16; 6.5 -> 5.8 ms at 46,800
 // tokens, 16 x 96, offsets biased by up to 4 voxels; 2.04 -> 1.46 ms at 32,768
 // tokens, 8 x 64, fp32; 44 -> 30 us at 2,048 tokens, 4 x 64, fp32; unchanged
-// (12.3 -> 12.2 ms) at 131,072 tokens, 24 x 128.  Tried and slower: a persistent
+// (12.3 -> 12.2 ms) at 131,072 tokens, 24 x 128.  Slower where the box's voxel past
+// the far face weighs: 0.21 -> 0.24 ms at 2 x 60 x 90, 4 x 64, a plane in three.  Tried and slower: a persistent
 // grid with the next tile's offsets loaded ahead (registers spill), 8 or 10
 // blocks of K rows in flight per wave instead of 6.
 #pragma once
