@@ -8,9 +8,12 @@
 // visit, where a table of one plane at a time has every tap tested on every
 // plane of the box and costs two or three barriers per plane.
 //
-// A box of more than kBoxCap voxels is cut into equal pieces that overlap by one
-// voxel along the cut axes, so the 2 x 2 x 2 footprint of every tap lies in
-// exactly one piece; the pieces are taken in turn.
+// A box of more than kBoxCap voxels is cut along its longest axis into equal slabs
+// that overlap by one voxel, so that the 2 x 2 x 2 footprint of every tap lies in
+// exactly one; they are taken in turn.  (A box of more than 296 voxels per layer
+// is first cut into such columns across that axis.)  The weighted sum gives the
+// layer that two slabs share to the later one, so that a voxel's weight is
+// rounded to the products' element type once, as in a box of one piece.
 //
 // The box reaches one voxel past the largest lower corner on every axis, also
 // where that is outside the volume: those rows read as zero (buffer loads past
@@ -30,53 +33,54 @@ constexpr int kBoxCap = 1184;  // voxels of a table: a multiple of 32
 constexpr int kBoxRow = 1188;
 static_assert(kBoxCap % 32 == 0 && kBoxRow >= kBoxCap + 2 && (kBoxRow / 4) % 2 == 1);
 
-// Pieces of a tile's box: origins lo + p (c - 1), c voxels, per axis.
+// A tile's box and its pieces: slabs along `axis` of columns that the other two
+// axes are cut into, a piece at every (extent - 1)-th voxel of the box.  A voxel's
+// index in a table row counts along `axis` slowest, then along the middle axis (y
+// where axis is z, else z), then along the last (y where axis is x, else x).
 struct BoxPieces {
   int zlo, ylo, xlo;     // the box's first voxel
   int zhi, yhi, xhi;     // its last voxel inside the volume
-  int cz, cy, cx;        // piece size
-  int py, px, n;         // pieces along y, x; in all
-  int sz, nv;            // voxels of a plane of a piece, of a piece
-  float rcx, rsz;        // 1 / cx, 1 / sz for division-free voxel coordinates
+  int n;                 // pieces; 1: the whole box, axis z
+  int axis;              // 0 x, 1 y, 2 z
+  int len, slabs;        // the box's layers along the axis; slabs of a column
+  int pn;                // columns along the last axis
+  int ca, cm, cn;        // voxels of a piece along the axis, the middle and the last
+  int dz, dy, dx;        // distances of neighbours in a table row
+  int nv;                // voxels of a piece
+  float rlayer, rrow;    // 1 / (cm cn), 1 / cn for division-free voxel coordinates
 };
 
-// One piece.
+// One piece: its first voxel; the taps' words (BoxTaps) count from `base` there,
+// words from `taps` on are of other pieces, and so are voxels from `own` on (the
+// layer shared with the next slab).
 struct BoxSeg {
-  int z0, y0, x0;
+  int z0, y0, x0, base, taps, own;
 };
 
-// Piece sizes for a box of nz x ny x nx voxels: the longest axis is cut first
-// (the shared voxel of a cut costs least there), into halves until a whole
-// number of pieces of that axis fits, and the pieces of an axis are equal.
-__device__ __forceinline__ void box_cut(int nz, int ny, int nx, int& cz, int& cy, int& cx) {
-  cz = nz;
-  cy = ny;
-  cx = nx;
+// Piece sizes for a box of na x nm x nn voxels, na the largest: columns are halved
+// until slabs of 4 layers (of which 3 are new) fit the table.
+__device__ __forceinline__ void box_cut(int na, int nm, int nn, int& ca, int& cm, int& cn) {
+  cm = nm;
+  cn = nn;
 #pragma nounroll
-  while (cz * cy * cx > kBoxCap) {
-    const int big = max(cz, max(cy, cx));
-    const bool isx = cx == big, isy = !isx && cy == big;
-    const int rest = isx ? cz * cy : isy ? cz * cx : cy * cx;
-    const int full = isx ? nx : isy ? ny : nz;
-    int c = max(kBoxCap / rest, big / 2 + 1);
-    const int p = (full - 2) / (c - 1) + 1;  // ceil((full - 1) / (c - 1))
-    c = (full - 2) / p + 2;                  // ceil((full - 1) / p) + 1
-    if (isx) cx = c;
-    else if (isy) cy = c;
-    else cz = c;
+  while (cm * cn * 4 > kBoxCap) {
+    if (cm > cn) cm = cm / 2 + 1;
+    else cn = cn / 2 + 1;
   }
+  ca = min(kBoxCap / (cm * cn), na);
+  const int p = (na - 2) / (ca - 1) + 1;  // ceil((na - 1) / (ca - 1))
+  ca = (na - 2) / p + 2;                  // ceil((na - 1) / p) + 1
 }
 
-// (A volume of less than 2^25 voxels, head_dim 32 at the host's size limit, has
-// less than 2^17 pieces: a piece of a cut box holds at least 8^3 of its own.)
-constexpr int kAtBits = 15;
-static_assert(kTQ * kBoxRow < 1 << kAtBits);
 // Geometry of this lane's taps: corner weights, and the word index of the
-// first corner in the query's table row (row offset included).
+// first corner in the query's table row (row offset included), or, where there
+// are several pieces, (column * len + layer) * (cm cn) + index within the
+// column's layer.  (A sample has less than 2^25 voxels, its box with the layers
+// past its faces and the columns' shared voxels less than 2^31.)
 template <int SLOTS>
 struct BoxTaps {
   float fx[SLOTS], fy[SLOTS], fz[SLOTS];
-  int at[SLOTS];    // where there are several pieces: | piece << kAtBits
+  int at[SLOTS];
   uint32_t flags;   // per tap, 4 bits: clamp-gradient mask x, y, z; dropped by dropout
 };
 
@@ -313,61 +317,77 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
   bx.zhi = min(zh + 1, a.T - 1);
   bx.yhi = min(yh + 1, a.H - 1);
   bx.xhi = min(xh + 1, a.W - 1);
-  bx.cz = nz;
-  bx.cy = ny;
-  bx.cx = nx;
-  bx.py = bx.px = bx.n = 1;
-  const int row = tl.q * kBoxRow;
-  auto index = [](int z, int y, int x, int sz, int cx) {
-    return static_cast<int>(__umul24(z, sz) + __umul24(y, cx)) + x;
-  };
+  bx.n = bx.slabs = bx.pn = 1;
+  bx.axis = 2;
+  bx.ca = bx.len = nz;
+  bx.cm = ny;
+  bx.cn = nx;
   if (nz * ny * nx <= kBoxCap) {
-    const int sz = nx * ny, base = row - (bx.zlo * sz + bx.ylo * nx + bx.xlo);
+    bx.dx = 1;
+    bx.dy = nx;
+    bx.dz = nx * ny;
+    const int base = tl.q * kBoxRow - (bx.zlo * bx.dz + bx.ylo * nx + bx.xlo);
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) tp.at[i] = index(zl[i], yl[i], xl[i], sz, nx) + base;
+    for (int i = 0; i < SLOTS; ++i)
+      tp.at[i] = static_cast<int>(__umul24(zl[i], bx.dz) + __umul24(yl[i], nx)) + xl[i] + base;
   } else {
-    box_cut(nz, ny, nx, bx.cz, bx.cy, bx.cx);
-    bx.cz = __builtin_amdgcn_readfirstlane(bx.cz);
-    bx.cy = __builtin_amdgcn_readfirstlane(bx.cy);
-    bx.cx = __builtin_amdgcn_readfirstlane(bx.cx);
-    bx.py = __builtin_amdgcn_readfirstlane((ny - 2) / (bx.cy - 1) + 1);
-    bx.px = __builtin_amdgcn_readfirstlane((nx - 2) / (bx.cx - 1) + 1);
-    bx.n = __builtin_amdgcn_readfirstlane((nz - 2) / (bx.cz - 1) + 1) * bx.py * bx.px;
-    const int sz = bx.cx * bx.cy;
-    // piece of a corner v (relative to the box): floor(v / (c - 1)); (v + 0.5) / d is at
-    // least 0.5 / d from an integer, far above the rounding for v < 2^15
-    const float rz = 1.0f / static_cast<float>(bx.cz - 1), ry = 1.0f / static_cast<float>(bx.cy - 1),
-                rx = 1.0f / static_cast<float>(bx.cx - 1);
+    const bool isx = nx >= ny && nx >= nz, isy = !isx && ny >= nz;
+    bx.axis = isx ? 0 : isy ? 1 : 2;
+    bx.len = isx ? nx : isy ? ny : nz;
+    const int nm = isx || isy ? nz : ny, nn = isx ? ny : nx;
+    box_cut(bx.len, nm, nn, bx.ca, bx.cm, bx.cn);
+    bx.ca = __builtin_amdgcn_readfirstlane(bx.ca);
+    bx.cm = __builtin_amdgcn_readfirstlane(bx.cm);
+    bx.cn = __builtin_amdgcn_readfirstlane(bx.cn);
+    bx.slabs = __builtin_amdgcn_readfirstlane((bx.len - 2) / (bx.ca - 1) + 1);
+    // (an axis of one voxel is a column of its own)
+    auto columns = [](int n, int c) { return n < 2 ? 1 : (n - 2) / (c - 1) + 1; };
+    const int pm = columns(nm, bx.cm);
+    bx.pn = __builtin_amdgcn_readfirstlane(columns(nn, bx.cn));
+    bx.n = __builtin_amdgcn_readfirstlane(bx.slabs * pm * bx.pn);
+    const int layer = bx.cm * bx.cn;
+    bx.dx = isx ? layer : 1;
+    bx.dy = isx ? 1 : isy ? layer : bx.cn;
+    bx.dz = isx || isy ? bx.cn : layer;
+    // column of a corner v along an axis: floor(v / (c - 1)); (v + 0.5) / d is at least
+    // 0.5 / d from an integer, far above the rounding for v < 2^15
+    const float rm = 1.0f / static_cast<float>(bx.cm - 1), rn = 1.0f / static_cast<float>(bx.cn - 1);
     auto div = [](int v, float r) { return static_cast<int>((static_cast<float>(v) + 0.5f) * r); };
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
       if (kSubs * i >= a.K) continue;
       const int z = zl[i] - bx.zlo, y = yl[i] - bx.ylo, x = xl[i] - bx.xlo;
-      const int pz = div(z, rz), py = div(y, ry), px = div(x, rx);
-      tp.at[i] = (row + index(z - pz * (bx.cz - 1), y - py * (bx.cy - 1), x - px * (bx.cx - 1),
-                              sz, bx.cx)) |
-                 ((pz * bx.py + py) * bx.px + px) << kAtBits;
+      const int la = isx ? x : isy ? y : z;
+      int m = isx || isy ? z : y, l = isx ? y : x, col = 0;
+      if (bx.n > bx.slabs) {
+        const int cm = pm > 1 ? div(m, rm) : 0, cn = bx.pn > 1 ? div(l, rn) : 0;
+        col = cm * bx.pn + cn;
+        m -= cm * (bx.cm - 1);
+        l -= cn * (bx.cn - 1);
+      }
+      tp.at[i] = (col * bx.len + la) * layer + m * bx.cn + l;
     }
   }
-  bx.sz = bx.cx * bx.cy;
-  bx.nv = bx.sz * bx.cz;
+  bx.nv = bx.ca * bx.cm * bx.cn;
   // hardware reciprocals (1 ulp): (v + 0.5) / d truncates exactly for v < kBoxCap
-  bx.rcx = __builtin_amdgcn_rcpf(static_cast<float>(bx.cx));
-  bx.rsz = __builtin_amdgcn_rcpf(static_cast<float>(bx.sz));
+  bx.rrow = __builtin_amdgcn_rcpf(static_cast<float>(bx.cn));
+  bx.rlayer = __builtin_amdgcn_rcpf(static_cast<float>(bx.cm * bx.cn));
 }
 
 __device__ __forceinline__ BoxSeg box_seg(const BoxPieces& bx, int s) {
-  BoxSeg g;
-  if (bx.n == 1) {
-    g.z0 = bx.zlo;
-    g.y0 = bx.ylo;
-    g.x0 = bx.xlo;
-    return g;
-  }
-  const int sx = s % bx.px, r = s / bx.px;
-  g.x0 = __builtin_amdgcn_readfirstlane(bx.xlo + sx * (bx.cx - 1));
-  g.y0 = __builtin_amdgcn_readfirstlane(bx.ylo + (r % bx.py) * (bx.cy - 1));
-  g.z0 = __builtin_amdgcn_readfirstlane(bx.zlo + (r / bx.py) * (bx.cz - 1));
+  BoxSeg g{bx.zlo, bx.ylo, bx.xlo, 0, 0, 0};
+  if (bx.n == 1) return g;
+  const int col = s / bx.slabs, a0 = (s - col * bx.slabs) * (bx.ca - 1);
+  const int m0 = col / bx.pn * (bx.cm - 1), l0 = col % bx.pn * (bx.cn - 1);
+  const int layer = bx.cm * bx.cn;
+  g.z0 = __builtin_amdgcn_readfirstlane(bx.zlo + (bx.axis == 2 ? a0 : m0));
+  g.y0 = __builtin_amdgcn_readfirstlane(bx.ylo + (bx.axis == 2 ? m0 : bx.axis == 1 ? a0 : l0));
+  g.x0 = __builtin_amdgcn_readfirstlane(bx.xlo + (bx.axis == 0 ? a0 : l0));
+  g.base = __builtin_amdgcn_readfirstlane((col * bx.len + a0) * layer);
+  // the box's last layer is no tap's first, and its last slab may reach past it
+  const int left = bx.len - a0;
+  g.taps = __builtin_amdgcn_readfirstlane((min(bx.ca, left) - 1) * layer);
+  g.own = __builtin_amdgcn_readfirstlane((left > bx.ca ? bx.ca - 1 : left) * layer);
   return g;
 }
 
@@ -399,10 +419,13 @@ __device__ __forceinline__ void box_row_offsets(const Args& a, const Tile& tl, c
 #pragma nounroll
   for (int p = tl.wave + kWaves * (tl.lane >> 5); p < np; p += 2 * kWaves) {
     const int vi = 32 * p + (tl.lane & 31);
-    const int vz = static_cast<int>((static_cast<float>(vi) + 0.5f) * bx.rsz);
-    const int r = vi - vz * bx.sz;
-    const int vy = static_cast<int>((static_cast<float>(r) + 0.5f) * bx.rcx);
-    const int z = g.z0 + vz, y = g.y0 + vy, x = g.x0 + r - vy * bx.cx;
+    const int va = static_cast<int>((static_cast<float>(vi) + 0.5f) * bx.rlayer);
+    const int r = vi - va * (bx.cm * bx.cn);
+    const int vm = static_cast<int>((static_cast<float>(r) + 0.5f) * bx.rrow);
+    const int vl = r - vm * bx.cn;
+    const int z = g.z0 + (bx.axis == 2 ? va : vm);
+    const int y = g.y0 + (bx.axis == 2 ? vm : bx.axis == 1 ? va : vl);
+    const int x = g.x0 + (bx.axis == 0 ? va : vl);
     const bool ok = vi < bx.nv && z <= bx.zhi && y <= bx.yhi && x <= bx.xhi;
     const uint32_t row = (static_cast<uint32_t>(z) * a.H + y) * static_cast<uint32_t>(a.W) + x;
     rows[vi] = ok ? row * stride : kNoRow;
@@ -765,12 +788,12 @@ __device__ __forceinline__ void box_zero(int* table, int n4) {
 
 // The tap's value interpolated from a table: lo / hi planes combined with their
 // weights (0 * value for the upper one where the position is on the plane).
-__device__ __forceinline__ float box_gather(const float* table, int at, int cx, int sz, float fx,
-                                            float fy, float fz) {
+__device__ __forceinline__ float box_gather(const float* table, int at, int dx, int dy, int dz,
+                                            float fx, float fy, float fz) {
   const float* const p = &table[at];
-  const float* const pz = p + sz;
+  const float* const pz = p + dz;
   auto plane = [&](const float* q) {
-    const float t0 = q[0], t1 = q[1], b0 = q[cx], b1 = q[cx + 1];
+    const float t0 = q[0], t1 = q[dx], b0 = q[dy], b1 = q[dy + dx];
     const float top = __builtin_fmaf(fx, t1 - t0, t0), bot = __builtin_fmaf(fx, b1 - b0, b0);
     return __builtin_fmaf(fy, bot - top, top);
   };
@@ -786,34 +809,58 @@ struct BoxTap {
 };
 template <int SLOTS>
 __device__ __forceinline__ BoxTap box_tap(const BoxTaps<SLOTS>& tp, int i) {
-  BoxTap t{tp.at[i] & ((1 << kAtBits) - 1), tp.fx[i], tp.fy[i], tp.fz[i]};
+  BoxTap t{tp.at[i], tp.fx[i], tp.fy[i], tp.fz[i]};
   asm volatile("" : "+v"(t.at), "+v"(t.fx), "+v"(t.fy), "+v"(t.fz));
   return t;
 }
-// Tap i in piece s of several, or in the only piece (s < 0)?
-template <int SLOTS>
-__device__ __forceinline__ bool box_in(const BoxTaps<SLOTS>& tp, int i, int s) {
-  return s < 0 || static_cast<uint32_t>(tp.at[i]) >> kAtBits == static_cast<uint32_t>(s);
+// Whether piece g (of several) holds the tap's footprint; t.at becomes the word index
+// of its first corner in the row of lane query q.
+__device__ __forceinline__ bool box_in(const BoxSeg& g, int q, BoxTap& t) {
+  const int r = t.at - g.base;
+  t.at = q * kBoxRow + r;
+  return static_cast<uint32_t>(r) < static_cast<uint32_t>(g.taps);
 }
 
 // Adds the tap's weight v (fixed-point units) to its eight corners.  TOUCH: at
 // least one unit (2^-30) each, which marks the corners of zero weight too
 // (grid_sample reads those as well: 0 times a non-finite value is not 0).
-template <bool TOUCH = false>
-__device__ __forceinline__ void box_scatter(int* table, int at, int cx, int sz, float fx, float fy,
-                                            float fz, float v) {
-  int* const p = &table[at];
-  int* const pz = p + sz;
-  auto plane = [&](int* q, float w) {
-    const float w1 = w * fy, w0 = w * (1.0f - fy), gx = 1.0f - fx;
-    auto fix = [](float x) { return TOUCH ? max(to_fix(x), 1) : to_fix(x); };
-    atomicAdd(q, fix(w0 * gx));
-    atomicAdd(q + 1, fix(w0 * fx));
-    atomicAdd(q + cx, fix(w1 * gx));
-    atomicAdd(q + cx + 1, fix(w1 * fx));
-  };
-  plane(p, v * (1.0f - fz));
-  plane(pz, v * fz);
+template <bool TOUCH>
+__device__ __forceinline__ void box_add4(int* q, int d0, int d1, float w, float f0, float f1) {
+  const float w1 = w * f1, w0 = w * (1.0f - f1), g0 = 1.0f - f0;
+  auto fix = [](float x) { return TOUCH ? max(to_fix(x), 1) : to_fix(x); };
+  atomicAdd(q, fix(w0 * g0));
+  atomicAdd(q + d0, fix(w0 * f0));
+  atomicAdd(q + d1, fix(w1 * g0));
+  atomicAdd(q + d1 + d0, fix(w1 * f0));
+}
+template <bool TOUCH>
+__device__ __forceinline__ void box_scatter(int* table, const BoxPieces& bx, const BoxTap& t, float v) {
+  int* const p = &table[t.at];
+  box_add4<TOUCH>(p, 1, bx.dy, v * (1.0f - t.fz), t.fx, t.fy);
+  box_add4<TOUCH>(p + bx.dz, 1, bx.dy, v * t.fz, t.fx, t.fy);
+}
+// The same to the corners that piece g (of several) owns: those of the tap's two
+// layers along the axis that lie in it.
+template <bool TOUCH>
+__device__ __forceinline__ void box_scatter(int* table, const BoxPieces& bx, const BoxSeg& g, int q,
+                                            const BoxTap& t, float v) {
+  const int r = t.at - g.base, layer = bx.cm * bx.cn;
+  const bool lo = static_cast<uint32_t>(r) < static_cast<uint32_t>(g.own);
+  const bool hi = static_cast<uint32_t>(r + layer) < static_cast<uint32_t>(g.own);
+  if (!(lo | hi)) return;
+  const float fx = t.fx, fy = t.fy, fz = t.fz;
+  float fa = fz, fm = fy, fl = fx;  // along z
+  if (bx.axis == 1) {
+    fa = fy;
+    fm = fz;
+  } else if (bx.axis == 0) {
+    fa = fx;
+    fm = fz;
+    fl = fy;
+  }
+  int* const p = &table[q * kBoxRow + r];
+  if (lo) box_add4<TOUCH>(p, 1, bx.cn, v * (1.0f - fa), fl, fm);
+  if (hi) box_add4<TOUCH>(p + layer, 1, bx.cn, v * fa, fl, fm);
 }
 
 }  // namespace tiled

@@ -32,12 +32,12 @@ using namespace tiled;
 struct TapGrad {
   float v, dx, dy, dz;
 };
-__device__ __forceinline__ TapGrad box_gather_grad(const float* table, const BoxTap& t, int cx,
-                                                   int sz) {
+__device__ __forceinline__ TapGrad box_gather_grad(const float* table, const BoxTap& t, int dx,
+                                                   int dy, int dz) {
   const float* const p = &table[t.at];
-  const float* const pz = p + sz;
+  const float* const pz = p + dz;
   auto plane = [&](const float* q) {
-    return bilerp(t.fx, t.fy, q[0], q[1], q[cx], q[cx + 1]);
+    return bilerp(t.fx, t.fy, q[0], q[dx], q[dy], q[dy + dx]);
   };
   const Bilerp lo = plane(p), hi = plane(pz);
   const float gz = 1.0f - t.fz;
@@ -106,19 +106,27 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
     const __amdgpu_buffer_rsrc_t rows =
         box_rows(p, ((a.N - 1) * stride + HD) * static_cast<int64_t>(sizeof(E)));
     auto row_off = [&](int v) { return s_row[v]; };
-#pragma nounroll
-    for (int s = 0; s < bx.n; ++s) {
-      if (!keep_rows || bx.n > 1)
-        box_row_offsets(a, tl, bx, box_seg(bx, s), static_cast<uint32_t>(stride * sizeof(E)), s_row);
+    auto piece = [&](int s, auto only) __attribute__((always_inline)) {  // `only`: of one
+      constexpr bool kOnly = decltype(only)::value;
+      const BoxSeg g = box_seg(bx, s);
+      if (!kOnly || !keep_rows)
+        box_row_offsets(a, tl, bx, g, static_cast<uint32_t>(stride * sizeof(E)), s_row);
       box_scores<HD, E, E, false, NB>(tl, rows, row_off, bx.nv, HD, x, s_tab);
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < kSlots; ++i) {
         if (kSubs * i >= a.K) continue;
-        if (!box_in(tp, i, bx.n > 1 ? s : -1)) continue;
-        tg[i] = box_gather_grad(s_tab, box_tap(tp, i), bx.cx, bx.sz);
+        BoxTap t = box_tap(tp, i);
+        if (!kOnly && !box_in(g, tl.q, t)) continue;
+        tg[i] = box_gather_grad(s_tab, t, kOnly ? 1 : bx.dx, bx.dy, bx.dz);
       }
       __syncthreads();  // the next table takes this one's place
+    };
+    if (bx.n == 1) {
+      piece(0, std::true_type{});
+    } else {
+#pragma nounroll
+      for (int s = 0; s < bx.n; ++s) piece(s, std::false_type{});
     }
   };
   sweep(a.k, a.ks, false, ts);
@@ -179,23 +187,31 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
       REC ? static_cast<int64_t>(tl.head) * rc.tiles +
                 rec_tile(a, tl.b, tl.t0, tl.h0 / kTileH, tl.w0 / kTileW)
           : 0;
-  // lower corner of tap i: its table index within the piece, and the piece's origin
+  // lower corner of tap i, from its word
+  const int layer = bx.cm * bx.cn;
+  const uint32_t m_col = REC && bx.n > 1 ? 0xffffffffu / static_cast<uint32_t>(bx.len * layer) : 0;
+  const uint32_t m_layer = REC && bx.n > 1 ? 0xffffffffu / static_cast<uint32_t>(layer) : 0;
   auto corner = [&](int i, int& z, int& y, int& xx) {
-    const int at = tp.at[i];
-    const int l = (at & ((1 << kAtBits) - 1)) - tl.q * kBoxRow;
-    const int vz = static_cast<int>((static_cast<float>(l) + 0.5f) * bx.rsz);
-    const int r = l - vz * bx.sz;
-    const int vy = static_cast<int>((static_cast<float>(r) + 0.5f) * bx.rcx);
-    z = bx.zlo + vz;
-    y = bx.ylo + vy;
-    xx = bx.xlo + r - vy * bx.cx;
+    int col = 0, r, va;
     if (bx.n > 1) {
-      const int s = static_cast<int>(static_cast<uint32_t>(at) >> kAtBits);
-      const int q = s / bx.px;
-      xx += (s - q * bx.px) * (bx.cx - 1);
-      y += (q % bx.py) * (bx.cy - 1);
-      z += (q / bx.py) * (bx.cz - 1);
+      col = bx.n > bx.slabs ? box_div(tp.at[i], bx.len * layer, m_col) : 0;
+      r = tp.at[i] - col * (bx.len * layer);
+      va = box_div(r, layer, m_layer);
+    } else {
+      r = tp.at[i] - tl.q * kBoxRow;
+      va = static_cast<int>((static_cast<float>(r) + 0.5f) * bx.rlayer);
     }
+    r -= va * layer;
+    int vm = static_cast<int>((static_cast<float>(r) + 0.5f) * bx.rrow);
+    int vl = r - vm * bx.cn;
+    if (bx.n > bx.slabs) {
+      const int q = col / bx.pn;
+      vm += q * (bx.cm - 1);
+      vl += (col - q * bx.pn) * (bx.cn - 1);
+    }
+    z = bx.zlo + (bx.axis == 2 ? va : vm);
+    y = bx.ylo + (bx.axis == 2 ? vm : bx.axis == 1 ? va : vl);
+    xx = bx.xlo + (bx.axis == 0 ? va : vl);
   };
   int pos[kSlots];
   if constexpr (REC) {

@@ -72,8 +72,8 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
     const S* p = static_cast<const S*>(base) + tl.sample0 * stride + static_cast<int64_t>(tl.head) * hd;
     return box_rows(p, ((a.N - 1) * stride + hd) * static_cast<int64_t>(sizeof(S)));
   };
-  auto set_rows = [&](int s, int64_t stride) {
-    box_row_offsets(a, tl, bx, box_seg(bx, s), static_cast<uint32_t>(stride * sizeof(S)), s_row);
+  auto set_rows = [&](const BoxSeg& g, int64_t stride) {
+    box_row_offsets(a, tl, bx, g, static_cast<uint32_t>(stride * sizeof(S)), s_row);
   };
   auto row_off = [&](int v) { return s_row[v]; };
   // extra keys: row g of the sample
@@ -95,19 +95,26 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   for (int i = 0; i < kSlots; ++i) sc[i] = 0.0f;
   {
     const __amdgpu_buffer_rsrc_t kr = rows_of(a.k, a.ks);
-#pragma nounroll
-    for (int s = 0; s < bx.n; ++s) {
-      set_rows(s, a.ks);
+    auto piece = [&](int s, auto only) __attribute__((always_inline)) {  // `only`: of one
+      constexpr bool kOnly = decltype(only)::value;
+      const BoxSeg g = box_seg(bx, s);
+      set_rows(g, a.ks);
       box_scores<HD, S, E, RG, NB>(tl, kr, row_off, bx.nv, hd, qx, s_val);
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < kSlots; ++i) {
         if (kSubs * i >= a.K) continue;
-        if (!box_in(tp, i, bx.n > 1 ? s : -1)) continue;
-        const BoxTap t = box_tap(tp, i);
-        sc[i] = box_gather(s_val, t.at, bx.cx, bx.sz, t.fx, t.fy, t.fz);
+        BoxTap t = box_tap(tp, i);
+        if (!kOnly && !box_in(g, tl.q, t)) continue;
+        sc[i] = box_gather(s_val, t.at, kOnly ? 1 : bx.dx, bx.dy, bx.dz, t.fx, t.fy, t.fz);
       }
       __syncthreads();  // the next piece, the extra keys or the weights take the table
+    };
+    if (bx.n == 1) {
+      piece(0, std::true_type{});
+    } else {
+#pragma nounroll
+      for (int s = 0; s < bx.n; ++s) piece(s, std::false_type{});
     }
   }
 
@@ -199,8 +206,10 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
     weighted(extra_rows(a.ev), extra_off, Gp, ah);
     __syncthreads();
   }
-  auto piece = [&](int s) {
-    if (s >= 0 || a.vs != a.ks) set_rows(max(s, 0), a.vs);  // else as the scores left them
+  auto piece = [&](int s, auto only) __attribute__((always_inline)) {
+    constexpr bool kOnly = decltype(only)::value;
+    const BoxSeg g = box_seg(bx, s);
+    if (!kOnly || a.vs != a.ks) set_rows(g, a.vs);  // else as the scores left them
     BoxAhead<HD, E> ah;
     box_weighted_begin<HD, S, E>(tl, vr, row_off, bx.nv, ah);
     box_zero(s_tab, ((bx.nv + 31) & ~31) >> 2);
@@ -208,20 +217,20 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
 #pragma unroll
     for (int i = 0; i < kSlots; ++i) {
       if (kSubs * i >= a.K) continue;
-      if (!box_in(tp, i, s)) continue;
-      const BoxTap t = box_tap(tp, i);
       if (SAFE && !has_tap(i)) continue;  // (a copy of another lane's tap)
-      box_scatter<SAFE>(s_tab, t.at, bx.cx, bx.sz, t.fx, t.fy, t.fz, sc[i]);
+      const BoxTap t = box_tap(tp, i);
+      if constexpr (kOnly) box_scatter<SAFE>(s_tab, bx, t, sc[i]);
+      else box_scatter<SAFE>(s_tab, bx, g, tl.q, t, sc[i]);
     }
     __syncthreads();
     weighted(vr, row_off, bx.nv, ah);
     __syncthreads();  // the products have read the table
   };
   if (bx.n == 1) {  // the usual case apart: no tap stays live through its products
-    piece(-1);
+    piece(0, std::true_type{});
   } else {
 #pragma nounroll
-    for (int s = 0; s < bx.n; ++s) piece(s);
+    for (int s = 0; s < bx.n; ++s) piece(s, std::false_type{});
   }
   // partial O of wave w: [w][query][channel]
   static_assert(kWaves * kTQ * HD <= kTQ * kBoxRow, "the partial sums fit the table");

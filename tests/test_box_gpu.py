@@ -187,3 +187,31 @@ def test_both_second_backward_kernels_match_direct(case, hd):
     b = _grads(ins, [], (T, H, W), nh, win, algo="direct")
     for x, y in zip(a, b):
         assert (x.float() - y.float()).abs().max() <= 2e-2 * y.float().abs().max()
+
+
+def test_cut_boxes_round_each_weight_once():
+    """bf16: the weight of a voxel that two pieces of a cut box share is rounded once, as every
+    other.  With q = 0 every tap weighs 1 / K, and a channel of V that is 1 at one voxel leaves
+    that voxel's weight as the output: the direct kernels' fp32 weight, rounded.  A fixed-point
+    weight is below that by less than one unit of 2^-30 a tap and corner: ~1e-8 of a bf16 step
+    of at least 2^-17 (weights from 2^-9), so that the rounding differs for under 1 %."""
+    from megaslide_amd import dsa3d_core
+
+    T, H, W, nh, win, _ = case = (12, 16, 16, 1, (3, 7, 7), 1.3)
+    hd, N = 128, 12 * 16 * 16
+    q, _, _, off = _inputs(case, hd, torch.bfloat16)
+    q.zero_()
+    differ = total = 0
+    for v0 in range(0, N, hd):
+        v = torch.zeros(1, N, hd, device="cuda")
+        n = min(hd, N - v0)
+        v[0, torch.arange(v0, v0 + n), torch.arange(n)] = 1.0
+        with torch.no_grad():
+            out = dsa3d_core(q, q, v.bfloat16(), off, (T, H, W), nh, win)
+            ref = dsa3d_core(q.float(), q.float(), v, off.float(), (T, H, W), nh, win,
+                             algo="direct")
+        big = ref >= 2.0 ** -9
+        differ += (out != ref.bfloat16())[big].sum().item()
+        total += big.sum().item()
+    print(f"[cut boxes] {differ} of {total} weights rounded otherwise", flush=True)
+    assert total > 10000 and differ < 0.01 * total
