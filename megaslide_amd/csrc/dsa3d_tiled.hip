@@ -1834,9 +1834,11 @@ struct TiledWs {
 };
 
 // Calls that the column-streaming dq/dK/dV kernel can take: bf16 storage with fp32
-// dK/dV accumulation and no extra keys.
+// dK/dV accumulation and no extra keys, and rows and columns that its tap records'
+// 14-bit coordinates hold.
 bool tiled_streams(const msd_dsa3d_desc& d) {
-  return d.dtype == MSD_BF16 && d.dkv_accum == MSD_ACCUM_F32 && d.extra_g == 0;
+  return d.dtype == MSD_BF16 && d.dkv_accum == MSD_ACCUM_F32 && d.extra_g == 0 &&
+         d.H <= kRecAxis && d.W <= kRecAxis;
 }
 
 // Whether such a call has the columns to keep the streaming kernel's one workgroup

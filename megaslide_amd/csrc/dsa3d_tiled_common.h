@@ -163,13 +163,15 @@ constexpr int kMaxExtra = 256;   // extra keys the tiled kernels take (a table r
 //   [0..5] the tile's corner box zlo, zhi, ylo, yhi, xlo, xhi; [6] bins used
 //   (0: no tap; -1: the planes span more than kRecBins bins, no records);
 //   [8 + b] first record of bin b (b <= bins used: [8 + bins] = count).
-// Record words: y0 | x0 << 14 | query << 28 (the tile's query 0..15); fx and
+// Record words: y0 | x0 << 14 | query << 28 (the tile's query 0..15; axes of up
+// to kRecAxis voxels: longer ones take the tile kernel); fx and
 // fy as 16-bit fractions (lo, hi); fz (fp32 bits); the fp16 pair (p * dropout
 // factor, ds * scale / l1) of the tap, l1 = sum over the query's taps of
 // |ds * scale|.  Per (head, tile) too: q and dO of the tile's 16 queries,
 // transposed ([tensor][channel][query], bf16), q times l1 / 2^30 and dO times
 // 1 / fix_a: the scales of the B and A tables' fixed point.
 constexpr int kRecBins = 16;
+constexpr int kRecAxis = 1 << 14;
 constexpr int kRecHdr = 32;
 struct RecArgs {
   u32x4_t* rec;    // [nh][tiles][K * 16] records

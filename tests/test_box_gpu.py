@@ -215,3 +215,16 @@ def test_cut_boxes_round_each_weight_once():
         total += big.sum().item()
     print(f"[cut boxes] {differ} of {total} weights rounded otherwise", flush=True)
     assert total > 10000 and differ < 0.01 * total
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 16384), (1, 2, 16390), (2, 16390, 1)])
+def test_axes_beyond_the_tap_records(shape):
+    """bf16 gradients on both sides of the longest axis that the column-streaming kernel's tap
+    records address (enough columns for it in each): operands of 2^-9 as above."""
+    print(f"[long axis] {shape}", flush=True)
+    case = (*shape, 1, (1, 3, 5) if shape[2] > 1 else (2, 5, 1), 1.0)
+    ins = _inputs(case, 32, torch.bfloat16)
+    a = _grads(ins, [], shape, 1, case[4], algo="tiled")
+    b = _grads(ins, [], shape, 1, case[4], algo="direct")
+    for x, y in zip(a, b):
+        assert (x.float() - y.float()).abs().max() <= 2e-2 * y.float().abs().max()
