@@ -116,7 +116,7 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* v, const void* off, const void* ek, const void* ev,
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                  void* dek, void* dev, void* ws, hipStream_t s);
+                                  void* dek, void* dev, void* ws, hipStream_t s, bool padded = false);
 bool dsa3d_ragged_supported(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v);
 hipError_t launch_dsa3d_fwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,
                                    const void* v, const void* off, const void* ek, const void* ev,

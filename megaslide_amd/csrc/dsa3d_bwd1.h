@@ -5,7 +5,7 @@
 
 namespace msd {
 
-template <int HD, typename E, int AE, bool REC>
+template <int HD, typename E, int AE, bool REC, bool SPLIT = false>
 void launch_bwd_p1(const tiled::Args& a, const E* dout, const float* lse, const float* dlse, E* doff,
                    float* p_ws, float* b_ws, void* dk_acc, void* dv_acc, int64_t acc_ks,
                    int64_t acc_vs, const tiled::RecArgs& rc, hipStream_t s);

@@ -51,8 +51,9 @@ __device__ __forceinline__ TapGrad box_gather_grad(const float* table, const Box
 
 // AE: bytes of one dK / dV accumulator element (4 = fp32 rows, 2 = scaled fp16).
 // REC: also write the tap records, tile header and transposed q / dO of the
-// column-streaming kernel (bf16 storage).
-template <int HD, typename E, int AE, bool REC, bool DROP>
+// column-streaming kernel (bf16 storage).  SPLIT: the scores' sums in short chains
+// (padded head sizes, box_scores_split).
+template <int HD, typename E, int AE, bool REC, bool DROP, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
     Args a, const E* __restrict__ dout, const float* __restrict__ lse,
     const float* __restrict__ dlse, E* __restrict__ doff, float* __restrict__ p_ws,
@@ -111,7 +112,8 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
       const BoxSeg g = box_seg(bx, s);
       if (!kOnly || !keep_rows)
         box_row_offsets(a, tl, bx, g, static_cast<uint32_t>(stride * sizeof(E)), s_row);
-      box_scores<HD, E, E, false, NB>(tl, rows, row_off, bx.nv, HD, x, s_tab);
+      if constexpr (SPLIT) box_scores_split<HD, E, false>(tl, rows, row_off, bx.nv, HD, x, s_tab);
+      else box_scores<HD, E, E, false, NB>(tl, rows, row_off, bx.nv, HD, x, s_tab);
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < kSlots; ++i) {
@@ -328,28 +330,29 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
 
 }  // namespace
 
-template <int HD, typename E, int AE, bool REC>
+template <int HD, typename E, int AE, bool REC, bool SPLIT>
 void launch_bwd_p1(const Args& a, const E* dout, const float* lse, const float* dlse, E* doff,
                    float* p_ws, float* b_ws, void* dk_acc, void* dv_acc, int64_t acc_ks,
                    int64_t acc_vs, const RecArgs& rc, hipStream_t s) {
   const dim3 grid = box_grid(a.B, a.T, a.H, a.W, a.nh), block(kThreads);
   if (a.drop.threshold != 0)
-    hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, AE, REC, true>), grid, block, 0, s, a, dout, lse,
-                       dlse, doff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, rc);
-  else
-    hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, AE, REC, false>), grid, block, 0, s, a, dout,
+    hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, AE, REC, true, SPLIT>), grid, block, 0, s, a, dout,
                        lse, dlse, doff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, rc);
+  else
+    hipLaunchKernelGGL((dsa3d_bwd_p1_kernel<HD, E, AE, REC, false, SPLIT>), grid, block, 0, s, a,
+                       dout, lse, dlse, doff, p_ws, b_ws, dk_acc, dv_acc, acc_ks, acc_vs, rc);
 }
 
-#define MSD_P1(HD, E, AE, REC)                                                                    \
-  template void launch_bwd_p1<HD, E, AE, REC>(                                                    \
+#define MSD_P1(HD, E, AE, REC, SPLIT)                                                             \
+  template void launch_bwd_p1<HD, E, AE, REC, SPLIT>(                                             \
       const Args&, const E*, const float*, const float*, E*, float*, float*, void*, void*,        \
       int64_t, int64_t, const RecArgs&, hipStream_t);
-#define MSD_P1_HD(HD)         \
-  MSD_P1(HD, float, 4, false) \
-  MSD_P1(HD, bf16, 4, false)  \
-  MSD_P1(HD, bf16, 4, true)   \
-  MSD_P1(HD, bf16, 2, false)
+#define MSD_P1_HD(HD)                \
+  MSD_P1(HD, float, 4, false, false) \
+  MSD_P1(HD, float, 4, false, true)  \
+  MSD_P1(HD, bf16, 4, false, false)  \
+  MSD_P1(HD, bf16, 4, true, false)   \
+  MSD_P1(HD, bf16, 2, false, false)
 MSD_P1_HD(32)
 MSD_P1_HD(64)
 MSD_P1_HD(96)

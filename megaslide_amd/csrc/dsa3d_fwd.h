@@ -88,6 +88,10 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
     return g < G ? static_cast<uint32_t>(g * static_cast<int>(D * sizeof(S))) : kNoRow;
   };
   constexpr int NB = box_score_blocks<HD, E>();
+  auto scores = [&](__amdgpu_buffer_rsrc_t r, const auto& off, int n) {
+    if constexpr (RG) box_scores_split<HD, S, RG>(tl, r, off, n, hd, qx, s_val);
+    else box_scores<HD, S, E, RG, NB>(tl, r, off, n, hd, qx, s_val);
+  };
 
   // ---- scores ---------------------------------------------------------------
   float sc[kSlots];
@@ -99,7 +103,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
       constexpr bool kOnly = decltype(only)::value;
       const BoxSeg g = box_seg(bx, s);
       set_rows(g, a.ks);
-      box_scores<HD, S, E, RG, NB>(tl, kr, row_off, bx.nv, hd, qx, s_val);
+      scores(kr, row_off, bx.nv);
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < kSlots; ++i) {
@@ -123,7 +127,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   constexpr int EPL = XK ? kMaxExtra / kSubs : 1;
   float se[EPL];
   if constexpr (XK) {
-    box_scores<HD, S, E, RG, NB>(tl, extra_rows(a.ek), extra_off, Gp, hd, qx, s_val);
+    scores(extra_rows(a.ek), extra_off, Gp);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {

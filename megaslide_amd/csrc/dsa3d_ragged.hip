@@ -168,7 +168,7 @@ hipError_t bwd_typed(const msd_dsa3d_desc& d, const void* q, const void* k, cons
   const hipError_t e = launch_dsa3d_bwd_tiled(
       p, f32(L.row[0]), f32(L.row[1]), f32(L.row[2]), off32, extra(0), extra(1), nullptr,
       f32(L.row[3]), lse, dlse, f32(L.row[4]), f32(L.row[5]), f32(L.row[6]), doff32, extra(2),
-      extra(3), ws + L.inner, s);
+      extra(3), ws + L.inner, s, true);
   if (e != hipSuccess) return e;
   unpad(L.row[4], rows, dq, d.q_stride);
   unpad(L.row[5], rows, dk, d.k_stride);

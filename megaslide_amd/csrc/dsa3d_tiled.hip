@@ -1166,8 +1166,8 @@ __global__ __launch_bounds__(256) void dsa3d_bwd_extra_kernel(
     for (int c = 0; c < HD / 32; ++c) {
       const op_t<E> yk = g < G ? load_op<E>(ek + static_cast<int64_t>(g) * D + 32 * c + kq) : zero_op<E>();
       const op_t<E> yv = g < G ? load_op<E>(ev + static_cast<int64_t>(g) * D + 32 * c + kq) : zero_op<E>();
-      sacc = mma16(xq[c], yk, sacc);
-      dacc = mma16(xo[c], yv, dacc);
+      sacc = mma16_add(xq[c], yk, sacc);
+      dacc = mma16_add(xo[c], yv, dacc);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(256) void dsa3d_bwd_extra_kernel(
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       const int ct = wave + 4 * t;
-      if (ct < CT) dqa[t] = mma16(bp, load_op<E>(&s_ekt[(16 * ct + mq) * EKR + kq]), dqa[t]);
+      if (ct < CT) dqa[t] = mma16_add(bp, load_op<E>(&s_ekt[(16 * ct + mq) * EKR + kq]), dqa[t]);
     }
   }
 #pragma unroll
@@ -1687,6 +1687,7 @@ struct BwdBufs {
   float* dqx;      // extra keys: their part of dq, fp32 [rows, D] (null without them)
   float* dlt;      // extra keys: Delta per (token, head), fp32 [rows, nh] (null without them)
   RecArgs rec;     // column-streaming kernel's records (rec.rec null: not used)
+  bool split;      // fp32: the first kernel's scores in short chains (padded head sizes)
 };
 
 template <int HD, typename E>
@@ -1733,7 +1734,12 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
       launch_bwd_p1<HD, E, 2, false>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
                                      acc_vs, RecArgs{}, s);
   }
-  if (!h16)
+  if constexpr (sizeof(E) == 4) {
+    if (w.split)
+      launch_bwd_p1<HD, E, 4, false, true>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc,
+                                           acc_ks, acc_vs, RecArgs{}, s);
+  }
+  if (!h16 && !w.split)
     launch_bwd_p1<HD, E, 4, false>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
                                    acc_vs, RecArgs{}, s);
   if (d.extra_g > 0)
@@ -1904,7 +1910,7 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
                            const void* off, const void* ek, const void* ev, const void* out,
                            const void* dout, const float* lse, const float* dlse, void* dq,
                            void* dk, void* dv, void* doff, void* dek, void* dev, void* ws,
-                           hipStream_t s) {
+                           bool padded, hipStream_t s) {
   const int64_t rows = static_cast<int64_t>(d.B) * d.T * d.H * d.W;
   const int D = d.num_heads * d.head_dim;
   const int64_t erows = static_cast<int64_t>(d.B) * d.extra_g;
@@ -1938,6 +1944,7 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
   w.dqx = erows > 0 ? reinterpret_cast<float*>(base + L.dqx) : nullptr;
   w.dlt = erows > 0 ? reinterpret_cast<float*>(base + L.dlt) : nullptr;
   w.rec = RecArgs{};
+  w.split = padded;
   if (tiled_streams(d) && enough_columns(d)) {
     w.rec.rec = reinterpret_cast<tiled::u32x4_t*>(base + L.rec);
     w.rec.hdr = reinterpret_cast<int*>(base + L.hdr);
@@ -2005,15 +2012,15 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* v, const void* off, const void* ek, const void* ev,
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                  void* dek, void* dev, void* ws, hipStream_t s) {
+                                  void* dek, void* dev, void* ws, hipStream_t s, bool padded) {
   if (!tiled::rows_below_limit(d))
     return launch_dsa3d_bwd_direct(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
                                    dek, dev, ws, s);
   if (d.dtype == MSD_BF16)
     return bwd_tiled_typed<bf16>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
-                                 dek, dev, ws, s);
+                                 dek, dev, ws, false, s);
   return bwd_tiled_typed<float>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
-                                dek, dev, ws, s);
+                                dek, dev, ws, padded, s);
 }
 
 }  // namespace msd

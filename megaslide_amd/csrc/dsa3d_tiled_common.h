@@ -106,6 +106,22 @@ __device__ __forceinline__ f32x4_t mma16(const f32x8_t& a, const f32x8_t& b, f32
   for (int j = 0; j < 8; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
   return c;
 }
+// mma16 with fp32's 32 products in two chains of 16 that are then added to c: over many
+// blocks, one chain through c loses twice as much to rounding and more.
+__device__ __forceinline__ f32x4_t mma16_add(const bf16x8_t& a, const bf16x8_t& b, f32x4_t c) {
+  return mma16(a, b, c);
+}
+__device__ __forceinline__ f32x4_t mma16_add(const f32x8_t& a, const f32x8_t& b, f32x4_t c) {
+#pragma unroll
+  for (int h = 0; h < 8; h += 4) {
+    f32x4_t part = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = h; j < h + 4; ++j)
+      part = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], part, 0, 0, 0);
+    c += part;
+  }
+  return c;
+}
 __device__ __forceinline__ f32x16_t mma32(const bf16x8_t& a, const bf16x8_t& b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -721,6 +737,12 @@ __device__ __forceinline__ f32x4_t mma16(const PreciseOp<bf16>& a, const bf16x8_
 }
 __device__ __forceinline__ f32x4_t mma16(const PreciseOp<float>& a, const f32x8_t& b, f32x4_t c) {
   return mma16(a.v, b, c);
+}
+__device__ __forceinline__ f32x4_t mma16_add(const PreciseOp<bf16>& a, const bf16x8_t& b, f32x4_t c) {
+  return mma16(a, b, c);
+}
+__device__ __forceinline__ f32x4_t mma16_add(const PreciseOp<float>& a, const f32x8_t& b, f32x4_t c) {
+  return mma16_add(a.v, b, c);
 }
 
 }  // namespace tiled
