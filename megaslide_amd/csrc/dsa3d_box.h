@@ -610,7 +610,7 @@ __device__ __forceinline__ int box_channel(int t, int n) {
 }
 
 // acc[t] += sum over this wave's voxels v of table[q][v] * Y[v][channels], the
-// table in fixed point; blocks of 32 voxels over the waves (bf16), of 16
+// table in fixed point, or (FT) floats; blocks of 32 voxels over the waves (bf16), of 16
 // (fp32).  acc[t] register r: query 4 (lane / 16) + r, channel box_channel(t).
 //
 // bf16: the product contracts over voxels, so its B operand needs 8 voxels of
@@ -626,7 +626,6 @@ __device__ __forceinline__ int box_channel(int t, int n) {
 // the B operand's layout directly.
 // The rows of the wave's first pairs of blocks are loaded by
 // box_weighted_begin, ahead of the table's last updates and barrier.
-// HL: the table value as a bf16 (hi, lo) pair (two products) for bf16 rows.
 template <int HD, typename E>
 constexpr int box_ahead() {  // pairs of blocks in flight
   return sizeof(E) == 4 ? 0 : 1;
@@ -657,7 +656,19 @@ __device__ __forceinline__ void box_weighted_begin(const Tile& tl, __amdgpu_buff
         box_weighted_load<HD, S, E>(tl, rows, off, tl.wave + kWaves * u, ah.y[u]);
   }
 }
-template <int HD, typename S, typename E, bool RG, bool HL, typename Off>
+// 8 words of a table as a bf16 operand.
+template <bool FT>
+__device__ __forceinline__ bf16x8_t table_op(const int (&w)[8]) {
+  if constexpr (!FT) return fix_to_op<bf16>(w);
+  u32x4_t r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x2_t f = {__int_as_float(w[2 * i]), __int_as_float(w[2 * i + 1])};
+    r[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
+  }
+  return __builtin_bit_cast(bf16x8_t, r);
+}
+template <int HD, typename S, typename E, bool RG, bool FT, typename Off>
 __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
                                              const Off& off, int n, int hd, const int* table,
                                              BoxAhead<HD, E>& ah, f32x4_t (&acc)[HD / 16]) {
@@ -693,16 +704,7 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
         o0 = off(32 * pn + m) + cb;
         o1 = off(32 * pn + 16 + m) + cb;
       }
-      PreciseOp<bf16> ap;
-      bf16x8_t av;
-      if constexpr (HL) {
-        float f[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = static_cast<float>(w[i]);
-        ap = precise_op<bf16>(f);
-      } else {
-        av = fix_to_op<bf16>(w);
-      }
+      const bf16x8_t av = table_op<FT>(w);
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         f32x4_t d[2][2];
@@ -726,10 +728,7 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
                                                  __float_as_uint(d[h][j][2]), 0x07060302u);
           }
           const bf16x8_t bo = __builtin_bit_cast(bf16x8_t, b);
-          if constexpr (HL)
-            acc[2 * c + h] = mma16(ap, bo, acc[2 * c + h]);
-          else
-            acc[2 * c + h] = mma16(av, bo, acc[2 * c + h]);
+          acc[2 * c + h] = mma16(av, bo, acc[2 * c + h]);
         }
       }
     };
@@ -751,7 +750,7 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t o = off(16 * blk + 4 * g + j);
-        const float av = static_cast<float>(w[j]);
+        const float av = FT ? __int_as_float(w[j]) : static_cast<float>(w[j]);
 #pragma unroll
         for (int c = 0; c < N4; ++c) {
           float y[4];
@@ -784,7 +783,7 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
 // box_scatter), as grid_sample reads them: taken after a non-finite result, where
 // a product of a row's non-finite value and a zero weight would spoil queries
 // that do not sample the row, and the transposition the row's other channels.
-template <int HD, typename S, typename E, bool RG, typename Off>
+template <int HD, typename S, typename E, bool RG, bool FT, typename Off>
 __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
                                                   const Off& off, int n, int hd, const int* table,
                                                   f32x4_t (&acc)[HD / 16]) {
@@ -811,7 +810,7 @@ __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffe
             static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rows, at, 0, 0)));
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float f = static_cast<float>(w[r]);
+        float f = FT ? __int_as_float(w[r]) : static_cast<float>(w[r]);
         if constexpr (sizeof(E) == 2) f = to_f32(from_f32<bf16>(f));  // the products' operand
         if (w[r] != 0) acc[t][r] = __builtin_fmaf(f, y, acc[t][r]);
       }

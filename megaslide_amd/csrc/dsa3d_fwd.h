@@ -191,23 +191,27 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   f32x4_t acc[HD / 16];
 #pragma unroll
   for (int t = 0; t < HD / 16; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  auto weighted = [&](__amdgpu_buffer_rsrc_t r, const auto& off, int n, BoxAhead<HD, E>& ah) {
+  auto weighted = [&](auto floats, __amdgpu_buffer_rsrc_t r, const auto& off, int n,
+                      BoxAhead<HD, E>& ah) {
+    constexpr bool FT = decltype(floats)::value;
     if constexpr (SAFE)
-      box_weighted_safe<HD, S, E, RG>(tl, r, off, n, hd, s_tab, acc);
+      box_weighted_safe<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, acc);
     else
-      box_weighted<HD, S, E, RG, false>(tl, r, off, n, hd, s_tab, ah, acc);
+      box_weighted<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, ah, acc);
   };
   if constexpr (XK) {
     __syncthreads();  // every lane has read its extra keys' scores
+    // the weights as they are, in the units of the taps' (a key's is one number, not a sum of
+    // corners); SAFE: the smallest above 0 marks a key of weight 0
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
       if (tl.sub + kSubs * j < Gp)
-        s_tab[tl.q * kBoxRow + tl.sub + kSubs * j] =
-            SAFE && tl.sub + kSubs * j < G ? max(to_fix(se[j]), 1) : to_fix(se[j]);
+        s_val[tl.q * kBoxRow + tl.sub + kSubs * j] =
+            SAFE && tl.sub + kSubs * j < G ? fmaxf(se[j], 1e-30f) : se[j];
     __syncthreads();
     BoxAhead<HD, E> ah;
     box_weighted_begin<HD, S, E>(tl, extra_rows(a.ev), extra_off, Gp, ah);
-    weighted(extra_rows(a.ev), extra_off, Gp, ah);
+    weighted(std::true_type{}, extra_rows(a.ev), extra_off, Gp, ah);
     __syncthreads();
   }
   auto piece = [&](int s, auto only) __attribute__((always_inline)) {
@@ -227,7 +231,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
       else box_scatter<SAFE>(s_tab, bx, g, tl.q, t, sc[i]);
     }
     __syncthreads();
-    weighted(vr, row_off, bx.nv, ah);
+    weighted(std::false_type{}, vr, row_off, bx.nv, ah);
     __syncthreads();  // the products have read the table
   };
   if (bx.n == 1) {  // the usual case apart: no tap stays live through its products

@@ -130,3 +130,31 @@ def test_extra_keys_peaked_softmax_delta(algo):
         e = rel_err(t.grad.float().cpu(), r.grad)
         print(f"  {name}: {e:.2e}", flush=True)
         assert e < 8e-3, name
+
+
+@pytest.mark.parametrize("hd,dt", [(64, torch.float32), (64, torch.bfloat16), (96, torch.float32),
+                                   (40, torch.float32)])
+def test_small_weights_of_extra_keys(hd, dt):
+    """Extra keys of weight exp(-14) / (K + ...) = 6e-9 with values of 1e8: the weights are
+    floats (2^-24 of their own size each; fixed point of 2^-30 would hold 6 units of such a
+    one).  Sums of 75 taps and 8 keys: 1e-5; bf16: operands and result of 2^-9, 1e-2."""
+    from megaslide_amd import dsa3d_core
+
+    T, H, W, nh, win, G = 3, 8, 9, 2, (3, 5, 5), 8
+    N, D, K = T * H * W, 2 * hd, 75
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.zeros(1, N, nh, hd, device="cuda")
+    q[..., 0] = 1.0
+    ek = torch.zeros(1, G, nh, hd, device="cuda")
+    ek[..., 0] = -14.0 * hd ** 0.5
+    k, v = torch.zeros(1, N, D, device="cuda"), torch.zeros(1, N, D, device="cuda")
+    ev = 1e8 * (1.0 + torch.rand(1, G, D, generator=g, device="cuda"))
+    off = torch.randn(1, N, nh * K * 3, generator=g, device="cuda") * 0.5
+    ins = [t.reshape(1, -1, t.shape[-1] if t.dim() == 3 else D).to(dt) for t in (q, k, v, off)]
+    ex = [t.reshape(1, G, D).to(dt) for t in (ek, ev)]
+    p = torch.exp(ex[0].double().view(1, G, nh, hd)[..., 0] / hd ** 0.5)       # [1, G, nh]
+    ref = (p[..., None] * ex[1].double().view(1, G, nh, hd)).sum(1) / (K + p.sum(1))[..., None]
+    with torch.no_grad():
+        out = dsa3d_core(*ins, (T, H, W), nh, win, extra_k=ex[0], extra_v=ex[1])
+    err = (out.double().view(1, N, nh, hd) / ref[:, None] - 1.0).abs().max().item()
+    assert err < (1e-5 if dt == torch.float32 else 1e-2)
