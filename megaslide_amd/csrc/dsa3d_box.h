@@ -15,10 +15,11 @@
 // layer that two slabs share to the later one, so that a voxel's weight is
 // rounded to the products' element type once, as in a box of one piece.
 //
-// The box reaches one voxel past the largest lower corner on every axis, also
-// where that is outside the volume: those rows read as zero (buffer loads past
-// the end), so the corners of a tap sit at constant distances from its first,
-// and a corner outside the volume contributes 0 * 0.
+// The box ends at the volume.  A position on the last voxel of an axis is taken as the
+// voxel before it with all weight on the upper corner (the reference samples the last
+// alone: what reads a table leaves the lower corner out, box_gather), so that the
+// corners of every tap sit at constant distances from its first.  An axis of one voxel
+// has distance 0 (x: a column of zeros past it, rows that read past the end).
 #pragma once
 
 #include "dsa3d_tiled_common.h"
@@ -48,6 +49,7 @@ struct BoxPieces {
   int dz, dy, dx;        // distances of neighbours in a table row
   int nv;                // voxels of a piece
   float rlayer, rrow;    // 1 / (cm cn), 1 / cn for division-free voxel coordinates
+  bool edge;             // the box reaches a last voxel: taps may have weight 1 on it
 };
 
 // One piece: its first voxel; the taps' words (BoxTaps) count from `base` there,
@@ -114,8 +116,8 @@ __device__ __forceinline__ float half_reduce(float v) {
   return op(v, __shfl_xor(v, 16));
 }
 
-// One axis of a tap's sampling position: lower corner, upper weight, and whether
-// the position lies strictly inside the volume.  The operations and their
+// One axis of a tap's sampling position: lower corner (at most `last` = max(S - 2, 0)),
+// upper weight, and whether the position lies strictly inside the volume.  The operations and their
 // rounding are those of base_coord_rn / grid_coord_rn / axis_sample: the tap
 // index enters as an exact small float, and the halving of ((g + 1) S - 1) / 2 is
 // taken into S and 1 (a power of two, which rounding commutes with).  `o` is 0
@@ -126,13 +128,13 @@ struct AxisTap {
   bool in;
 };
 __device__ __forceinline__ AxisTap axis_tap(float pos2, float o, float bdiv, float rbdiv,
-                                            float div, float rdiv, float S) {
+                                            float div, float rdiv, float S, float last) {
 #pragma clang fp contract(off)
   const float g = (div_rn(pos2, bdiv, rbdiv) - 1.0f) + div_rn(o, div, rdiv);
   const float u = (g + 1.0f) * (0.5f * S) - 0.5f;
   // (a NaN position samples voxel 0, as fmaxf / fminf leave it)
   const float c = __builtin_amdgcn_fmed3f(u, 0.0f, S - 1.0f);
-  const float fl = floorf(c);
+  const float fl = fminf(floorf(c), last);
   AxisTap r;
   r.lo = static_cast<int>(fl);
   r.f = c - fl;
@@ -248,6 +250,8 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
   const float pz2 = static_cast<float>(2 * (tl.t - a.kt / 2));
   const float Wf = static_cast<float>(a.W), Hf = static_cast<float>(a.H),
               Tf = static_cast<float>(a.T);
+  const float Wl = static_cast<float>(max(a.W - 2, 0)), Hl = static_cast<float>(max(a.H - 2, 0)),
+              Tl = static_cast<float>(max(a.T - 2, 0));
   int zl[SLOTS], yl[SLOTS], xl[SLOTS];
   // a slot whose axis has one voxel is dropped (attention.py:118-127)
   const uint32_t kx = a.div_x > 0.0f ? ~0u : 0u, ky = a.div_y > 0.0f ? ~0u : 0u,
@@ -269,11 +273,11 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
     const float cj = floorf(__builtin_fmaf(rem, a.r_kw, h2));
     const float ck = __builtin_fmaf(-kw, cj, rem);
     const AxisTap ax = axis_tap(__builtin_fmaf(2.0f, ck, px2), raw_offset(raw, i, 0, kx) * a.offset_scale, a.bdiv_x,
-                                a.rbdiv_x, a.div_x, a.rdiv_x, Wf);
+                                a.rbdiv_x, a.div_x, a.rdiv_x, Wf, Wl);
     const AxisTap ay = axis_tap(__builtin_fmaf(2.0f, cj, py2), raw_offset(raw, i, 1, ky) * a.offset_scale, a.bdiv_y,
-                                a.rbdiv_y, a.div_y, a.rdiv_y, Hf);
+                                a.rbdiv_y, a.div_y, a.rdiv_y, Hf, Hl);
     const AxisTap az = axis_tap(__builtin_fmaf(2.0f, ci, pz2), raw_offset(raw, i, 2, kz) * a.offset_scale, a.bdiv_z,
-                                a.rbdiv_z, a.div_z, a.rdiv_z, Tf);
+                                a.rbdiv_z, a.div_z, a.rdiv_z, Tf, Tl);
     tp.fx[i] = ax.f;
     tp.fy[i] = ay.f;
     tp.fz[i] = az.f;
@@ -313,7 +317,9 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
   const int yh = -__builtin_amdgcn_readfirstlane(s_box[3]);
   bx.xlo = __builtin_amdgcn_readfirstlane(s_box[4]);
   const int xh = -__builtin_amdgcn_readfirstlane(s_box[5]);
-  const int nz = zh - bx.zlo + 2, ny = yh - bx.ylo + 2, nx = xh - bx.xlo + 2;
+  const int nz = zh - bx.zlo + (a.T > 1 ? 2 : 1), ny = yh - bx.ylo + (a.H > 1 ? 2 : 1);
+  const int nx = xh - bx.xlo + 2;
+  bx.edge = zh == a.T - 2 || yh == a.H - 2 || xh == a.W - 2;
   bx.zhi = min(zh + 1, a.T - 1);
   bx.yhi = min(yh + 1, a.H - 1);
   bx.xhi = min(xh + 1, a.W - 1);
@@ -323,13 +329,14 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
   bx.cm = ny;
   bx.cn = nx;
   if (nz * ny * nx <= kBoxCap) {
+    const int layer = nx * ny;
     bx.dx = 1;
-    bx.dy = nx;
-    bx.dz = nx * ny;
-    const int base = tl.q * kBoxRow - (bx.zlo * bx.dz + bx.ylo * nx + bx.xlo);
+    bx.dy = a.H > 1 ? nx : 0;
+    bx.dz = a.T > 1 ? layer : 0;
+    const int base = tl.q * kBoxRow - (bx.zlo * layer + bx.ylo * nx + bx.xlo);
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i)
-      tp.at[i] = static_cast<int>(__umul24(zl[i], bx.dz) + __umul24(yl[i], nx)) + xl[i] + base;
+      tp.at[i] = static_cast<int>(__umul24(zl[i], layer) + __umul24(yl[i], nx)) + xl[i] + base;
   } else {
     const bool isx = nx >= ny && nx >= nz, isy = !isx && ny >= nz;
     bx.axis = isx ? 0 : isy ? 1 : 2;
@@ -347,8 +354,8 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
     bx.n = __builtin_amdgcn_readfirstlane(bx.slabs * pm * bx.pn);
     const int layer = bx.cm * bx.cn;
     bx.dx = isx ? layer : 1;
-    bx.dy = isx ? 1 : isy ? layer : bx.cn;
-    bx.dz = isx || isy ? bx.cn : layer;
+    bx.dy = a.H == 1 ? 0 : isx ? 1 : isy ? layer : bx.cn;
+    bx.dz = a.T == 1 ? 0 : isx || isy ? bx.cn : layer;
     // column of a corner v along an axis: floor(v / (c - 1)); (v + 0.5) / d is at least
     // 0.5 / d from an integer, far above the rounding for v < 2^15
     const float rm = 1.0f / static_cast<float>(bx.cm - 1), rn = 1.0f / static_cast<float>(bx.cn - 1);
@@ -828,17 +835,27 @@ __device__ __forceinline__ void box_zero(int* table, int n4) {
 }
 
 // The tap's value interpolated from a table: lo / hi planes combined with their
-// weights (0 * value for the upper one where the position is on the plane).
+// weights (0 * value for the upper one where the position is on the plane).  EDGE:
+// where an upper weight is 1 the lower corner, which the position does not sample, is
+// replaced by the upper one (0 times a non-finite value is not 0).
+template <bool EDGE>
 __device__ __forceinline__ float box_gather(const float* table, int at, int dx, int dy, int dz,
                                             float fx, float fy, float fz) {
   const float* const p = &table[at];
   const float* const pz = p + dz;
   auto plane = [&](const float* q) {
-    const float t0 = q[0], t1 = q[dx], b0 = q[dy], b1 = q[dy + dx];
-    const float top = __builtin_fmaf(fx, t1 - t0, t0), bot = __builtin_fmaf(fx, b1 - b0, b0);
+    float t0 = q[0], t1 = q[dx], b0 = q[dy], b1 = q[dy + dx];
+    if (EDGE && fx == 1.0f) {
+      t0 = t1;
+      b0 = b1;
+    }
+    float top = __builtin_fmaf(fx, t1 - t0, t0), bot = __builtin_fmaf(fx, b1 - b0, b0);
+    if (EDGE && fy == 1.0f) top = bot;
     return __builtin_fmaf(fy, bot - top, top);
   };
-  return __builtin_fmaf(fz, plane(pz), (1.0f - fz) * plane(p));
+  const float lo = plane(p), hi = plane(pz);
+  const float v = __builtin_fmaf(fz, hi, (1.0f - fz) * lo);
+  return EDGE && fz == 1.0f ? hi : v;
 }
 
 // A tap's words as opaque values at this point: keeps the compiler from hoisting
@@ -864,20 +881,24 @@ __device__ __forceinline__ bool box_in(const BoxSeg& g, int q, BoxTap& t) {
 
 // Adds the tap's weight v (fixed-point units) to its eight corners.  TOUCH: at
 // least one unit (2^-30) each, which marks the corners of zero weight too
-// (grid_sample reads those as well: 0 times a non-finite value is not 0).
+// (grid_sample reads those as well: 0 times a non-finite value is not 0), but for
+// the lower ones where the upper weight is 1.
 template <bool TOUCH>
 __device__ __forceinline__ void box_add4(int* q, int d0, int d1, float w, float f0, float f1) {
   const float w1 = w * f1, w0 = w * (1.0f - f1), g0 = 1.0f - f0;
-  auto fix = [](float x) { return TOUCH ? max(to_fix(x), 1) : to_fix(x); };
-  atomicAdd(q, fix(w0 * g0));
-  atomicAdd(q + d0, fix(w0 * f0));
-  atomicAdd(q + d1, fix(w1 * g0));
-  atomicAdd(q + d1 + d0, fix(w1 * f0));
+  auto add = [](int* p, float x, bool read) {
+    if (!TOUCH) atomicAdd(p, to_fix(x));
+    else if (read) atomicAdd(p, max(to_fix(x), 1));
+  };
+  add(q, w0 * g0, f0 != 1.0f && f1 != 1.0f);
+  add(q + d0, w0 * f0, f1 != 1.0f);
+  add(q + d1, w1 * g0, f0 != 1.0f);
+  add(q + d1 + d0, w1 * f0, true);
 }
 template <bool TOUCH>
 __device__ __forceinline__ void box_scatter(int* table, const BoxPieces& bx, const BoxTap& t, float v) {
   int* const p = &table[t.at];
-  box_add4<TOUCH>(p, 1, bx.dy, v * (1.0f - t.fz), t.fx, t.fy);
+  if (!TOUCH || t.fz != 1.0f) box_add4<TOUCH>(p, 1, bx.dy, v * (1.0f - t.fz), t.fx, t.fy);
   box_add4<TOUCH>(p + bx.dz, 1, bx.dy, v * t.fz, t.fx, t.fy);
 }
 // The same to the corners that piece g (of several) owns: those of the tap's two
@@ -891,17 +912,21 @@ __device__ __forceinline__ void box_scatter(int* table, const BoxPieces& bx, con
   if (!(lo | hi)) return;
   const float fx = t.fx, fy = t.fy, fz = t.fz;
   float fa = fz, fm = fy, fl = fx;  // along z
+  int dm = bx.dy, dl = 1;
   if (bx.axis == 1) {
     fa = fy;
     fm = fz;
+    dm = bx.dz;
   } else if (bx.axis == 0) {
     fa = fx;
     fm = fz;
+    dm = bx.dz;
     fl = fy;
+    dl = bx.dy;
   }
   int* const p = &table[q * kBoxRow + r];
-  if (lo) box_add4<TOUCH>(p, 1, bx.cn, v * (1.0f - fa), fl, fm);
-  if (hi) box_add4<TOUCH>(p + layer, 1, bx.cn, v * fa, fl, fm);
+  if (lo && (!TOUCH || fa != 1.0f)) box_add4<TOUCH>(p, dl, dm, v * (1.0f - fa), fl, fm);
+  if (hi) box_add4<TOUCH>(p + layer, dl, dm, v * fa, fl, fm);
 }
 
 }  // namespace tiled

@@ -28,18 +28,30 @@ namespace {
 using namespace tiled;
 
 // A tap's interpolated value and its derivatives with respect to the sampling
-// coordinates, from a table.
+// coordinates, from a table (EDGE: see box_gather; the derivative along an axis with
+// upper weight 1 is masked, the position is on the volume's last voxel).
 struct TapGrad {
   float v, dx, dy, dz;
 };
+template <bool EDGE>
 __device__ __forceinline__ TapGrad box_gather_grad(const float* table, const BoxTap& t, int dx,
                                                    int dy, int dz) {
   const float* const p = &table[t.at];
   const float* const pz = p + dz;
   auto plane = [&](const float* q) {
-    return bilerp(t.fx, t.fy, q[0], q[dx], q[dy], q[dy + dx]);
+    float t0 = q[0], t1 = q[dx], b0 = q[dy], b1 = q[dy + dx];
+    if (EDGE && t.fx == 1.0f) {
+      t0 = t1;
+      b0 = b1;
+    }
+    if (EDGE && t.fy == 1.0f) {
+      t0 = b0;
+      t1 = b1;
+    }
+    return bilerp(t.fx, t.fy, t0, t1, b0, b1);
   };
-  const Bilerp lo = plane(p), hi = plane(pz);
+  Bilerp lo = plane(p), hi = plane(pz);
+  if (EDGE && t.fz == 1.0f) lo = hi;
   const float gz = 1.0f - t.fz;
   TapGrad r;
   r.v = __builtin_fmaf(t.fz, hi.val, gz * lo.val);
@@ -115,13 +127,17 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
       if constexpr (SPLIT) box_scores_split<HD, E, false>(tl, rows, row_off, bx.nv, HD, x, s_tab);
       else box_scores<HD, E, E, false, NB>(tl, rows, row_off, bx.nv, HD, x, s_tab);
       __syncthreads();
+      auto gather = [&](auto edge) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < kSlots; ++i) {
-        if (kSubs * i >= a.K) continue;
-        BoxTap t = box_tap(tp, i);
-        if (!kOnly && !box_in(g, tl.q, t)) continue;
-        tg[i] = box_gather_grad(s_tab, t, kOnly ? 1 : bx.dx, bx.dy, bx.dz);
-      }
+        for (int i = 0; i < kSlots; ++i) {
+          if (kSubs * i >= a.K) continue;
+          BoxTap t = box_tap(tp, i);
+          if (!kOnly && !box_in(g, tl.q, t)) continue;
+          tg[i] = box_gather_grad<decltype(edge)::value>(s_tab, t, kOnly ? 1 : bx.dx, bx.dy, bx.dz);
+        }
+      };
+      if (kOnly && !bx.edge) gather(std::false_type{});
+      else gather(std::true_type{});
       __syncthreads();  // the next table takes this one's place
     };
     if (bx.n == 1) {
@@ -211,9 +227,10 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
       vm += q * (bx.cm - 1);
       vl += (col - q * bx.pn) * (bx.cn - 1);
     }
-    z = bx.zlo + (bx.axis == 2 ? va : vm);
-    y = bx.ylo + (bx.axis == 2 ? vm : bx.axis == 1 ? va : vl);
-    xx = bx.xlo + (bx.axis == 0 ? va : vl);
+    // (a position on the last voxel is that voxel's, with weight 0 above it)
+    z = bx.zlo + (bx.axis == 2 ? va : vm) + (tp.fz[i] == 1.0f);
+    y = bx.ylo + (bx.axis == 2 ? vm : bx.axis == 1 ? va : vl) + (tp.fy[i] == 1.0f);
+    xx = bx.xlo + (bx.axis == 0 ? va : vl) + (tp.fx[i] == 1.0f);
   };
   int pos[kSlots];
   if constexpr (REC) {
@@ -315,13 +332,14 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
       if (rec_wide) continue;
       int z, y, xx;
       corner(i, z, y, xx);
-      const uint32_t ux = min(65535u, static_cast<uint32_t>(tp.fx[i] * 65536.0f + 0.5f));
-      const uint32_t uy = min(65535u, static_cast<uint32_t>(tp.fy[i] * 65536.0f + 0.5f));
+      auto upper = [](float f) { return f == 1.0f ? 0.0f : f; };
+      const uint32_t ux = min(65535u, static_cast<uint32_t>(upper(tp.fx[i]) * 65536.0f + 0.5f));
+      const uint32_t uy = min(65535u, static_cast<uint32_t>(upper(tp.fy[i]) * 65536.0f + 0.5f));
       u32x4_t r;
       r[0] = static_cast<uint32_t>(y) | (static_cast<uint32_t>(xx) << 14) |
              (static_cast<uint32_t>(tl.q) << 28);
       r[1] = ux | (uy << 16);
-      r[2] = __float_as_uint(tp.fz[i]);
+      r[2] = __float_as_uint(upper(tp.fz[i]));
       r[3] = pair;
       rec[s_bin[kRecBins + z - bx.zlo] + pos[i]] = r;
     }

@@ -22,6 +22,9 @@ CASES = [
     (40, 5, 1, 1, (5, 7, 4), 9.0),     # a unit axis, a long one, 140 taps
     (1, 3, 70, 2, (1, 4, 40), 2.0),    # 160 taps, wide and flat
     (6, 1, 9, 1, (3, 1, 11), 1.0),     # 33 taps
+    (2, 15, 18, 1, (3, 7, 7), 3.0),    # two frames: every box ends at the volume
+    (1, 45, 60, 1, (3, 7, 7), 12.0),   # one frame, cut
+    (14, 1, 90, 1, (3, 1, 7), 30.0),   # one row, cut
 ]
 
 
