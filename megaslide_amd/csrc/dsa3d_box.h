@@ -49,7 +49,7 @@ struct BoxPieces {
   int dz, dy, dx;        // distances of neighbours in a table row
   int nv;                // voxels of a piece
   float rlayer, rrow;    // 1 / (cm cn), 1 / cn for division-free voxel coordinates
-  bool edge;             // the box reaches a last voxel: taps may have weight 1 on it
+  bool edge;             // taps may have weight 1 on a last voxel, or there is one frame
 };
 
 // One piece: its first voxel; the taps' words (BoxTaps) count from `base` there,
@@ -319,7 +319,7 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
   const int xh = -__builtin_amdgcn_readfirstlane(s_box[5]);
   const int nz = zh - bx.zlo + (a.T > 1 ? 2 : 1), ny = yh - bx.ylo + (a.H > 1 ? 2 : 1);
   const int nx = xh - bx.xlo + 2;
-  bx.edge = zh == a.T - 2 || yh == a.H - 2 || xh == a.W - 2;
+  bx.edge = zh == a.T - 2 || yh == a.H - 2 || xh == a.W - 2 || a.T == 1;
   bx.zhi = min(zh + 1, a.T - 1);
   bx.yhi = min(yh + 1, a.H - 1);
   bx.xhi = min(xh + 1, a.W - 1);
@@ -631,36 +631,34 @@ __device__ __forceinline__ int box_channel(int t, int n) {
 // box_weighted_safe then.)
 // fp32: a 16x16x4 product takes one voxel per lane group, so rows are loaded in
 // the B operand's layout directly.
-// The rows of the wave's first pairs of blocks are loaded by
+// The rows of the wave's first pair of blocks are loaded by
 // box_weighted_begin, ahead of the table's last updates and barrier.
-template <int HD, typename E>
-constexpr int box_ahead() {  // pairs of blocks in flight
-  return sizeof(E) == 4 ? 0 : 1;
+// bf16: over the groups C0 .. C1 - 1 of 32 channels.  A caller that keeps its taps over
+// the call (KEEP) takes fewer groups at a time: registers beside the accumulators (HD / 4)
+// are 8 a group for the rows in flight, ~50 for the transposition, the table's operand and
+// addresses, and ~30 for the taps (and extra keys, XK), of 128.
+template <int HD, bool KEEP, bool XK>
+constexpr int box_groups() {
+  return !KEEP || HD == 32 ? HD / 32 : XK ? 1 : 2;
 }
-template <int HD, typename E>
+template <int N, typename E>
 struct BoxAhead {
-  bf16x8_t y[box_ahead<HD, E>() > 0 ? box_ahead<HD, E>() : 1][HD / 32][2];
+  bf16x8_t y[sizeof(E) == 4 ? 1 : N][2];
 };
-template <int HD, typename S, typename E, typename Off>
-__device__ __forceinline__ void box_weighted_load(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
-                                                  const Off& off, int p, bf16x8_t (&y)[HD / 32][2]) {
-  const uint32_t cb = static_cast<uint32_t>(8 * (tl.lane >> 4)) * sizeof(S);
-  const uint32_t o0 = off(32 * p + (tl.lane & 15)) + cb, o1 = off(32 * p + 16 + (tl.lane & 15)) + cb;
-#pragma unroll
-  for (int c = 0; c < HD / 32; ++c) {
-    y[c][0] = buf_op<S, E>(rows, o0, 64 * c);
-    y[c][1] = buf_op<S, E>(rows, o1, 64 * c);
-  }
-}
-template <int HD, typename S, typename E, typename Off>
+template <int N, typename S, typename E, typename Off>
 __device__ __forceinline__ void box_weighted_begin(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
-                                                   const Off& off, int n, BoxAhead<HD, E>& ah) {
+                                                   const Off& off, int n, int c0,
+                                                   BoxAhead<N, E>& ah) {
   if constexpr (sizeof(E) == 2) {
-    const int np = (n + 31) >> 5;
+    if (tl.wave >= (n + 31) >> 5) return;
+    const uint32_t cb = static_cast<uint32_t>(8 * (tl.lane >> 4) + 32 * c0) * sizeof(S);
+    const int v = 32 * tl.wave + (tl.lane & 15);
+    const uint32_t o0 = off(v) + cb, o1 = off(v + 16) + cb;
 #pragma unroll
-    for (int u = 0; u < box_ahead<HD, E>(); ++u)
-      if (tl.wave + kWaves * u < np)
-        box_weighted_load<HD, S, E>(tl, rows, off, tl.wave + kWaves * u, ah.y[u]);
+    for (int c = 0; c < N; ++c) {
+      ah.y[c][0] = buf_op<S, E>(rows, o0, 64 * c);
+      ah.y[c][1] = buf_op<S, E>(rows, o1, 64 * c);
+    }
   }
 }
 // 8 words of a table as a bf16 operand.
@@ -675,13 +673,12 @@ __device__ __forceinline__ bf16x8_t table_op(const int (&w)[8]) {
   }
   return __builtin_bit_cast(bf16x8_t, r);
 }
-template <int HD, typename S, typename E, bool RG, bool FT, typename Off>
+template <int HD, typename S, typename E, bool RG, bool FT, int C0, int C1, typename Off>
 __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
                                              const Off& off, int n, int hd, const int* table,
-                                             BoxAhead<HD, E>& ah, f32x4_t (&acc)[HD / 16]) {
+                                             BoxAhead<C1 - C0, E>& ah, f32x4_t (&acc)[HD / 16]) {
   const int m = tl.lane & 15, g = tl.lane >> 4;
   if constexpr (sizeof(E) == 2) {
-    constexpr int NC = HD / 32, U = box_ahead<HD, E>();
     static_assert(!RG, "bf16 products take whole 32-channel groups");
     // selection operands: lane (n, g) holds rows k = 8 g + [0, 8) of column n,
     // one where k = n (first 16 channels) or n + 16 (second)
@@ -696,15 +693,17 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
       }
       sel[h] = __builtin_bit_cast(bf16x8_t, w);
     }
-    const uint32_t cb = static_cast<uint32_t>(8 * g) * sizeof(S);
+    const uint32_t cb = static_cast<uint32_t>(8 * g + 32 * C0) * sizeof(S);
     const int np = (n + 31) >> 5;
     const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto step = [&](int p, bf16x8_t (&y)[NC][2]) {
+    auto& y = ah.y;
+#pragma nounroll
+    for (int p = tl.wave; p < np; p += kWaves) {
       const int* const tr = &table[m * kBoxRow + 32 * p + 4 * g];
       int w[8];
       __builtin_memcpy(&w[0], tr, 16);
       __builtin_memcpy(&w[4], tr + 16, 16);
-      const int pn = p + U * kWaves;
+      const int pn = p + kWaves;
       const bool more = pn < np;
       uint32_t o0 = kNoRow, o1 = kNoRow;
       if (more) {
@@ -713,19 +712,13 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
       }
       const bf16x8_t av = table_op<FT>(w);
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
+      for (int c = 0; c < C1 - C0; ++c) {
         f32x4_t d[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        auto transpose = [&](int h) {
           d[h][0] = mma16(y[c][0], sel[h], zero);
           d[h][1] = mma16(y[c][1], sel[h], zero);
-        }
-        if (more) {  // later blocks' rows take these registers
-          y[c][0] = buf_op<S, E>(rows, o0, 64 * c);
-          y[c][1] = buf_op<S, E>(rows, o1, 64 * c);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        };
+        auto product = [&](int h) {
           u32x4_t b;
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
@@ -735,15 +728,17 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
                                                  __float_as_uint(d[h][j][2]), 0x07060302u);
           }
           const bf16x8_t bo = __builtin_bit_cast(bf16x8_t, b);
-          acc[2 * c + h] = mma16(av, bo, acc[2 * c + h]);
+          acc[2 * (C0 + c) + h] = mma16(av, bo, acc[2 * (C0 + c) + h]);
+        };
+        transpose(0);
+        if (C1 - C0 < HD / 32) product(0);  // (with the taps in registers)
+        transpose(1);
+        if (more) {  // later blocks' rows take these registers
+          y[c][0] = buf_op<S, E>(rows, o0, 64 * c);
+          y[c][1] = buf_op<S, E>(rows, o1, 64 * c);
         }
-      }
-    };
-#pragma nounroll
-    for (int p = tl.wave; p < np; p += U * kWaves) {
-      step(p, ah.y[0]);
-      if constexpr (U == 2) {
-        if (p + kWaves < np) step(p + kWaves, ah.y[1]);
+        if (C1 - C0 == HD / 32) product(0);
+        product(1);
       }
     }
   } else {
@@ -821,6 +816,7 @@ __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffe
         if constexpr (sizeof(E) == 2) f = to_f32(from_f32<bf16>(f));  // the products' operand
         if (w[r] != 0) acc[t][r] = __builtin_fmaf(f, y, acc[t][r]);
       }
+      __builtin_amdgcn_sched_barrier(0);  // one load at a time: the caller keeps its taps
     }
   }
 }
@@ -853,7 +849,9 @@ __device__ __forceinline__ float box_gather(const float* table, int at, int dx, 
     if (EDGE && fy == 1.0f) top = bot;
     return __builtin_fmaf(fy, bot - top, top);
   };
-  const float lo = plane(p), hi = plane(pz);
+  const float lo = plane(p);
+  if (EDGE && dz == 0) return lo;  // one frame (uniform)
+  const float hi = plane(pz);
   const float v = __builtin_fmaf(fz, hi, (1.0f - fz) * lo);
   return EDGE && fz == 1.0f ? hi : v;
 }
@@ -899,7 +897,7 @@ template <bool TOUCH>
 __device__ __forceinline__ void box_scatter(int* table, const BoxPieces& bx, const BoxTap& t, float v) {
   int* const p = &table[t.at];
   if (!TOUCH || t.fz != 1.0f) box_add4<TOUCH>(p, 1, bx.dy, v * (1.0f - t.fz), t.fx, t.fy);
-  box_add4<TOUCH>(p + bx.dz, 1, bx.dy, v * t.fz, t.fx, t.fy);
+  if (bx.dz != 0) box_add4<TOUCH>(p + bx.dz, 1, bx.dy, v * t.fz, t.fx, t.fy);
 }
 // The same to the corners that piece g (of several) owns: those of the tap's two
 // layers along the axis that lie in it.

@@ -50,7 +50,9 @@ __device__ __forceinline__ TapGrad box_gather_grad(const float* table, const Box
     }
     return bilerp(t.fx, t.fy, t0, t1, b0, b1);
   };
-  Bilerp lo = plane(p), hi = plane(pz);
+  Bilerp lo = plane(p);
+  if (EDGE && dz == 0) return TapGrad{lo.val, lo.dx, lo.dy, 0.0f};  // one frame (uniform)
+  const Bilerp hi = plane(pz);
   if (EDGE && t.fz == 1.0f) lo = hi;
   const float gz = 1.0f - t.fz;
   TapGrad r;

@@ -44,15 +44,16 @@ constexpr int fwd_min_waves() {
   return sizeof(E) == 4 && HD > 64 ? 2 : 4;
 }
 
-// S: storage, E: element type of the products.  XK: extra keys (a.G > 0).
+// S: storage, E: element type of the products.  EPL: extra keys a lane holds (0: none).
 // RG: head_dim hd below HD (a multiple of 8), channels past it read as zero.
 // SAFE: the weighted sum by plain arithmetic.
 // Returns whether a sum was not finite.
-template <int HD, typename S, typename E, bool XK, bool RG, bool DROP, bool SAFE>
+template <int HD, typename S, typename E, int EPL, bool RG, bool DROP, bool SAFE>
 __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
                                          float* __restrict__ lse, int hd_arg, unsigned tid,
                                          int* s_tab, uint32_t* s_row, int* s_box,
                                          float* s_qnan) {
+  constexpr bool XK = EPL > 0;
   float* const s_val = reinterpret_cast<float*>(s_tab);
   const int hd = RG ? hd_arg : HD;
 
@@ -87,7 +88,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   auto extra_off = [&](int g) {
     return g < G ? static_cast<uint32_t>(g * static_cast<int>(D * sizeof(S))) : kNoRow;
   };
-  constexpr int NB = box_score_blocks<HD, E>();
+  constexpr int NB = SAFE ? 2 : box_score_blocks<HD, E>();
   auto scores = [&](__amdgpu_buffer_rsrc_t r, const auto& off, int n) {
     if constexpr (RG) box_scores_split<HD, S, RG>(tl, r, off, n, hd, qx, s_val);
     else box_scores<HD, S, E, RG, NB>(tl, r, off, n, hd, qx, s_val);
@@ -129,8 +130,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
 
   // ---- extra keys (attention.py:160-173): lane `sub` of a query takes keys
   // sub + 32 j ------------------------------------------------------------------
-  constexpr int EPL = XK ? kMaxExtra / kSubs : 1;
-  float se[EPL];
+  float se[XK ? EPL : 1];
   if constexpr (XK) {
     scores(extra_rows(a.ek), extra_off, Gp);
     __syncthreads();
@@ -139,6 +139,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
       const int g = tl.sub + kSubs * j;
       se[j] = g < G ? s_val[tl.q * kBoxRow + g] * a.softmax_scale : -INFINITY;
     }
+    __syncthreads();  // the weights take the table
   }
 
   // ---- softmax over each query's taps (32 lanes x kSlots) and extra keys ----
@@ -196,47 +197,49 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   f32x4_t acc[HD / 16];
 #pragma unroll
   for (int t = 0; t < HD / 16; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  auto weighted = [&](auto floats, __amdgpu_buffer_rsrc_t r, const auto& off, int n,
-                      BoxAhead<HD, E>& ah) {
+  // begin: loads of the first rows; fill: what the table still needs, barriers included.
+  // taps: whether the caller keeps its taps over the call
+  auto weighted = [&](auto floats, auto taps, __amdgpu_buffer_rsrc_t r, const auto& off, int n,
+                      const auto& fill) __attribute__((always_inline)) {
     constexpr bool FT = decltype(floats)::value;
-    if constexpr (SAFE)
+    constexpr int NC = HD / 32;
+    constexpr int C = sizeof(E) == 2 ? box_groups<HD, decltype(taps)::value, XK>() : NC;
+    if constexpr (SAFE) {
+      fill();
       box_weighted_safe<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, acc);
-    else
-      box_weighted<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, ah, acc);
+    } else {
+      auto pass = [&](auto first) __attribute__((always_inline)) {
+        constexpr int C0 = decltype(first)::value, C1 = C0 + C < NC ? C0 + C : NC;
+        if constexpr (C0 < NC) {
+          BoxAhead<C1 - C0, E> ah;
+          box_weighted_begin<C1 - C0, S, E>(tl, r, off, n, C0, ah);
+          if (C0 == 0) fill();
+          box_weighted<HD, S, E, RG, FT, C0, C1>(tl, r, off, n, hd, s_tab, ah, acc);
+        }
+      };
+      pass(std::integral_constant<int, 0>{});
+      pass(std::integral_constant<int, C>{});
+      pass(std::integral_constant<int, 2 * C>{});
+      pass(std::integral_constant<int, 3 * C>{});
+    }
   };
-  if constexpr (XK) {
-    __syncthreads();  // every lane has read its extra keys' scores
-    // the weights as they are, in the units of the taps' (a key's is one number, not a sum of
-    // corners); SAFE: the smallest above 0 marks a key of weight 0
-#pragma unroll
-    for (int j = 0; j < EPL; ++j)
-      if (tl.sub + kSubs * j < Gp)
-        s_val[tl.q * kBoxRow + tl.sub + kSubs * j] =
-            SAFE && tl.sub + kSubs * j < G ? fmaxf(se[j], 1e-30f) : se[j];
-    __syncthreads();
-    BoxAhead<HD, E> ah;
-    box_weighted_begin<HD, S, E>(tl, extra_rows(a.ev), extra_off, Gp, ah);
-    weighted(std::true_type{}, extra_rows(a.ev), extra_off, Gp, ah);
-    __syncthreads();
-  }
   auto piece = [&](int s, auto only) __attribute__((always_inline)) {
     constexpr bool kOnly = decltype(only)::value;
     const BoxSeg g = box_seg(bx, s);
     if (!kOnly || a.vs != a.ks) set_rows(g, a.vs);  // else as the scores left them
-    BoxAhead<HD, E> ah;
-    box_weighted_begin<HD, S, E>(tl, vr, row_off, bx.nv, ah);
-    box_zero(s_tab, ((bx.nv + 31) & ~31) >> 2);
-    __syncthreads();
+    weighted(std::false_type{}, std::bool_constant<!kOnly || XK>{}, vr, row_off, bx.nv, [&] {
+      box_zero(s_tab, ((bx.nv + 31) & ~31) >> 2);
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      if (kSubs * i >= a.K) continue;
-      if (SAFE && !has_tap(i)) continue;  // (a copy of another lane's tap)
-      const BoxTap t = box_tap(tp, i);
-      if constexpr (kOnly) box_scatter<SAFE>(s_tab, bx, t, sc[i]);
-      else box_scatter<SAFE>(s_tab, bx, g, tl.q, t, sc[i]);
-    }
-    __syncthreads();
-    weighted(std::false_type{}, vr, row_off, bx.nv, ah);
+      for (int i = 0; i < kSlots; ++i) {
+        if (kSubs * i >= a.K) continue;
+        if (SAFE && !has_tap(i)) continue;  // (a copy of another lane's tap)
+        const BoxTap t = box_tap(tp, i);
+        if constexpr (kOnly) box_scatter<SAFE>(s_tab, bx, t, sc[i]);
+        else box_scatter<SAFE>(s_tab, bx, g, tl.q, t, sc[i]);
+      }
+      __syncthreads();
+    });
     __syncthreads();  // the products have read the table
   };
   if (bx.n == 1) {  // the usual case apart: no tap stays live through its products
@@ -244,6 +247,19 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   } else {
 #pragma nounroll
     for (int s = 0; s < bx.n; ++s) piece(s, std::false_type{});
+  }
+  if constexpr (XK) {
+    // (after the taps, which are not kept over these products then)  The weights as they
+    // are, in the units of the taps' (a key's is one number, not a sum of corners); SAFE:
+    // the smallest above 0 marks a key of weight 0
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      if (tl.sub + kSubs * j < Gp)
+        s_val[tl.q * kBoxRow + tl.sub + kSubs * j] =
+            SAFE && tl.sub + kSubs * j < G ? fmaxf(se[j], 1e-30f) : se[j];
+    __syncthreads();
+    weighted(std::true_type{}, std::false_type{}, extra_rows(a.ev), extra_off, Gp, [] {});
+    __syncthreads();
   }
   // partial O of wave w: [w][query][channel]
   static_assert(kWaves * kTQ * HD <= kTQ * kBoxRow, "the partial sums fit the table");
@@ -275,7 +291,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
 // and (bf16) over its channels.  The tile is then done again with the sum by
 // plain arithmetic over what each query samples (from the start, so that nothing
 // is kept live for it).  Whole-head fp32 products (32, 64, 96, 128) go without.
-template <int HD, typename S, typename E, bool XK, bool RG, bool DROP>
+template <int HD, typename S, typename E, int EPL, bool RG, bool DROP>
 __global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_box_kernel(
     Args a, S* __restrict__ out, float* __restrict__ lse, int hd) {
   __shared__ __attribute__((aligned(16))) int s_tab[kTQ * kBoxRow];
@@ -288,7 +304,7 @@ __global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_
   if (box_unit(a) < 0) return;  // the grid is rounded up to the 8 XCDs
   constexpr bool kCheck = sizeof(E) == 2 || RG;
   if (kCheck && threadIdx.x == 0) s_bad = 0;
-  const bool bad = fwd_tile<HD, S, E, XK, RG, DROP, false>(a, out, lse, hd, threadIdx.x, s_tab,
+  const bool bad = fwd_tile<HD, S, E, EPL, RG, DROP, false>(a, out, lse, hd, threadIdx.x, s_tab,
                                                             s_row, s_box, s_qnan);
   if constexpr (kCheck) {
     if (__builtin_amdgcn_ballot_w64(bad) != 0 && (threadIdx.x & 63) == 0) s_bad = 1;
@@ -306,7 +322,7 @@ __global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_
     asm volatile("" : "+v"(tid), "+s"(kp));
     KernArgs k;
     __builtin_memcpy(&k, (const void*)kp, sizeof(k));
-    fwd_tile<HD, S, E, XK, RG, DROP, true>(k.a, k.out, k.lse, k.hd, tid, s_tab, s_row, s_box,
+    fwd_tile<HD, S, E, EPL, RG, DROP, true>(k.a, k.out, k.lse, k.hd, tid, s_tab, s_row, s_box,
                                            s_qnan);
   }
 }
@@ -317,13 +333,19 @@ hipError_t fwd_typed(const msd_dsa3d_desc& d, const Args& a, void* out, float* l
   const dim3 block(kThreads);
   S* const o = static_cast<S*>(out);
   auto go = [&]<int HD>() {
-    auto run = [&]<bool XK, bool DROP>() {
-      hipLaunchKernelGGL((dsa3d_fwd_box_kernel<HD, S, E, XK, RG, DROP>), grid, block, 0, s, a, o,
+    auto run = [&]<int EPL, bool DROP>() {
+      hipLaunchKernelGGL((dsa3d_fwd_box_kernel<HD, S, E, EPL, RG, DROP>), grid, block, 0, s, a, o,
                          lse, d.head_dim);
     };
     const bool drop = a.drop.threshold != 0;
-    if (a.G > 0) drop ? run.template operator()<true, true>() : run.template operator()<true, false>();
-    else drop ? run.template operator()<false, true>() : run.template operator()<false, false>();
+    // lanes hold the keys' weights in registers: half as many for up to 128 keys
+    constexpr int kMost = kMaxExtra / kSubs;
+    auto keys = [&]<int EPL>() {
+      drop ? run.template operator()<EPL, true>() : run.template operator()<EPL, false>();
+    };
+    if (a.G == 0) keys.template operator()<0>();
+    else if (a.G <= kSubs * kMost / 2) keys.template operator()<kMost / 2>();
+    else keys.template operator()<kMost>();
   };
   if (d.head_dim <= 32) go.template operator()<32>();
   else if (d.head_dim <= 64) go.template operator()<64>();
