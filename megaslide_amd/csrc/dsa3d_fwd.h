@@ -106,18 +106,25 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
       set_rows(g, a.ks);
       scores(kr, row_off, bx.nv);
       __syncthreads();
-      auto gather = [&](auto edge) __attribute__((always_inline)) {
+      auto gather = [&](auto edge, auto dx, auto dy) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kSlots; ++i) {
           if (kSubs * i >= a.K) continue;
           BoxTap t = box_tap(tp, i);
           if (!kOnly && !box_in(g, tl.q, t)) continue;
-          sc[i] = box_gather<decltype(edge)::value>(s_val, t.at, kOnly ? 1 : bx.dx, bx.dy, bx.dz,
-                                                    t.fx, t.fy, t.fz);
+          sc[i] = box_gather<decltype(edge)::value>(s_val, t.at, dx, dy, bx.dz, t.fx, t.fy, t.fz);
         }
       };
-      if (kOnly && !bx.edge) gather(std::false_type{});
-      else gather(std::true_type{});
+      // neighbours at distance 1 along x, or along y in slabs along x, come in one read
+      constexpr std::integral_constant<int, 1> kNext{};
+      if (kOnly || bx.axis != 0) {
+        if (bx.edge) gather(std::true_type{}, kNext, bx.dy);
+        else gather(std::false_type{}, kNext, bx.dy);
+      } else if (bx.edge || a.H == 1) {
+        gather(std::true_type{}, bx.dx, bx.dy);
+      } else {
+        gather(std::false_type{}, bx.dx, kNext);
+      }
       __syncthreads();  // the next piece, the extra keys or the weights take the table
     };
     if (bx.n == 1) {
