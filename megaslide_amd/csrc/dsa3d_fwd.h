@@ -177,24 +177,26 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   }
   den = half_reduce<false>(den);
   const float inv_den = 1.0f / den;
+  // a query past the grid's edge weighs nothing (its lanes hold copies of the tile's taps),
+  // nor does one with a score that is not finite (its output is NaN: s_qnan)
+  const bool weighs = tl.q_ok && den == den;
 #pragma unroll
   for (int i = 0; i < kSlots; ++i) {
     // p times its dropout factor, in fixed-point units
     const float f = !DROP ? 1.0f : ((tp.flags >> (4 * i)) & 8u) ? 0.0f : a.drop.scale;
-    sc[i] *= inv_den * f * a.fix_a;
+    sc[i] = weighs ? sc[i] * (inv_den * f * a.fix_a) : 0.0f;
   }
   if (tl.sub == 0) {
     s_qnan[tl.q] = den == den ? 1.0f : __builtin_nanf("");
     if (lse != nullptr && tl.q_ok) lse[tl.qn * a.nh + tl.head] = mx + logf(den);
   }
   if constexpr (XK) {
-    // the keys' weights, in fixed-point units
+    // the keys' weights, in the units of the taps'
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
       const int g = tl.sub + kSubs * j;
-      se[j] = g < G ? se[j] * inv_den * a.fix_a *
-                            (DROP ? dropout_factor(a.drop, tl.qn, tl.head, a.K + g) : 1.0f)
-                      : 0.0f;
+      const float f = DROP ? dropout_factor(a.drop, tl.qn, tl.head, a.K + g) : 1.0f;
+      se[j] = g < G && weighs ? se[j] * inv_den * a.fix_a * f : 0.0f;
     }
   }
 
