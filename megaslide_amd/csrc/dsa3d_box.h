@@ -236,7 +236,9 @@ __device__ __forceinline__ void box_init(int* s_box) {
   if (threadIdx.x < 8) s_box[threadIdx.x] = 0x7fffffff;
 }
 
-template <typename S, int SLOTS, bool MASK, bool DROP>
+// CLAMP: an infinite offset samples the volume's face (div_rn makes it NaN, which
+// samples voxel 0), as any offset beyond 10^30 does.
+template <typename S, int SLOTS, bool MASK, bool DROP, bool CLAMP>
 __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
                                           const RawOffsets<S, SLOTS>& raw, BoxTaps<SLOTS>& tp,
                                           BoxPieces& bx, int* s_box) {
@@ -272,12 +274,16 @@ __device__ __forceinline__ void box_setup(const Args& a, const Tile& tl,
     const float rem = __builtin_fmaf(-khkw, ci, kf);
     const float cj = floorf(__builtin_fmaf(rem, a.r_kw, h2));
     const float ck = __builtin_fmaf(-kw, cj, rem);
-    const AxisTap ax = axis_tap(__builtin_fmaf(2.0f, ck, px2), raw_offset(raw, i, 0, kx) * a.offset_scale, a.bdiv_x,
-                                a.rbdiv_x, a.div_x, a.rdiv_x, Wf, Wl);
-    const AxisTap ay = axis_tap(__builtin_fmaf(2.0f, cj, py2), raw_offset(raw, i, 1, ky) * a.offset_scale, a.bdiv_y,
-                                a.rbdiv_y, a.div_y, a.rdiv_y, Hf, Hl);
-    const AxisTap az = axis_tap(__builtin_fmaf(2.0f, ci, pz2), raw_offset(raw, i, 2, kz) * a.offset_scale, a.bdiv_z,
-                                a.rbdiv_z, a.div_z, a.rdiv_z, Tf, Tl);
+    auto offset = [&](int j, uint32_t keep) {
+      const float o = raw_offset(raw, i, j, keep) * a.offset_scale;
+      return CLAMP ? __builtin_amdgcn_fmed3f(o, -1e30f, 1e30f) : o;
+    };
+    const AxisTap ax = axis_tap(__builtin_fmaf(2.0f, ck, px2), offset(0, kx), a.bdiv_x, a.rbdiv_x,
+                                a.div_x, a.rdiv_x, Wf, Wl);
+    const AxisTap ay = axis_tap(__builtin_fmaf(2.0f, cj, py2), offset(1, ky), a.bdiv_y, a.rbdiv_y,
+                                a.div_y, a.rdiv_y, Hf, Hl);
+    const AxisTap az = axis_tap(__builtin_fmaf(2.0f, ci, pz2), offset(2, kz), a.bdiv_z, a.rbdiv_z,
+                                a.div_z, a.rdiv_z, Tf, Tl);
     tp.fx[i] = ax.f;
     tp.fy[i] = ay.f;
     tp.fz[i] = az.f;
@@ -784,11 +790,13 @@ __device__ __forceinline__ void box_weighted(const Tile& tl, __amdgpu_buffer_rsr
 // acc), over the voxels a query's taps touch (a non-zero table entry: see
 // box_scatter), as grid_sample reads them: taken after a non-finite result, where
 // a product of a row's non-finite value and a zero weight would spoil queries
-// that do not sample the row, and the transposition the row's other channels.
+// that do not sample the row, and the transposition the row's other channels.  `unit`:
+// the weights' unit (the products take it off the sum, where large values times 2^30
+// overflow).
 template <int HD, typename S, typename E, bool RG, bool FT, typename Off>
 __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffer_rsrc_t rows,
                                                   const Off& off, int n, int hd, const int* table,
-                                                  f32x4_t (&acc)[HD / 16]) {
+                                                  float unit, f32x4_t (&acc)[HD / 16]) {
   const int m = tl.lane & 15, g = tl.lane >> 4;
 #pragma nounroll
   for (int e = 0;; ++e) {  // the wave's voxels: pairs w, w + 8, ... of blocks
@@ -814,6 +822,7 @@ __device__ __forceinline__ void box_weighted_safe(const Tile& tl, __amdgpu_buffe
       for (int r = 0; r < 4; ++r) {
         float f = FT ? __int_as_float(w[r]) : static_cast<float>(w[r]);
         if constexpr (sizeof(E) == 2) f = to_f32(from_f32<bf16>(f));  // the products' operand
+        f *= unit;
         if (w[r] != 0) acc[t][r] = __builtin_fmaf(f, y, acc[t][r]);
       }
       __builtin_amdgcn_sched_barrier(0);  // one load at a time: the caller keeps its taps
@@ -854,6 +863,23 @@ __device__ __forceinline__ float box_gather(const float* table, int at, int dx, 
   const float hi = plane(pz);
   const float v = __builtin_fmaf(fz, hi, (1.0f - fz) * lo);
   return EDGE && fz == 1.0f ? hi : v;
+}
+
+// The same as the reference sums it, corner by corner of those it reads: a score that is
+// infinite stays so (differences of table entries would make it NaN).
+__device__ __forceinline__ float box_gather_safe(const float* table, int at, int dx, int dy, int dz,
+                                                 float fx, float fy, float fz) {
+  float s = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const bool hx = c & 1, hy = c & 2, hz = c & 4;
+    if (hz && dz == 0 || hy && dy == 0) continue;  // one frame, one row (uniform)
+    const float w = (hz ? fz : 1.0f - fz) * (hy ? fy : 1.0f - fy) * (hx ? fx : 1.0f - fx);
+    const bool read = (hx || fx != 1.0f) && (hy || fy != 1.0f) && (hz || fz != 1.0f);
+    const float t = table[at + (hz ? dz : 0) + (hy ? dy : 0) + (hx ? dx : 0)];
+    if (read) s = __builtin_fmaf(w, t, s);
+  }
+  return s;
 }
 
 // A tap's words as opaque values at this point: keeps the compiler from hoisting

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
     box_init(s_box);
     if (REC && threadIdx.x < kRecBins) s_bin[threadIdx.x] = 0;
     __syncthreads();
-    box_setup<E, kSlots, true, DROP>(a, tl, raw, tp, bx, s_box);
+    box_setup<E, kSlots, true, DROP, false>(a, tl, raw, tp, bx, s_box);
   }
   {
     // The second kernel adds dK and dV into accumulator rows (the fp32 outputs

@@ -47,7 +47,7 @@ constexpr int fwd_min_waves() {
 // S: storage, E: element type of the products.  EPL: extra keys a lane holds (0: none).
 // RG: head_dim hd below HD (a multiple of 8), channels past it read as zero.
 // SAFE: the weighted sum by plain arithmetic.
-// Returns whether a sum was not finite.
+// Returns whether a sum (RG: or a score) was not finite.
 template <int HD, typename S, typename E, int EPL, bool RG, bool DROP, bool SAFE>
 __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
                                          float* __restrict__ lse, int hd_arg, unsigned tid,
@@ -65,9 +65,16 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   // the tile's q rows load while the taps are set up
   op_t<E> qx[HD / 32];
   box_tile_rows<HD, S, E, RG>(a, tl, static_cast<const S*>(a.q), a.qs, hd, qx);
+  // (a score below the type's limit whose terms are beyond it: q times a power of two)
+  constexpr float kDown = SAFE && RG ? 0x1p-16f : 1.0f;
+  if constexpr (SAFE && RG) {
+#pragma unroll
+    for (int c = 0; c < HD / 32; ++c) qx[c] *= kDown;
+  }
+  const float scale = a.softmax_scale * (1.0f / kDown);
   BoxTaps<kSlots> tp;
   BoxPieces bx;
-  box_setup<S, kSlots, false, DROP>(a, tl, raw, tp, bx, s_box);
+  box_setup<S, kSlots, false, DROP, RG>(a, tl, raw, tp, bx, s_box);
 
   auto rows_of = [&](const void* base, int64_t stride) {
     const S* p = static_cast<const S*>(base) + tl.sample0 * stride + static_cast<int64_t>(tl.head) * hd;
@@ -112,12 +119,17 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
           if (kSubs * i >= a.K) continue;
           BoxTap t = box_tap(tp, i);
           if (!kOnly && !box_in(g, tl.q, t)) continue;
-          sc[i] = box_gather<decltype(edge)::value>(s_val, t.at, dx, dy, bx.dz, t.fx, t.fy, t.fz);
+          if constexpr (SAFE && RG)
+            sc[i] = box_gather_safe(s_val, t.at, dx, dy, bx.dz, t.fx, t.fy, t.fz);
+          else
+            sc[i] = box_gather<decltype(edge)::value>(s_val, t.at, dx, dy, bx.dz, t.fx, t.fy, t.fz);
         }
       };
       // neighbours at distance 1 along x, or along y in slabs along x, come in one read
       constexpr std::integral_constant<int, 1> kNext{};
-      if (kOnly || bx.axis != 0) {
+      if constexpr (SAFE) {
+        gather(std::true_type{}, bx.dx, bx.dy);
+      } else if (kOnly || bx.axis != 0) {
         if (bx.edge) gather(std::true_type{}, kNext, bx.dy);
         else gather(std::false_type{}, kNext, bx.dy);
       } else if (bx.edge || a.H == 1) {
@@ -144,7 +156,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
       const int g = tl.sub + kSubs * j;
-      se[j] = g < G ? s_val[tl.q * kBoxRow + g] * a.softmax_scale : -INFINITY;
+      se[j] = g < G ? s_val[tl.q * kBoxRow + g] * scale : -INFINITY;
     }
     __syncthreads();  // the weights take the table
   }
@@ -154,7 +166,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < kSlots; ++i) {
-    sc[i] = has_tap(i) ? sc[i] * a.softmax_scale : -INFINITY;
+    sc[i] = has_tap(i) ? sc[i] * scale : -INFINITY;
     mx = fmaxf(mx, sc[i]);
   }
   if constexpr (XK) {
@@ -215,7 +227,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
     constexpr int C = sizeof(E) == 2 ? box_groups<HD, decltype(taps)::value, XK>() : NC;
     if constexpr (SAFE) {
       fill();
-      box_weighted_safe<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, acc);
+      box_weighted_safe<HD, S, E, RG, FT>(tl, r, off, n, hd, s_tab, a.fix_a_inv, acc);
     } else {
       auto pass = [&](auto first) __attribute__((always_inline)) {
         constexpr int C0 = decltype(first)::value, C1 = C0 + C < NC ? C0 + C : NC;
@@ -279,7 +291,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
       s_val[(tl.wave * kTQ + 4 * (tl.lane >> 4) + r) * HD +
             box_channel<HD, E>(t, tl.lane & 15)] = acc[t][r];
   __syncthreads();
-  bool bad = false;
+  bool bad = RG && tl.q_ok && !(den == den);
 #pragma unroll
   for (int e0 = 0; e0 < kTQ * HD; e0 += kThreads) {
     const int e = e0 + static_cast<int>(tid);
@@ -290,7 +302,7 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
     const int m = e / HD, ch = e - m * HD;
     const int64_t n = tile_row(a, tl, m);
     if (n >= 0 && (!RG || ch < hd))
-      out[n * D + tl.head * hd + ch] = from_f32<S>(o * a.fix_a_inv * s_qnan[m]);
+      out[n * D + tl.head * hd + ch] = from_f32<S>(SAFE ? o * s_qnan[m] : o * a.fix_a_inv * s_qnan[m]);
   }
   return bad;
 }
@@ -299,7 +311,9 @@ __device__ __forceinline__ bool fwd_tile(const Args& a, S* __restrict__ out,
 // which the products spread: to queries of the tile that do not sample the row
 // and (bf16) over its channels.  The tile is then done again with the sum by
 // plain arithmetic over what each query samples (from the start, so that nothing
-// is kept live for it).  Whole-head fp32 products (32, 64, 96, 128) go without.
+// is kept live for it).  Padded head sizes, which the general kernels took before, do so
+// for scores that are not finite too, and gather them as these do.  Whole-head fp32
+// products (32, 64, 96, 128) go without.
 template <int HD, typename S, typename E, int EPL, bool RG, bool DROP>
 __global__ __launch_bounds__(kThreads, (fwd_min_waves<HD, E>())) void dsa3d_fwd_box_kernel(
     Args a, S* __restrict__ out, float* __restrict__ lse, int hd) {

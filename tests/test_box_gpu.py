@@ -254,3 +254,46 @@ def test_other_head_sizes_as_precise_as_direct(hd, G):
     padded, direct = errors(), errors(algo="direct")
     print(f"[precision] {hd} {G} {padded} {direct}", flush=True)
     assert all(p <= 1.1 * d for p, d in zip(padded, direct))
+
+
+@pytest.mark.parametrize("what", ["k", "lowest k", "v and k", "huge v", "offsets"])
+@pytest.mark.parametrize("hd,dt", [(40, torch.float32), (80, torch.bfloat16),
+                                   (104, torch.float32), (24, torch.bfloat16)])
+@pytest.mark.parametrize("std", [0.5, 6.0])  # boxes of one piece, of several
+def test_other_head_sizes_sample_non_finite_values(what, hd, dt, std):
+    """Padded head sizes where inputs are infinite or at the type's limit: the outputs that are
+    finite in the oracle are so here, and equal (products in fp32, bf16 results of 2^-9).  An
+    infinite score of one sign leaves a query its other taps."""
+    from megaslide_amd import dsa3d_core
+    from oracle.dsa3d_ref import dsa3d_core_ref
+
+    case = (6, 9, 13, 2, (3, 7, 7), std)
+    shape = case[:3]
+    q, k, v, off = (t.cpu() for t in _inputs(case, hd, dt))
+    g = torch.Generator().manual_seed(12)
+    if "k" in what:
+        worst = torch.finfo(dt).min if "lowest" in what else float("-inf")
+        k[0, 300, 3] = worst
+        k[0, 411, hd + 2] = -worst
+    if what == "v and k":
+        v[0, 305, 1] = float("nan")
+        v[0, 400, hd + 1] = float("inf")
+    if what == "huge v":
+        v *= 1e30
+    if what == "offsets":
+        at = torch.randint(off.numel(), (200,), generator=g)
+        off.view(-1)[at] = float("inf")
+        off.view(-1)[at[:100]] = float("-inf")
+    ref = dsa3d_core_ref(*(t.float() for t in (q, k, v, off)), shape, 2, case[4], 1.0).double()
+    with torch.no_grad():
+        out = dsa3d_core(*(t.cuda() for t in (q, k, v, off)), shape, 2).double().cpu()
+    fin = torch.isfinite(ref)
+    print(f"[non-finite, padded] {what} {hd} {dt} {std}: {(~fin).sum()} "
+          f"{(torch.isfinite(out) != fin).sum()}", flush=True)
+    if what == "lowest k":  # a score that overflows before its scaling may stay finite here
+        assert torch.isfinite(out)[fin].all()
+    else:
+        assert torch.equal(torch.isfinite(out), fin)
+    assert fin.sum() > 0.3 * fin.numel()
+    tol = 1e-4 if dt == torch.float32 else 1e-2
+    assert (out - ref)[fin].abs().max() <= tol * ref[fin].abs().max()
