@@ -175,8 +175,8 @@ int dsa3d_bwd_impl(const msd_dsa3d_desc* desc, const void* q, const void* k, con
   // holds them
   if (msd::dsa3d_ragged_supported(*desc, q, k, v) &&
       workspace_bytes >= msd::dsa3d_ragged_bwd_ws_bytes(*desc))
-    return launch_status(msd::launch_dsa3d_bwd_ragged(*desc, q, k, v, offsets, ek, ev, dout, lse,
-                                                      dlse, dq, dk, dv, doffsets, dek, dev,
+    return launch_status(msd::launch_dsa3d_bwd_ragged(*desc, q, k, v, offsets, ek, ev, out, dout,
+                                                      lse, dlse, dq, dk, dv, doffsets, dek, dev,
                                                       workspace, s),
                          "dsa3d_bwd");
   return launch_status(msd::launch_dsa3d_bwd_direct(*desc, q, k, v, offsets, ek, ev, out, dout,

@@ -100,6 +100,12 @@ inline unsigned fill_blocks(int64_t n) {
 // Internal launchers (defined in dsa3d.hip / dwconv3d.hip), called by abi.cpp
 // after argument validation.  They return a hipError_t.
 namespace msd {
+// What the tiled backward is told of a call for a padded head size: the first of the
+// call's heads (dropout counts from it), and where it notes gradients that are not finite.
+struct PaddedBwd {
+  int head0;
+  int* flag;
+};
 hipError_t launch_dsa3d_fwd_direct(const msd_dsa3d_desc& d, const void* q, const void* k,
                                    const void* v, const void* off, const void* ek, const void* ev,
                                    void* out, float* lse, hipStream_t s);
@@ -107,7 +113,8 @@ hipError_t launch_dsa3d_bwd_direct(const msd_dsa3d_desc& d, const void* q, const
                                    const void* v, const void* off, const void* ek, const void* ev,
                                    const void* out, const void* dout, const float* lse,
                                    const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                   void* dek, void* dev, void* ws, hipStream_t s);
+                                   void* dek, void* dev, void* ws, hipStream_t s,
+                                   const int* flag = nullptr);
 bool dsa3d_tiled_supported(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v);
 hipError_t launch_dsa3d_fwd_tiled(const msd_dsa3d_desc& d, const void* q, const void* k,
                                   const void* v, const void* off, const void* ek, const void* ev,
@@ -116,15 +123,16 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* v, const void* off, const void* ek, const void* ev,
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                  void* dek, void* dev, void* ws, hipStream_t s, bool padded = false);
+                                  void* dek, void* dev, void* ws, hipStream_t s,
+                                  const PaddedBwd* padded = nullptr);
 bool dsa3d_ragged_supported(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v);
 hipError_t launch_dsa3d_fwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,
                                    const void* v, const void* off, const void* ek, const void* ev,
                                    void* out, float* lse, hipStream_t s);
 hipError_t launch_dsa3d_bwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,
                                    const void* v, const void* off, const void* ek, const void* ev,
-                                   const void* dout, const float* lse, const float* dlse, void* dq,
-                                   void* dk, void* dv, void* doff, void* dek, void* dev, void* ws,
+                                   const void* out, const void* dout, const float* lse,
+                                   const float* dlse, void* dq, void* dk, void* dv, void* doff, void* dek, void* dev, void* ws,
                                    hipStream_t s);
 size_t dsa3d_ragged_bwd_ws_bytes(const msd_dsa3d_desc& d);
 size_t dsa3d_bwd_ws_bytes(const msd_dsa3d_desc& d);

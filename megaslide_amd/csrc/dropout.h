@@ -28,6 +28,7 @@ struct DropoutArgs {
   uint32_t threshold;  // 0 = dropout off
   float scale;         // 1 / (1 - p)
   uint32_t key0, key1, offset;
+  int head0 = 0;       // head of a call's head 0 (a call over some of the heads)
 };
 
 // First output word of Philox4x32-10 for counter (c0, c1, c2, c3), key (k0, k1).
@@ -57,7 +58,7 @@ MSD_HD inline float dropout_factor(const DropoutArgs& d, int64_t row, int head, 
   const uint64_t r = static_cast<uint64_t>(row);
   const uint32_t u = philox4x32_10_first(static_cast<uint32_t>(tap), static_cast<uint32_t>(r),
                                          static_cast<uint32_t>((r >> 32) << 16) |
-                                             static_cast<uint32_t>(head),
+                                             static_cast<uint32_t>(head + d.head0),
                                          d.offset, d.key0, d.key1);
   return u >= d.threshold ? d.scale : 0.0f;
 }

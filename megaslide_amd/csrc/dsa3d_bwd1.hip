@@ -66,7 +66,8 @@ __device__ __forceinline__ TapGrad box_gather_grad(const float* table, const Box
 // AE: bytes of one dK / dV accumulator element (4 = fp32 rows, 2 = scaled fp16).
 // REC: also write the tap records, tile header and transposed q / dO of the
 // column-streaming kernel (bf16 storage).  SPLIT: the scores' sums in short chains
-// (padded head sizes, box_scores_split).
+// (padded head sizes, box_scores_split), and
+// rc.collist set where a tap's gradient is not finite.
 template <int HD, typename E, int AE, bool REC, bool DROP, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
     Args a, const E* __restrict__ dout, const float* __restrict__ lse,
@@ -189,6 +190,10 @@ __global__ __launch_bounds__(kThreads, 4) void dsa3d_bwd_p1_kernel(
     td[i].v = has_tap(i) ? ts[i].v * (f * td[i].v - delta) * a.softmax_scale : 0.0f;
     ts[i].v *= f;
     l1 += fabsf(td[i].v);
+  }
+  if constexpr (SPLIT) {  // l1 is a sum of absolute values: none cancels
+    if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(l1)) != 0 && (threadIdx.x & 63) == 0)
+      atomicOr(rc.collist, 1);
   }
   // bf16 storage: normalised ds lie in [-1, 1], where fp16 keeps 11 bits
   float rl1 = 1.0f;

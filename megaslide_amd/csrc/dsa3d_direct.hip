@@ -26,6 +26,8 @@
 // into an fp32 accumulator); d u = sum_c dw_c/du (ds scale q.K_c + p dO.V_c),
 // zeroed where u <= 0 or u >= S-1 (border clamp), times S/2 (unnormalise),
 // divided by the slot's divisor and times offset_scale.
+#include <algorithm>
+
 #include "common.h"
 #include "dsa3d_coords.h"
 
@@ -172,7 +174,8 @@ __global__ __launch_bounds__(kBlock) void dsa3d_bwd_direct_kernel(
     CoreArgs a, const T* __restrict__ out, const T* __restrict__ dout, const float* __restrict__ lse,
     const float* __restrict__ dlse, T* __restrict__ dq, float* __restrict__ dk_acc,
     float* __restrict__ dv_acc, T* __restrict__ doff, float* __restrict__ dek_acc,
-    float* __restrict__ dev_acc) {
+    float* __restrict__ dev_acc, const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
   (void)out;  // Delta comes from the taps, not from the stored output
   const int lane = threadIdx.x % kGroup;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * kGroupsPerBlock + threadIdx.x / kGroup;
@@ -391,16 +394,34 @@ __global__ __launch_bounds__(kBlock) void dsa3d_bwd_direct_kernel(
     if (lane * CPL + j < a.hd) st(dq, bn * a.qs + cbase + j, dqv[j]);
 }
 
-// Accumulator [rows, D] fp32 -> dst with token stride `stride`, element type T.
+// Accumulators [rows, D] fp32, two of them in a row (blockIdx.y) -> dst0 and dst1 with
+// token strides, element type T.  Grid-stride.  With `flag`, only when *flag != 0.
 template <typename T>
-__global__ __launch_bounds__(256) void strided_convert_kernel(const float* __restrict__ src,
-                                                              T* __restrict__ dst, int64_t rows,
-                                                              int D, int64_t stride) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= rows * D) return;
-  const int64_t r = i / D;
-  const int c = static_cast<int>(i - r * D);
-  st(dst, r * stride + c, src[i]);
+__global__ __launch_bounds__(256) void strided_convert_kernel(const float* __restrict__ acc,
+                                                              T* __restrict__ dst0,
+                                                              T* __restrict__ dst1, int64_t rows,
+                                                              int D, int64_t stride0,
+                                                              int64_t stride1,
+                                                              const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
+  const int64_t n = rows * D;
+  const float* const src = acc + blockIdx.y * n;
+  T* const dst = blockIdx.y == 0 ? dst0 : dst1;
+  const int64_t stride = blockIdx.y == 0 ? stride0 : stride1;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t r = i / D;
+    const int c = static_cast<int>(i - r * D);
+    st(dst, r * stride + c, src[i]);
+  }
+}
+
+// fill_zero_f32, only when *flag != 0 (or without a flag).
+__global__ void zero_acc_kernel(float* __restrict__ p, int64_t n, const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    p[i] = 0.0f;
 }
 
 CoreArgs make_args(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,
@@ -467,7 +488,7 @@ hipError_t fwd_typed(const msd_dsa3d_desc& d, const CoreArgs& a, void* out, floa
 template <typename T>
 hipError_t bwd_typed(const msd_dsa3d_desc& d, const CoreArgs& a, const void* out, const void* dout,
                      const float* lse, const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                     void* dek, void* dev, void* ws, hipStream_t s) {
+                     void* dek, void* dev, void* ws, hipStream_t s, const int* flag) {
   const int64_t rows = static_cast<int64_t>(a.B) * a.N;
   const int D = a.nh * a.hd;
   const int64_t erows = static_cast<int64_t>(a.B) * a.G;
@@ -476,7 +497,9 @@ hipError_t bwd_typed(const msd_dsa3d_desc& d, const CoreArgs& a, const void* out
   float* dek_acc = dv_acc + rows * D;
   float* dev_acc = dek_acc + erows * D;
   const int64_t nacc = 2 * (rows + erows) * D;
-  hipLaunchKernelGGL(fill_zero_f32, dim3(fill_blocks(nacc)), dim3(256), 0, s, dk_acc, nacc);
+  // (small grids where there is most likely nothing to do)
+  auto blocks = [&](int64_t n) { return flag != nullptr ? std::min(fill_blocks(n), 1024u) : fill_blocks(n); };
+  hipLaunchKernelGGL(zero_acc_kernel, dim3(blocks(nacc)), dim3(256), 0, s, dk_acc, nacc, flag);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t groups = rows * a.nh;
@@ -485,22 +508,16 @@ hipError_t bwd_typed(const msd_dsa3d_desc& d, const CoreArgs& a, const void* out
     hipLaunchKernelGGL((dsa3d_bwd_direct_kernel<T, CPL>), grid, dim3(kBlock), 0, s, a,
                        static_cast<const T*>(out), static_cast<const T*>(dout), lse, dlse,
                        static_cast<T*>(dq), dk_acc, dv_acc, static_cast<T*>(doff), dek_acc,
-                       dev_acc);
+                       dev_acc, flag);
     return hipGetLastError();
   });
   if (e != hipSuccess) return e;
-  const dim3 cgrid(static_cast<unsigned>((rows * D + 255) / 256));
-  hipLaunchKernelGGL((strided_convert_kernel<T>), cgrid, dim3(256), 0, s, dk_acc,
-                     static_cast<T*>(dk), rows, D, a.ks);
-  hipLaunchKernelGGL((strided_convert_kernel<T>), cgrid, dim3(256), 0, s, dv_acc,
-                     static_cast<T*>(dv), rows, D, a.vs);
-  if (erows > 0) {
-    const dim3 egrid(static_cast<unsigned>((erows * D + 255) / 256));
-    hipLaunchKernelGGL((strided_convert_kernel<T>), egrid, dim3(256), 0, s, dek_acc,
-                       static_cast<T*>(dek), erows, D, static_cast<int64_t>(D));
-    hipLaunchKernelGGL((strided_convert_kernel<T>), egrid, dim3(256), 0, s, dev_acc,
-                       static_cast<T*>(dev), erows, D, static_cast<int64_t>(D));
-  }
+  hipLaunchKernelGGL((strided_convert_kernel<T>), dim3(blocks(rows * D), 2), dim3(256), 0, s, dk_acc,
+                     static_cast<T*>(dk), static_cast<T*>(dv), rows, D, a.ks, a.vs, flag);
+  if (erows > 0)
+    hipLaunchKernelGGL((strided_convert_kernel<T>), dim3(blocks(erows * D), 2), dim3(256), 0, s,
+                       dek_acc, static_cast<T*>(dek), static_cast<T*>(dev), erows, D,
+                       static_cast<int64_t>(D), static_cast<int64_t>(D), flag);
   return hipGetLastError();
 }
 
@@ -532,11 +549,11 @@ hipError_t launch_dsa3d_bwd_direct(const msd_dsa3d_desc& d, const void* q, const
                                    const void* v, const void* off, const void* ek, const void* ev,
                                    const void* out, const void* dout, const float* lse,
                                    const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                   void* dek, void* dev, void* ws, hipStream_t s) {
+                                   void* dek, void* dev, void* ws, hipStream_t s, const int* flag) {
   const CoreArgs a = make_args(d, q, k, v, off, ek, ev);
   if (d.dtype == MSD_BF16)
-    return bwd_typed<bf16>(d, a, out, dout, lse, dlse, dq, dk, dv, doff, dek, dev, ws, s);
-  return bwd_typed<float>(d, a, out, dout, lse, dlse, dq, dk, dv, doff, dek, dev, ws, s);
+    return bwd_typed<bf16>(d, a, out, dout, lse, dlse, dq, dk, dv, doff, dek, dev, ws, s, flag);
+  return bwd_typed<float>(d, a, out, dout, lse, dlse, dq, dk, dv, doff, dek, dev, ws, s, flag);
 }
 
 }  // namespace msd

@@ -1687,7 +1687,8 @@ struct BwdBufs {
   float* dqx;      // extra keys: their part of dq, fp32 [rows, D] (null without them)
   float* dlt;      // extra keys: Delta per (token, head), fp32 [rows, nh] (null without them)
   RecArgs rec;     // column-streaming kernel's records (rec.rec null: not used)
-  bool split;      // fp32: the first kernel's scores in short chains (padded head sizes)
+  const PaddedBwd* padded;  // padded head sizes (fp32): the first kernel's scores in short
+                            // chains, its gradients tested
 };
 
 template <int HD, typename E>
@@ -1698,6 +1699,7 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
   constexpr int CW = p2_window<HD, E>(), FR = p2_frames<HD, E>();
   tiled::Args a1 = make_tiled_args(d, q, k, v, off, tiled_tiles<1>(d), ek, ev);
   a1.dlt = w.dlt;
+  if (w.padded != nullptr) a1.drop.head0 = w.padded->head0;
   const tiled::Args a2 = make_tiled_args(d, q, k, v, off, tiled_tiles<FR>(d), ek, ev);
   dim3 g2 = tiled_grid<FR>(d);
   g2.z = HD / CW;
@@ -1735,11 +1737,14 @@ void launch_bwd_pair(const msd_dsa3d_desc& d, const void* q, const void* k, cons
                                      acc_vs, RecArgs{}, s);
   }
   if constexpr (sizeof(E) == 4) {
-    if (w.split)
+    if (w.padded != nullptr) {
+      RecArgs rc{};
+      rc.collist = w.padded->flag;
       launch_bwd_p1<HD, E, 4, false, true>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc,
-                                           acc_ks, acc_vs, RecArgs{}, s);
+                                           acc_ks, acc_vs, rc, s);
+    }
   }
-  if (!h16 && !w.split)
+  if (!h16 && w.padded == nullptr)
     launch_bwd_p1<HD, E, 4, false>(a1, go, lse, dlse, goff, p_ws, b_ws, dk_acc, dv_acc, acc_ks,
                                    acc_vs, RecArgs{}, s);
   if (d.extra_g > 0)
@@ -1910,7 +1915,7 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
                            const void* off, const void* ek, const void* ev, const void* out,
                            const void* dout, const float* lse, const float* dlse, void* dq,
                            void* dk, void* dv, void* doff, void* dek, void* dev, void* ws,
-                           bool padded, hipStream_t s) {
+                           const PaddedBwd* padded, hipStream_t s) {
   const int64_t rows = static_cast<int64_t>(d.B) * d.T * d.H * d.W;
   const int D = d.num_heads * d.head_dim;
   const int64_t erows = static_cast<int64_t>(d.B) * d.extra_g;
@@ -1944,7 +1949,7 @@ hipError_t bwd_tiled_typed(const msd_dsa3d_desc& d, const void* q, const void* k
   w.dqx = erows > 0 ? reinterpret_cast<float*>(base + L.dqx) : nullptr;
   w.dlt = erows > 0 ? reinterpret_cast<float*>(base + L.dlt) : nullptr;
   w.rec = RecArgs{};
-  w.split = padded;
+  w.padded = padded;
   if (tiled_streams(d) && enough_columns(d)) {
     w.rec.rec = reinterpret_cast<tiled::u32x4_t*>(base + L.rec);
     w.rec.hdr = reinterpret_cast<int*>(base + L.hdr);
@@ -2012,13 +2017,14 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const void* v, const void* off, const void* ek, const void* ev,
                                   const void* out, const void* dout, const float* lse,
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
-                                  void* dek, void* dev, void* ws, hipStream_t s, bool padded) {
+                                  void* dek, void* dev, void* ws, hipStream_t s,
+                                  const PaddedBwd* padded) {
   if (!tiled::rows_below_limit(d))
     return launch_dsa3d_bwd_direct(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
                                    dek, dev, ws, s);
   if (d.dtype == MSD_BF16)
     return bwd_tiled_typed<bf16>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
-                                 dek, dev, ws, false, s);
+                                 dek, dev, ws, nullptr, s);
   return bwd_tiled_typed<float>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
                                 dek, dev, ws, padded, s);
 }

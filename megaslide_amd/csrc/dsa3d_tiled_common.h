@@ -194,7 +194,7 @@ struct RecArgs {
   int* hdr;        // [nh][tiles][kRecHdr]
   void* qt;        // [nh][tiles][2][HD][16] element type
   int* collist;    // [0]: count, then head * columns + column of each column
-                   // left to the tile kernel
+                   // left to the tile kernel (padded head sizes: see dsa3d_bwd_p1_kernel)
   int64_t tiles;   // one-frame tiles per head
 };
 
