@@ -183,3 +183,21 @@ def test_noalloc_scratch_limit_and_rejection():
     rc = lib.msd_dsa3d_bwd_noalloc(ctypes.byref(big), *([16] * 4), None, None, *([16] * 3), None,
                                    *([16] * 4), None, None, None)
     assert rc == -4 and b"maximum" in lib.msd_last_error()
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("hd,nh,shape", [(80, 16, (64, 32, 32)), (40, 24, (13, 45, 80)),
+                                         (120, 24, (32, 64, 64)), (24, 64, (16, 64, 64))])
+def test_padded_backward_workspace_is_bounded(hd, nh, shape, dtype):
+    """Head sizes between the compiled ones: the workspace for the padded copies stays within
+    1 GiB, what the general kernels need, or what one head takes (seven rows of the padded
+    channels, the offsets and their gradients, two words a tap, in fp32)."""
+    lib = _lib.load()
+    T, H, W = shape
+    N, taps = T * H * W, 147
+    d = _desc(T=T, H=H, W=W, num_heads=nh, head_dim=hd, dtype=dtype, q_stride=nh * hd,
+              k_stride=nh * hd, v_stride=nh * hd)
+    need = lib.msd_dsa3d_bwd_workspace_size(ctypes.byref(d))
+    best = lib.msd_dsa3d_bwd_best_workspace_size(ctypes.byref(d))
+    head = N * 4 * (7 * ((hd + 31) // 32 * 32) + 8 * taps + 2)
+    assert need <= best <= max(1 << 30, need, head + (1 << 20)) + 4096

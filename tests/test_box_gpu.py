@@ -354,3 +354,20 @@ def test_other_head_sizes_differentiate_non_finite_values_as_direct(what, hd, dt
             tol = 2e-5 if dt == torch.float32 else 2.0 ** -8
             assert (x - y)[fin].abs().max() <= tol * y[fin].abs().max(), f"gradient {i}"
     assert some > 0.5 * sum(t.numel() for t in ins)
+
+
+@pytest.mark.parametrize("dt,p,G", [(torch.float32, 0.2, 7), (torch.bfloat16, 0.0, 0)])
+def test_padded_backward_over_groups_of_heads(dt, p, G):
+    """More heads than the padded copies' workspace takes at once: the groups' gradients against
+    the direct kernels' (tolerances as above; dropout's counters run over all heads)."""
+    print(f"[groups of heads] {dt} {p} {G}", flush=True)
+    case = (16, 24, 26, 19, (3, 7, 7), 0.5)
+    ins = _inputs(case, 40, dt)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    extra = [torch.randn(1, G, 19 * 40, generator=g, device="cuda").to(dt) for _ in range(2 * (G > 0))]
+    kw = dict(dropout_p=p, dropout_seed=11)
+    a = _grads(ins, extra, case[:3], 19, case[4], **kw)
+    b = _grads(ins, extra, case[:3], 19, case[4], algo="direct", **kw)
+    for x, y in zip(a, b):
+        tol = 3e-5 if dt == torch.float32 else 2.0 ** -8
+        assert (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
