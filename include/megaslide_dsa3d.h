@@ -94,10 +94,12 @@ typedef enum msd_accum { MSD_ACCUM_F32 = 0, MSD_ACCUM_F16 = 1 } msd_accum;
 
 /* Kernel family for the attention core.  AUTO picks the matrix-core tiled
  * kernels when the call qualifies (bf16 or fp32, head_dim 32/64/96/128, <= 160
- * taps, token strides multiples of 8 elements, 16-byte aligned rows; also other
- * head_dim that are multiples of 8 up to 120, in the backward given the workspace
- * of msd_dsa3d_bwd_best_workspace_size) and the direct kernels otherwise.  DIRECT and TILED force one family (TILED fails
- * with MSD_ERR_UNSUPPORTED if not eligible). */
+ * taps, <= 256 extra keys, token strides multiples of 8 elements, 16-byte aligned
+ * rows, K and V samples of less than 2^30 elements and, in fp32, 4 GiB less 2 KiB),
+ * their padded form for other head_dim that are multiples of 8 up to 120 (in the
+ * backward given the workspace of msd_dsa3d_bwd_best_workspace_size), and the
+ * direct kernels otherwise.  DIRECT and TILED force one family (TILED, without the
+ * padded form, fails with MSD_ERR_UNSUPPORTED if not eligible). */
 typedef enum msd_algo { MSD_ALGO_AUTO = 0, MSD_ALGO_DIRECT = 1, MSD_ALGO_TILED = 2 } msd_algo;
 
 /* Shape and options of one depthwise-conv call. */
@@ -142,8 +144,9 @@ size_t msd_dsa3d_bwd_workspace_size(const msd_dsa3d_desc* desc);
  * Bytes with which msd_dsa3d_bwd is fastest for `desc`, at least what it needs.
  * More than that for MSD_ALGO_AUTO calls whose head_dim is a multiple of 8 up to
  * 120 but not of 32: with that much workspace they take the matrix-core kernels
- * on padded fp32 copies, else the direct kernels (e.g. 4,096 tokens, 16 x 80,
- * window 3x5x5, bf16: 3 ms against 113).
+ * on padded fp32 copies, else the direct kernels (4,096 tokens, 16 x 80, window
+ * 3x5x5, bf16, forward and backward: 1.7 ms against 116).  At most 1 GiB, what the
+ * direct kernels need, or what the copies of one head take, whichever is largest.
  */
 size_t msd_dsa3d_bwd_best_workspace_size(const msd_dsa3d_desc* desc);
 

@@ -165,7 +165,7 @@ int dsa3d_bwd_impl(const msd_dsa3d_desc* desc, const void* q, const void* k, con
   if (desc->algo == MSD_ALGO_TILED && !tiled_ok)
     return fail(MSD_ERR_UNSUPPORTED,
                 "dsa3d_bwd: tiled kernels need bf16 or fp32, head_dim 32, 64, 96 or 128, <= 160 taps, "
-                "<= 256 extra keys and 16-byte aligned rows");
+                "<= 256 extra keys, 16-byte aligned rows and samples that 32-bit row offsets address");
   if (tiled_ok && desc->algo != MSD_ALGO_DIRECT)
     return launch_status(msd::launch_dsa3d_bwd_tiled(*desc, q, k, v, offsets, ek, ev, out, dout,
                                                      lse, dlse, dq, dk, dv, doffsets, dek, dev,
@@ -209,7 +209,7 @@ int msd_dsa3d_fwd(const msd_dsa3d_desc* desc, const void* q, const void* k, cons
   if (desc->algo == MSD_ALGO_TILED && !tiled_ok)
     return fail(MSD_ERR_UNSUPPORTED,
                 "dsa3d_fwd: tiled kernels need bf16 or fp32, head_dim 32, 64, 96 or 128, <= 160 taps, "
-                "<= 256 extra keys and 16-byte aligned rows");
+                "<= 256 extra keys, 16-byte aligned rows and samples that 32-bit row offsets address");
   if (desc->B == 0) return MSD_OK;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (tiled_ok && desc->algo != MSD_ALGO_DIRECT)

@@ -6,8 +6,6 @@ namespace msd {
 hipError_t launch_dsa3d_fwd_tiled(const msd_dsa3d_desc& d, const void* q, const void* k,
                                   const void* v, const void* off, const void* ek, const void* ev,
                                   void* out, float* lse, hipStream_t s) {
-  if (!rows_below_limit(d))
-    return launch_dsa3d_fwd_direct(d, q, k, v, off, ek, ev, out, lse, s);
   const Args a = make_tiled_args(d, q, k, v, off, tile_count<1>(d.B, d.T, d.H, d.W), ek, ev);
   if (d.dtype == MSD_BF16) return fwd_typed<bf16, bf16, false>(d, a, out, lse, s);
   return fwd_typed<float, float, false>(d, a, out, lse, s);

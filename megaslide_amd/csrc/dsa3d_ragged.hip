@@ -293,13 +293,11 @@ bool dsa3d_ragged_supported(const msd_dsa3d_desc& d, const void* q, const void* 
   if ((d.q_stride % 8) || (d.k_stride % 8) || (d.v_stride % 8)) return false;
   for (const void* p : {q, k, v})
     if (reinterpret_cast<uintptr_t>(p) % 16) return false;
-  // the forward addresses a sample's rows with 32-bit byte offsets, and packs a
-  // tap's piece of a cut box into 17 bits (a sample of less than 2^25 voxels)
-  const msd_dsa3d_desc p = padded_desc(d, d.num_heads);
-  if (static_cast<int64_t>(d.T) * d.H * d.W >= int64_t{1} << 25 || !rows_below_limit(d) ||
-      !rows_below_limit(p))
+  // the forward addresses the sample's own rows with 32-bit byte offsets, and its taps'
+  // words hold a sample of less than 2^25 voxels
+  if (static_cast<int64_t>(d.T) * d.H * d.W >= int64_t{1} << 25 || !rows_below_limit(d))
     return false;
-  return dsa3d_tiled_supported(p, nullptr, nullptr, nullptr);
+  return dsa3d_tiled_supported(padded_desc(d, d.num_heads), nullptr, nullptr, nullptr);
 }
 
 hipError_t launch_dsa3d_fwd_ragged(const msd_dsa3d_desc& d, const void* q, const void* k,

@@ -1466,6 +1466,8 @@ bool dsa3d_tiled_supported(const msd_dsa3d_desc& d, const void* q, const void* k
   // below 2^30, so bytes below 2^32 even for fp32)
   const int64_t n = static_cast<int64_t>(d.T) * d.H * d.W;
   if (n * d.k_stride >= (int64_t{1} << 30) || n * d.v_stride >= (int64_t{1} << 30)) return false;
+  // and K/V rows behind 32-bit buffer offsets, below the one that stands for no row
+  if (!tiled::rows_below_limit(d)) return false;
   // K/V chunk rows are addressed as a 64-bit chunk base plus a 32-bit lane byte
   // offset (24-bit multiplies): kChunk * (W + 1) rows must span < 2^31 bytes
   for (const int64_t st : {d.k_stride, d.v_stride})
@@ -2019,9 +2021,6 @@ hipError_t launch_dsa3d_bwd_tiled(const msd_dsa3d_desc& d, const void* q, const 
                                   const float* dlse, void* dq, void* dk, void* dv, void* doff,
                                   void* dek, void* dev, void* ws, hipStream_t s,
                                   const PaddedBwd* padded) {
-  if (!tiled::rows_below_limit(d))
-    return launch_dsa3d_bwd_direct(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
-                                   dek, dev, ws, s);
   if (d.dtype == MSD_BF16)
     return bwd_tiled_typed<bf16>(d, q, k, v, off, ek, ev, out, dout, lse, dlse, dq, dk, dv, doff,
                                  dek, dev, ws, nullptr, s);

@@ -45,7 +45,7 @@ constexpr int kSRow = kChunkNV + 4;
 // Byte offset that stands for a row outside the volume or the box (dsa3d_box.h):
 // past the end of a sample's rows, and no lane or immediate offset added to it
 // wraps.  Samples that reach it (or extra keys whose signed offsets overflow)
-// take the direct kernels.
+// are not for the tiled kernels.
 constexpr uint32_t kNoRow = 0xfffff800u;
 inline bool rows_below_limit(const msd_dsa3d_desc& d) {
   const int64_t st = d.k_stride > d.v_stride ? d.k_stride : d.v_stride;

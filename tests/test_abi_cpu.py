@@ -201,3 +201,16 @@ def test_padded_backward_workspace_is_bounded(hd, nh, shape, dtype):
     best = lib.msd_dsa3d_bwd_best_workspace_size(ctypes.byref(d))
     head = N * 4 * (7 * ((hd + 31) // 32 * 32) + 8 * taps + 2)
     assert need <= best <= max(1 << 30, need, head + (1 << 20)) + 4096
+
+
+def test_tiled_refuses_samples_beyond_its_row_offsets():
+    """fp32 K/V samples in the last 2 KiB below 4 GiB: their rows reach the byte offset that
+    stands for no row, so MSD_ALGO_TILED refuses them (and AUTO takes the direct kernels)."""
+    lib = _lib.load()
+    shape = dict(T=49, H=127, W=337, num_heads=8, head_dim=64)  # 2^21 - 1 tokens of 512
+    d = _desc(**shape, q_stride=512, k_stride=512, v_stride=512, algo=2)
+    assert _fwd(d) == -2 and b"row offsets" in lib.msd_last_error()
+    big = ctypes.c_size_t(1 << 60)
+    rc = lib.msd_dsa3d_bwd(ctypes.byref(d), *(16,) * 4, None, None, 16, 16, 16, None, *(16,) * 4,
+                           None, None, 16, big, None)
+    assert rc == -2 and b"row offsets" in lib.msd_last_error()
