@@ -77,8 +77,8 @@ __device__ __forceinline__ void box_cut(int na, int nm, int nn, int& ca, int& cm
 // Geometry of this lane's taps: corner weights, and the word index of the
 // first corner in the query's table row (row offset included), or, where there
 // are several pieces, (column * len + layer) * (cm cn) + index within the
-// column's layer.  (A sample has less than 2^25 voxels, its box with the layers
-// past its faces and the columns' shared voxels less than 2^31.)
+// column's layer.  (A sample has less than 2^25 voxels, a box at W = 1 twice its
+// voxels of the sample, and columns share at most 37 % more: less than 2^27.)
 template <int SLOTS>
 struct BoxTaps {
   float fx[SLOTS], fy[SLOTS], fz[SLOTS];

@@ -9,7 +9,7 @@
 // with l1 = sum over the query's taps of |ds * scale| per token and head).
 //
 // Bound: like the forward, the latency of the K and V rows' loads and VALU issue;
-// then the per-tap results (22 bytes a tap in bf16 with records).  Against tables
+// then the per-tap results (26 bytes a tap in bf16 with records).  Against tables
 // of one plane at a time, two of them (S and dP) double-buffered: 4.37 -> 3.99 ms
 // at 65,536 tokens, 16 x 64, bf16; 6.84 -> 6.46 ms at 46,800 tokens, 16 x 96,
 // offsets biased by up to 4 voxels; 16.3 -> 15.9 ms at 131,072 tokens, 24 x 128;

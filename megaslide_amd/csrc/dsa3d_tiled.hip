@@ -297,8 +297,8 @@ __device__ __forceinline__ void p2_tile(const Args& a, int tile, const E* __rest
       // outstanding atomic)
       Slot si = sl[i];
       asm volatile("" : "+v"(si.zc), "+v"(si.idx), "+v"(si.fx), "+v"(si.fy));
-      float wz, dwz;
-      if (!slot_hits(si, step_key(c.id, z), wz, dwz)) continue;
+      float wz;
+      if (!slot_hits(si, step_key(c.id, z), wz)) continue;
       const float pz = p[i] * wz, bz = bsc[i] * wz;
       const float fx = si.fx, fy = si.fy, gx = 1.0f - fx, gy = 1.0f - fy;
       const float w00 = gy * gx, w01 = gy * fx, w10 = fy * gx, w11 = fy * fx;

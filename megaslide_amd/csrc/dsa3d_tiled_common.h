@@ -162,8 +162,8 @@ struct Args {
                                  //   their part, then (first backward kernel) the whole
 };
 
-// Kernel arguments for a launch over `tiles` workgroups per head (dsa3d_tiled.hip).
 }  // namespace tiled
+// Kernel arguments for a launch over `tiles` workgroups per head (dsa3d_tiled.hip).
 tiled::Args make_tiled_args(const msd_dsa3d_desc& d, const void* q, const void* k, const void* v,
                             const void* off, int64_t tiles, const void* ek, const void* ev);
 // CUs of the current device (dsa3d_tiled.hip).
@@ -618,11 +618,10 @@ __device__ __forceinline__ uint32_t slot_key(const Slot& s) {
 }
 
 // Does this slot have corners on the step's plane?  Returns the z weight.
-__device__ __forceinline__ bool slot_hits(const Slot& s, uint32_t key, float& wz, float& dwz) {
+__device__ __forceinline__ bool slot_hits(const Slot& s, uint32_t key, float& wz) {
   const uint32_t d = key - slot_key(s);
   if (d > static_cast<uint32_t>(slot_hz(s))) return false;
   wz = d == 0 ? 1.0f - s.fz : s.fz;
-  dwz = d == 0 ? -1.0f : 1.0f;
   return true;
 }
 

@@ -371,3 +371,84 @@ def test_padded_backward_over_groups_of_heads(dt, p, G):
     for x, y in zip(a, b):
         tol = 3e-5 if dt == torch.float32 else 2.0 ** -8
         assert (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
+
+
+@pytest.mark.parametrize("hd,dt,inf", [
+    *((hd, dt, inf) for inf in (False, True)
+      for hd, dt in ((32, torch.bfloat16), (96, torch.bfloat16), (128, torch.bfloat16),
+                     (72, torch.float32))),
+    # (whole-head fp32 products have no plain-arithmetic pass)
+    (64, torch.float32, False), (128, torch.float32, False)])
+@pytest.mark.parametrize("G,p", [(20, 0.0), (128, 0.3), (200, 0.0), (0, 0.3)])
+def test_cut_boxes_with_extra_keys_and_dropout(G, p, hd, dt, inf):
+    """Boxes of several pieces together with extra keys and dropout, and with an infinite value in
+    a V row (and one in an extra value: its weight reaches every query), which sends tiles to the
+    plain-arithmetic pass: against the direct kernels, tolerances as above."""
+    from megaslide_amd import dsa3d_core
+
+    case = (9, 13, 21, 2, (3, 7, 7), 6.0)
+    q, k, v, off = _inputs(case, hd, dt)
+    g = torch.Generator().manual_seed(4)
+    ek = ev = None
+    if G:
+        ek, ev = (torch.randn(1, G, 2 * hd, generator=g).to(dt).cuda() for _ in range(2))
+    if inf:
+        v[0, 1000, hd - 3] = float("inf")
+        v[0, 1500, hd + 5] = float("-inf")
+        if G:
+            ev[0, G - 1, 2] = float("inf")
+    kw = dict(extra_k=ek, extra_v=ev, dropout_p=p, dropout_seed=5)
+    with torch.no_grad():
+        out = dsa3d_core(q, k, v, off, case[:3], 2, **kw).double()
+        ref = dsa3d_core(q, k, v, off, case[:3], 2, algo="direct", **kw).double()
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(out), fin) and fin.all() == (not inf)
+    tol = 1e-5 if dt == torch.float32 else 2e-2
+    assert (out - ref)[fin].abs().max() <= tol * ref[fin].abs().max()
+
+
+@pytest.mark.parametrize("hd,dt", [(64, torch.bfloat16), (96, torch.float32), (40, torch.bfloat16),
+                                   (72, torch.float32)])
+@pytest.mark.parametrize("std", [0.5, 6.0])
+def test_strides_of_their_own(hd, dt, std):
+    """q, k and v (and their gradients) with three different token strides, through the C entry
+    points, equal the contiguous call bit for bit in the forward and up to the order of fp32
+    atomics (2e-5; bf16 one rounding) in the backward."""
+    import ctypes
+    from megaslide_amd import _lib, dsa3d_core
+
+    lib = _lib.load()
+    case = (7, 9, 14, 3, (3, 5, 5), std)
+    T, H, W, nh, win, _ = case
+    ins = _inputs(case, hd, dt)
+    N, D = T * H * W, nh * hd
+    g = torch.Generator(device="cuda").manual_seed(8)
+    dout = torch.randn(1, N, D, generator=g, device="cuda").to(dt)
+    ts = [t.detach().clone().requires_grad_(True) for t in ins]
+    ref, rlse = dsa3d_core(*ts, case[:3], nh, win, return_lse=True)
+    grads = torch.autograd.grad(ref, ts, dout)
+
+    strides = (D + 8, 2 * D, 3 * D + 16)
+    wide = [torch.full((N, s), 7.0, dtype=dt, device="cuda") for s in strides]
+    outs = [torch.full((N, s), 7.0, dtype=dt, device="cuda") for s in strides]
+    for w, t in zip(wide, ins):
+        w[:, :D] = t[0]
+    desc = _lib.DsaDesc(1, T, H, W, nh, hd, *win, _lib.dtype_code(dt), *strides, 1.0, hd ** -0.5)
+    out, lse = torch.empty_like(ref), torch.empty_like(rlse)
+    stream = _lib.stream_handle(out.device)
+    _lib.check(lib.msd_dsa3d_fwd(ctypes.byref(desc), *(w.data_ptr() for w in wide),
+                                 ins[3].data_ptr(), None, None, out.data_ptr(), lse.data_ptr(),
+                                 stream), "fwd")
+    assert torch.equal(out, ref) and torch.equal(lse, rlse)
+    size = lib.msd_dsa3d_bwd_best_workspace_size(ctypes.byref(desc))
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    doff = torch.empty_like(ins[3])
+    _lib.check(lib.msd_dsa3d_bwd(ctypes.byref(desc), *(w.data_ptr() for w in wide),
+                                 ins[3].data_ptr(), None, None, out.data_ptr(), dout.data_ptr(),
+                                 lse.data_ptr(), None, *(o.data_ptr() for o in outs),
+                                 doff.data_ptr(), None, None, ws.data_ptr(), size, stream), "bwd")
+    tol = 2e-5 if dt == torch.float32 else 2.0 ** -7
+    for o, x in zip([w[:, :D] for w in outs] + [doff[0]], grads):
+        assert (o.float() - x[0].float()).abs().max() <= tol * x.float().abs().max()
+    for o in outs:  # nothing between the rows
+        assert (o[:, D:] == 7.0).all()

@@ -10,9 +10,10 @@ every gradient (dq, dK, dV, d offsets) against the oracle:
   - fp32 storage (fp32 matrix-core kernels), 1e-4;
   - bf16 with G shared extra keys (their gradients checked too), 2e-2;
   - bf16 with attention dropout (the oracle applies the same Philox keep mask), 2e-2;
-  - head sizes and windows the tiled kernels do not take (head_dim 8 to 112 off the
-    32/64/96/128 set, windows of more than 160 taps), which the default dispatch
-    sends to the general (direct) kernels: bf16 2e-2, fp32 1e-4;
+  - head sizes and windows that MSD_ALGO_TILED does not take, through the default dispatch:
+    head_dim 8 to 112 off the 32/64/96/128 set (the tiled kernels' padded form) and windows
+    of more than 160 taps (the general, direct kernels): bf16 2e-2, fp32 1e-4;
+  - the direct kernels at such head sizes: bf16 2e-2, fp32 1e-4;
   - the returned log-sum-exp differentiated with the output (loss = sum(out g_out)
     + sum(lse g_lse), the dlse input of the backward), bf16 and fp32; lse itself
     within 1e-4 (bf16: 2e-3 of max|lse|).
@@ -35,6 +36,7 @@ MODES = {"bf16": (torch.bfloat16, "fp32", BF16_TOL), "bf16-f16acc": (torch.bfloa
          "fp32": (torch.float32, "fp32", FP32_TOL), "bf16-extra": (torch.bfloat16, "fp32", BF16_TOL),
          "bf16-dropout": (torch.bfloat16, "fp32", BF16_TOL),
          "general-bf16": (torch.bfloat16, "fp32", BF16_TOL), "general-fp32": (torch.float32, "fp32", FP32_TOL),
+         "direct-bf16": (torch.bfloat16, "fp32", BF16_TOL), "direct-fp32": (torch.float32, "fp32", FP32_TOL),
          "bf16-lse": (torch.bfloat16, "fp32", BF16_TOL), "fp32-lse": (torch.float32, "fp32", FP32_TOL)}
 WINDOWS = [(1, 1, 1), (1, 3, 3), (3, 3, 3), (3, 5, 5), (3, 7, 7), (1, 7, 7), (3, 1, 3),
            (5, 3, 3), (2, 3, 5), (3, 5, 7)]
@@ -66,15 +68,18 @@ CASES = ([("bf16", s) for s in range(48)] + [("bf16-f16acc", s) for s in range(4
          [("fp32", s) for s in range(64, 80)] + [("bf16-extra", s) for s in range(80, 96)] +
          [("bf16-dropout", s) for s in range(96, 112)] + [("general-bf16", s) for s in range(112, 120)] +
          [("general-fp32", s) for s in range(120, 128)] + [("bf16-lse", s) for s in range(128, 144)] +
-         [("fp32-lse", s) for s in range(144, 152)])
+         [("fp32-lse", s) for s in range(144, 152)] + [("direct-bf16", s) for s in range(152, 158)] +
+         [("direct-fp32", s) for s in range(158, 164)])
 
 
 @pytest.mark.parametrize("mode,seed", CASES)
 def test_tiled_random_shape_vs_oracle(mode, seed):
     dtype, accum, tol = MODES[mode]
     B, T, H, W, nh, ks, hd, off_std, shift, scale = draw(seed)
-    general = mode.startswith("general")
-    if general:
+    general = mode.startswith(("general", "direct"))
+    if mode.startswith("direct"):
+        hd = [8, 16, 40, 48, 80, 112][seed % 6]
+    elif general:
         # a head size off the tiled set, or (every third case) a 5x7x7 window of 245 taps
         hd = [8, 16, 40, 48, 80, 112][seed % 6]
         if seed % 3 == 0:
@@ -113,7 +118,7 @@ def test_tiled_random_shape_vs_oracle(mode, seed):
 
     from megaslide_amd import dsa3d_core
     ts = [t.detach().to(DEV).requires_grad_(True) for t in inputs]
-    kw = dict(algo="auto" if general else "tiled", dkv_accum=accum)
+    kw = dict(algo="direct" if mode.startswith("direct") else "auto" if general else "tiled", dkv_accum=accum)
     if G:
         kw.update(extra_k=ts[4], extra_v=ts[5])
     if drop:
