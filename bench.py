@@ -644,18 +644,18 @@ def phase_kernels(dtype, accum="fp32", extra=0):
     the dq/dK/dV kernel, the conversion, and the fp32 redo after an overflow,
     whose kernels return at once without one)."""
     if dtype != "bf16":
-        return {"dsa3d_fwd": ["dsa3d_fwd_tiled_kernel"],
+        return {"dsa3d_fwd": ["dsa3d_fwd_box_kernel"],
                 "dsa3d_bwd": ["dsa3d_bwd_p1_kernel", "dsa3d_bwd_p2_kernel"]}
     if accum == "fp32" and extra:
-        return {"dsa3d_fwd": ["dsa3d_fwd_tiled_kernel"],
+        return {"dsa3d_fwd": ["dsa3d_fwd_box_kernel"],
                 "dsa3d_bwd": ["dsa3d_bwd_p1_kernel", "dsa3d_bwd_extra_kernel",
                               "dsa3d_bwd_p2_kernel", "extra_grad_kernel",
                               "acc_to_bf16_kernel"]}
     if accum == "fp32":
-        return {"dsa3d_fwd": ["dsa3d_fwd_tiled_kernel"],
+        return {"dsa3d_fwd": ["dsa3d_fwd_box_kernel"],
                 "dsa3d_bwd": ["dsa3d_bwd_p1_kernel", "dsa3d_bwd_p2s_kernel",
                               "dsa3d_bwd_p2_list_kernel", "acc_to_bf16_kernel"]}
-    return {"dsa3d_fwd": ["dsa3d_fwd_tiled_kernel"],
+    return {"dsa3d_fwd": ["dsa3d_fwd_box_kernel"],
             "dsa3d_bwd": ["dsa3d_bwd_p1_kernel", "h16_bounds_kernel", "h16_scales_kernel",
                           "dsa3d_bwd_p2_kernel", "h16_to_bf16_kernel", "fill_zero_if_flag",
                           "dsa3d_bwd_p2_redo_kernel", "acc_to_bf16_kernel"]}
