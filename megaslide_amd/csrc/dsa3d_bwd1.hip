@@ -8,12 +8,13 @@
 // [token][head][tap]; bf16: one word of two fp16, p * factor and ds * scale / l1,
 // with l1 = sum over the query's taps of |ds * scale| per token and head).
 //
-// Bound: like the forward, the latency of the K and V rows' loads and VALU issue;
+// Bound: like the forward, waiting for the K and V rows' loads (0.53 of a wave's life,
+// 0.73 of all requests hit the L2) and VALU issue (2,379 instructions a wave, 50 %);
 // then the per-tap results (26 bytes a tap in bf16 with records).  Against tables
-// of one plane at a time, two of them (S and dP) double-buffered: 4.37 -> 3.99 ms
-// at 65,536 tokens, 16 x 64, bf16; 6.84 -> 6.46 ms at 46,800 tokens, 16 x 96,
-// offsets biased by up to 4 voxels; 16.3 -> 15.9 ms at 131,072 tokens, 24 x 128;
-// 1.90 -> 1.70 ms at 32,768 tokens, 8 x 64, fp32; 120 -> 84 us at 2,048 tokens,
+// of one plane at a time, two of them (S and dP) double-buffered: 4.37 -> 4.05 ms
+// at 65,536 tokens, 16 x 64, bf16; 6.84 -> 6.40 ms at 46,800 tokens, 16 x 96,
+// offsets biased by up to 4 units; 16.3 -> 16.1 ms at 131,072 tokens, 24 x 128;
+// 1.90 -> 1.75 ms at 32,768 tokens, 8 x 64, fp32; 120 -> 74 us at 2,048 tokens,
 // 16 x 64, window 3x5x5.
 #include <algorithm>
 #include <type_traits>

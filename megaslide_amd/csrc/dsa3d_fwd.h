@@ -13,17 +13,18 @@
 // the sampled rows.  Coordinates and corner choice round exactly as the fp32
 // reference does (div_rn, dsa3d_coords.h).
 //
-// Bound: the latency of the K and V rows' loads (half of a workgroup's time; the
-// box of a tile is about 1,000 rows of each, nine in ten from the L2) and VALU
-// issue (~1,450 instructions a wave).  Tables of the whole box against tables of
-// one plane at a time (tested by every tap on every plane, two or three barriers
-// each): 3.20 -> 2.86 ms at 65,536 tokens, 16 x 64, bf16; 6.5 -> 5.8 ms at 46,800
-// tokens, 16 x 96, offsets biased by up to 4 voxels; 2.04 -> 1.46 ms at 32,768
-// tokens, 8 x 64, fp32; 44 -> 30 us at 2,048 tokens, 4 x 64, fp32; unchanged
-// (12.3 -> 12.2 ms) at 131,072 tokens, 24 x 128.  Slower where the box's voxel past
-// the far face weighs: 0.21 -> 0.24 ms at 2 x 60 x 90, 4 x 64, a plane in three.  Tried and slower: a persistent
-// grid with the next tile's offsets loaded ahead (registers spill), 8 or 10
-// blocks of K rows in flight per wave instead of 6.
+// Bound: waiting (0.54 of a wave's life at 65,536 tokens, 16 x 64, bf16), for the K
+// and V rows' loads above all (the box of a tile is about 900 rows of each; 0.83 of
+// all requests hit the L2), and VALU issue (1,591 instructions a wave, 46 % of the
+// time).  Tables of the whole box against tables of one plane at a time (tested by
+// every tap on every plane, two or three barriers each): 3.21 -> 2.87 ms there; 5.9 ->
+// 5.2 ms at 46,800 tokens, 16 x 96, offsets biased by up to 4 units; 11.4 -> 11.1 ms at
+// 131,072 tokens, 24 x 128; 2.04 -> 1.53 ms at 32,768 tokens, 8 x 64, fp32; 41 -> 30 us
+// at 2,048 tokens, 4 x 64, fp32.  Slower where two frames stretch the box over the
+// volume's width (offsets of x count T - 1 to the axis): 0.205 -> 0.211 ms at 2 x 60 x
+// 90, 4 x 64, 0.275 -> 0.302 biased.  Tried and slower: a persistent grid with the next
+// tile's offsets loaded ahead (registers spill), 8 or 10 blocks of K rows in flight per
+// wave instead of 6.
 #pragma once
 
 #include <algorithm>
